@@ -206,6 +206,7 @@ struct vr_scene {
   KdTree kd_sky;                   // over the TRACE_ID_SKY triangles only
   std::vector<int32_t> sky_index;  // kd_sky triangle -> triangle index
   DBuf nodes, refs, planes, sky_nodes, sky_refs;
+  DBuf bvh, bvh_refs, sky_bvh, sky_bvh_refs;
   DevScene dev{};
   int has_sky = 0;
   int64_t device_bytes = 0;
@@ -653,71 +654,70 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
   const int kb = tuning().kd_build;
   const bool device = kb == 1 || (kb == 2 && s->n_tri >= tuning().kd_build_device_min);
   TRY(build_scene_trees(s, n_threads, device));
-  const int nt = host_threads(n_threads);
   const KdTree &kd = s->kd;
-  // device records of a tree: nodes, and 3 float4 per leaf reference whose
-  // meta holds the triangle's index in OptimizedTriangleList (`map` turns a
-  // tree's own triangle numbering into that index)
-  auto flatten = [&](const KdTree &t, const std::vector<int32_t> *map, std::vector<uint2> &nodes,
-                     std::vector<float4> &refs) {
-    nodes.resize(t.children.size());
-    parallel_for((int64_t)nodes.size(), nt, [&](int64_t b, int64_t e) {
-      for (int64_t k = b; k < e; ++k) {
-        uint32_t sb;
-        std::memcpy(&sb, &t.split[(size_t)k], 4);
-        nodes[(size_t)k] = make_uint2(t.children[(size_t)k], sb);
-      }
-    });
-    refs.resize(t.idx.size() * 3);
-    parallel_for((int64_t)t.idx.size(), nt, [&](int64_t b, int64_t e) {
-      for (int64_t k = b; k < e; ++k) {
-        const int32_t ti = map ? (*map)[(size_t)t.idx[(size_t)k]] : t.idx[(size_t)k];
-        const TriIntersect &tr = s->tris[(size_t)ti];
-        uint32_t meta = (uint32_t)ti | ((uint32_t)tr.c0 << 28) | ((uint32_t)tr.c1 << 30);
-        float idf, metaf;
-        std::memcpy(&idf, &tr.id, 4);
-        std::memcpy(&metaf, &meta, 4);
-        refs[(size_t)(3 * k + 0)] = make_float4(tr.nx, tr.ny, tr.nz, tr.d);
-        refs[(size_t)(3 * k + 1)] = make_float4(tr.e[0], tr.e[1], tr.e[2], tr.e[3]);
-        refs[(size_t)(3 * k + 2)] = make_float4(tr.e[4], tr.e[5], idf, metaf);
-      }
-    });
-  };
-  std::vector<uint2> nodes, sky_nodes;
-  std::vector<float4> refs, sky_refs;
-  flatten(kd, nullptr, nodes, refs);
-  if (s->has_sky) {
-    flatten(s->kd_sky, &s->sky_index, sky_nodes, sky_refs);
-    TRY(upload_vec(s->sky_nodes, sky_nodes, g_stream));
-    TRY(upload_vec(s->sky_refs, sky_refs, g_stream));
-  }
-  std::vector<float4> planes((size_t)s->n_tri);
-  parallel_for(s->n_tri, nt, [&](int64_t b, int64_t e) {
-    for (int64_t i = b; i < e; ++i) {
-      const TriIntersect &t = s->tris[(size_t)i];
-      planes[(size_t)i] = make_float4(t.nx, t.ny, t.nz, t.d);
-    }
-  });
-  TRY(upload_vec(s->nodes, nodes, g_stream));
-  TRY(upload_vec(s->refs, refs, g_stream));
-  TRY(upload_vec(s->planes, planes, g_stream));
-  VR_HIP(hipStreamSynchronize(g_stream));
+  float M = 1.0f;
+  for (int c = 0; c < 3; ++c)
+    M = std::max(M, std::max(std::fabs(kd.bmin[c]), std::fabs(kd.bmax[c])));
+  // Device records, made on the device from the triangles' intersection
+  // records and the trees' arrays: kd nodes and leaf records (3 float4 each,
+  // whose meta holds the triangle's index in OptimizedTriangleList), planes,
+  // and the hierarchies the optimised path walks.
+  hipStream_t st = g_stream;
+  DBuf tris, children, split, idx, map;
+  TRY(tris.upload(s->tris.data(), sizeof(TriIntersect) * s->tris.size(), st));
+  const float4 *dt = tris.as<float4>();
   DevScene d{};
+  auto tree = [&](const KdTree &t, const int32_t *own, DBuf &nodes, DBuf &refs, DBuf &bvh,
+                  DBuf &bvh_refs, bool all) -> int {
+    const int64_t nn = (int64_t)t.children.size(), ni = (int64_t)t.idx.size();
+    TRY(children.upload(t.children.data(), 4 * (size_t)nn, st));
+    TRY(split.upload(t.split.data(), 4 * (size_t)nn, st));
+    TRY(idx.upload(t.idx.data(), 4 * (size_t)ni, st));
+    TRY(nodes.alloc(8 * (size_t)nn));
+    TRY(refs.alloc(48 * (size_t)ni));
+    launch_kd_records(children.as<uint32_t>(), split.as<float>(), nn, idx.as<int32_t>(), ni, own,
+                      dt, nodes.as<uint2>(), refs.as<float4>(), st);
+    TRY(check_launch());
+    BvhBuild b;
+    const int rc = own ? build_bvh(dt, s->n_tri, own, (int64_t)s->sky_index.size(), all, M, st, &b)
+                       : build_bvh(dt, s->n_tri, idx.as<int32_t>(), ni, all, M, st, &b);
+    bvh.release();
+    bvh_refs.release();
+    bvh.p = b.nodes;
+    bvh.bytes = 128 * (size_t)b.n_nodes;
+    bvh_refs.p = b.refs;
+    bvh_refs.bytes = 48 * (size_t)b.n_refs;
+    if (b.n_nodes >= (1 << 25)) d.has_bvh = 0;
+    return rc;
+  };
+  d.has_bvh = 1;
+  TRY(tree(kd, nullptr, s->nodes, s->refs, s->bvh, s->bvh_refs, true));
+  if (s->has_sky) {
+    TRY(upload_vec(map, s->sky_index, st));
+    TRY(tree(s->kd_sky, map.as<int32_t>(), s->sky_nodes, s->sky_refs, s->sky_bvh,
+             s->sky_bvh_refs, false));
+  }
+  TRY(s->planes.alloc(16 * (size_t)s->n_tri));
+  launch_planes(dt, s->n_tri, s->planes.as<float4>(), st);
+  TRY(check_launch());
+  VR_HIP(hipStreamSynchronize(st));
   d.nodes = s->nodes.as<uint2>();
   d.refs = s->refs.as<float4>();
   d.planes = s->planes.as<float4>();
-  float M = 1.0f;
   for (int c = 0; c < 3; ++c) {
     d.bmin[c] = kd.bmin[c];
     d.bmax[c] = kd.bmax[c];
-    M = std::max(M, std::max(std::fabs(kd.bmin[c]), std::fabs(kd.bmax[c])));
   }
+  d.bvh = s->bvh.as<float4>();
+  d.bvh_refs = s->bvh_refs.as<float4>();
   d.M = M;
   d.has_sky = s->has_sky;
   d.empty = s->n_tri == 0 ? 1 : 0;
   if (s->has_sky) {
     d.sky_nodes = s->sky_nodes.as<uint2>();
     d.sky_refs = s->sky_refs.as<float4>();
+    d.sky_bvh = s->sky_bvh.as<float4>();
+    d.sky_bvh_refs = s->sky_bvh_refs.as<float4>();
     for (int c = 0; c < 3; ++c) {
       d.sky_bmin[c] = s->kd_sky.bmin[c];
       d.sky_bmax[c] = s->kd_sky.bmax[c];
@@ -725,7 +725,8 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
   }
   s->dev = d;
   s->device_bytes = (int64_t)(s->nodes.bytes + s->refs.bytes + s->planes.bytes +
-                              s->sky_nodes.bytes + s->sky_refs.bytes);
+                              s->sky_nodes.bytes + s->sky_refs.bytes + s->bvh.bytes +
+                              s->bvh_refs.bytes + s->sky_bvh.bytes + s->sky_bvh_refs.bytes);
   s->built = true;
   return VR_OK;
 }

@@ -51,6 +51,26 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
                         const float *vnorm, vr_patch *out, int64_t cap, int64_t *n_out,
                         hipStream_t st);
 
+// ---- trees' device records (bvh.hip) ----
+// The 4-wide hierarchy over the triangles listed in idx (positions in spatial
+// order; a triangle listed several times counts once) and, with `all`, every
+// triangle not listed; tris: n intersection records (48 bytes) in device
+// memory, M the scene's largest coordinate (at least 1).  Allocates nodes and
+// refs with hipMalloc; none when no triangle can be hit.
+struct BvhBuild {
+  void *nodes = nullptr, *refs = nullptr;
+  int64_t n_nodes = 0, n_refs = 0;
+  int levels = 0;
+};
+int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, bool all, float M,
+              hipStream_t st, BvhBuild *out);
+// kd-tree node pairs and leaf records from the tree's arrays (map: the tree's
+// triangle numbering, nullable), and the triangles' planes
+void launch_kd_records(const uint32_t *children, const float *split, int64_t n_nodes,
+                       const int32_t *idx, int64_t n_idx, const int32_t *map, const float4 *tris,
+                       uint2 *nodes, float4 *refs, hipStream_t st);
+void launch_planes(const float4 *tris, int64_t n, float4 *planes, hipStream_t st);
+
 // ---- kd-tree construction on the device (kdbuild.hip) ----
 struct KdTree;
 // The host builder's tree (build_kdtree) built on the GPU on stream st and

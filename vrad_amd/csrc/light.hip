@@ -8,8 +8,8 @@ namespace vr {
 
 #define VR_MAX_TRACE_LENGTH_F ((float)(1.732050807569 * 32768.0))
 
-template <int D, class Stack>
-__device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, float pz, float nx,
+template <class Tracer>
+__device__ void gather_one(const DevScene &sc, Tracer &tr, float px, float py, float pz, float nx,
                            float ny, float nz, const vr_light *__restrict__ lights,
                            int32_t n_lights, const float *__restrict__ dirs, float eps,
                            int32_t skip, float &r, float &g, float &b) {
@@ -30,7 +30,7 @@ __device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, fl
       if (!(dot > 0.0f)) continue;
       const float dot2 = -((L.normal[0] * ux + L.normal[1] * uy) + L.normal[2] * uz);
       if (!(dot2 > 0.0f)) continue;
-      if (!segment_visible<D>(sc, st, sx, sy, sz, L.origin[0], L.origin[1], L.origin[2], skip))
+      if (!segment_visible(sc, tr, sx, sy, sz, L.origin[0], L.origin[1], L.origin[2], skip))
         continue;
       scale = (dot * dot2) / dist2;
     } else if (L.type == VR_EMIT_POINT || L.type == VR_EMIT_SPOTLIGHT) {
@@ -63,7 +63,7 @@ __device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, fl
           fall = fall * (1.0f - sm);
         }
       }
-      if (!segment_visible<D>(sc, st, sx, sy, sz, L.origin[0], L.origin[1], L.origin[2], skip))
+      if (!segment_visible(sc, tr, sx, sy, sz, L.origin[0], L.origin[1], L.origin[2], skip))
         continue;
       scale = dot * fall;
     } else if (L.type == VR_EMIT_SKYLIGHT) {
@@ -71,7 +71,7 @@ __device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, fl
       if (!(dot > 0.0f)) continue;
       const float ex = sx - MTL * L.normal[0], ey = sy - MTL * L.normal[1],
                   ez = sz - MTL * L.normal[2];
-      if (!segment_visible<D>(sc, st, sx, sy, sz, ex, ey, ez, skip)) continue;
+      if (!segment_visible(sc, tr, sx, sy, sz, ex, ey, ez, skip)) continue;
       scale = dot;
     } else if (L.type == VR_EMIT_SKYAMBIENT) {
       float a = 0.0f, w = 0.0f;
@@ -81,7 +81,7 @@ __device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, fl
         if (!(ck > 0.0f)) continue;
         w = w + ck;
         const float ex = sx + MTL * dx, ey = sy + MTL * dy, ez = sz + MTL * dz;
-        if (segment_visible<D>(sc, st, sx, sy, sz, ex, ey, ez, skip)) a = a + ck;
+        if (segment_visible(sc, tr, sx, sy, sz, ex, ey, ez, skip)) a = a + ck;
       }
       if (!(w > 0.0f)) continue;
       scale = a / w;
@@ -97,20 +97,20 @@ __device__ void gather_one(const DevScene &sc, Stack &st, float px, float py, fl
   b = ab;
 }
 
-template <int S, int D>
+template <int S>
 __global__ __launch_bounds__(64) void k_gather_lds(DevScene sc, DevSamples s, int64_t n,
                                                    const vr_light *__restrict__ lights,
                                                    int32_t n_lights, const float *__restrict__ dirs,
                                                    float eps, int32_t skip,
                                                    float *__restrict__ rgb) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   const int64_t i =
       (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup) * 64 + threadIdx.x;
   if (i >= n) return;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
   float r, g, b;
-  gather_one<D>(sc, st, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], lights, n_lights,
+  gather_one(sc, tr, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], lights, n_lights,
                 dirs, eps, skip, r, g, b);
   rgb[3 * i + 0] = r;
   rgb[3 * i + 1] = g;
@@ -125,9 +125,9 @@ __global__ __launch_bounds__(256) void k_gather_plain(DevScene sc, DevSamples s,
                                                       int32_t skip, float *__restrict__ rgb) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  ScratchStack<D> st;
+  KdTracer<D> tr(sc);
   float r, g, b;
-  gather_one<D>(sc, st, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], lights, n_lights,
+  gather_one(sc, tr, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], lights, n_lights,
                 dirs, eps, skip, r, g, b);
   rgb[3 * i + 0] = r;
   rgb[3 * i + 1] = g;
@@ -138,11 +138,11 @@ __global__ __launch_bounds__(256) void k_gather_plain(DevScene sc, DevSamples s,
 // to the job whose block range holds it (binary search; the job index is
 // uniform per wave), and lane l gathers that job's sample
 // (b - first block) * 64 + l from the job's scene and lights.
-template <int S, int D>
+template <int S>
 __global__ __launch_bounds__(64) void k_gather_jobs(const GatherJob *__restrict__ jobs, int n_jobs,
                                                     const float *__restrict__ dirs, float eps,
                                                     int32_t skip) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   const int64_t b = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
   int lo = 0, hi = n_jobs - 1;
   while (lo < hi) {
@@ -154,11 +154,11 @@ __global__ __launch_bounds__(64) void k_gather_jobs(const GatherJob *__restrict_
   const GatherJob &J = jobs[jx];
   const int64_t i = (b - J.blk_begin) * 64 + threadIdx.x;
   if (i >= J.n) return;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(J.sc, s_stk, (int)threadIdx.x, spill);
   const DevSamples &s = J.s;
   float r, g, bb;
-  gather_one<D>(J.sc, st, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], J.lights,
+  gather_one(J.sc, tr, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], J.lights,
                 J.n_lights, dirs, eps, skip, r, g, bb);
   J.rgb[3 * i + 0] = r;
   J.rgb[3 * i + 1] = g;
@@ -170,7 +170,7 @@ void launch_gather_jobs(const GatherJob *jobs, int n_jobs, int64_t total_blocks,
                         hipStream_t st) {
   if (n_jobs <= 0 || total_blocks <= 0) return;
 #define VR_G_JOBS(S)                                                                          \
-  hipLaunchKernelGGL((k_gather_jobs<S, kStackDepth>), dim3((unsigned)total_blocks), dim3(64), 0, \
+  hipLaunchKernelGGL((k_gather_jobs<S>), dim3((unsigned)total_blocks), dim3(64), 0, \
                      st, jobs, n_jobs, sky_dirs, eps, skip)
   switch (lds_entries) {
     case 2: VR_G_JOBS(2); break;
@@ -192,16 +192,16 @@ void launch_gather_jobs(const GatherJob *jobs, int n_jobs, int64_t total_blocks,
 // -1, and the wave stops after the first round in which some lane's
 // segment is visible (a miss, or a sky hit before any other).  "Any" does
 // not depend on the order the directions are taken in.
-template <int S, int D>
+template <int S>
 __global__ __launch_bounds__(64) void k_leaf_sky(DevScene sc, const int16_t *__restrict__ mins,
                                                  const int16_t *__restrict__ maxs, int64_t n,
                                                  const float *__restrict__ dirs,
                                                  uint8_t *__restrict__ out) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   const int64_t leaf = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
   if (leaf >= n) return;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
   const float cx = (float)((int32_t)mins[3 * leaf + 0] + (int32_t)maxs[3 * leaf + 0]) * 0.5f;
   const float cy = (float)((int32_t)mins[3 * leaf + 1] + (int32_t)maxs[3 * leaf + 1]) * 0.5f;
   const float cz = (float)((int32_t)mins[3 * leaf + 2] + (int32_t)maxs[3 * leaf + 2]) * 0.5f;
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64) void k_leaf_sky(DevScene sc, const int16_t *__r
     const int k = k0 + (int)threadIdx.x;
     bool vis = false;
     if (k < 162) {
-      vis = segment_visible<D>(sc, st, cx, cy, cz, dirs[3 * k] * nm + cx,
+      vis = segment_visible(sc, tr, cx, cy, cz, dirs[3 * k] * nm + cx,
                                dirs[3 * k + 1] * nm + cy, dirs[3 * k + 2] * nm + cz, -1);
     }
     if (__any(vis)) {
@@ -226,7 +226,7 @@ void launch_leaf_sky(const DevScene &sc, const int16_t *mins, const int16_t *max
                      const float *sky_dirs, uint8_t *out, hipStream_t st) {
   if (n <= 0) return;
 #define VR_LEAFSKY(S)                                                                      \
-  hipLaunchKernelGGL((k_leaf_sky<S, kStackDepth>), dim3((unsigned)n), dim3(64), 0, st, sc, \
+  hipLaunchKernelGGL((k_leaf_sky<S>), dim3((unsigned)n), dim3(64), 0, st, sc, \
                      mins, maxs, n, sky_dirs, out)
   switch (tuning().trace_lds_entries) {
     case 2: VR_LEAFSKY(2); break;
@@ -246,13 +246,13 @@ void launch_gather_light(const DevScene &sc, const DevSamples &s, int64_t n,
                          float eps, int32_t skip, float *rgb, int path, int lds_entries,
                          hipStream_t st) {
   if (n <= 0) return;
-  if (path == VR_PATH_PLAIN)
+  if (path == VR_PATH_PLAIN || !sc.has_bvh)
     hipLaunchKernelGGL(k_gather_plain<kStackDepth>, dim3((unsigned)((n + 255) / 256)), dim3(256),
                        0, st, sc, s, n, lights, n_lights, sky_dirs, eps, skip, rgb);
   else {
     // the traversal-stack entries kept in LDS: the caller's (autotuned) knob
 #define VR_GATHER(S)                                                                           \
-  hipLaunchKernelGGL((k_gather_lds<S, kStackDepth>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, \
+  hipLaunchKernelGGL((k_gather_lds<S>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, \
                      st, sc, s, n, lights, n_lights, sky_dirs, eps, skip, rgb)
     switch (lds_entries) {
       case 2: VR_GATHER(2); break;

@@ -1,32 +1,34 @@
 // Visibility kernels: batched Trace4Rays (closest hit) and TestLine
-// (segment visibility) over the resident kd-tree.
+// (segment visibility) over the resident trees.
 //
-// Optimised path: one wave per block, XCD-aware ray ranges, per-lane
-// traversal stacks with the top S entries in LDS (S x 8 B x 64 lanes per
-// wave) and the rest in scratch.  Plain path: one thread per ray, 256-thread
-// blocks, the whole stack in private scratch memory.
+// Optimised path: one wave per block, XCD-aware ray ranges, the 4-wide
+// hierarchy with per-lane traversal stacks whose first S entries are in LDS
+// (4 bytes each, 8 for closest hits) and the rest in scratch.  Plain path: one
+// thread per ray, 256-thread blocks, the kd-tree with its whole stack in
+// private scratch memory; it also serves trees too large for the hierarchy's
+// 32-bit node offsets.
 #include "kernels.h"
 
 namespace vr {
 
 // R rays per lane: a wave takes 64 R consecutive rays in R rounds of 64
 // (round q: rays base + 64 q + lane), reusing its LDS stack.
-template <int S, int D, int R>
+template <int S, int R>
 __global__ __launch_bounds__(64) void k_trace_closest_lds(DevScene sc, DevRays r, int64_t n,
                                                           int32_t skip, int32_t *__restrict__ hit,
                                                           float *__restrict__ hit_t,
                                                           float *__restrict__ hit_n, uint32_t xg) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint64_t s_stk[S * 64];
   const int64_t base =
       (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, xg) * 64 * R + threadIdx.x;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
+  BvhSpill<S, uint64_t> spill;
+  BvhTracer<S, uint64_t> tr(sc, s_stk, (int)threadIdx.x, spill);
   for (int q = 0; q < R; ++q) {
     const int64_t i = base + 64 * q;
     if (i >= n) return;
     float t;
     int32_t best, id;
-    trace_ray<D, false>(sc, st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.tmin[i],
+    trace_ray(sc, tr, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.tmin[i],
                         r.tmax[i], skip, t, best, id);
     hit[i] = best;
     hit_t[i] = t;
@@ -45,10 +47,10 @@ __global__ __launch_bounds__(256) void k_trace_closest_plain(DevScene sc, DevRay
                                                              float *hit_t, float *hit_n) {
   const int64_t i = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  ScratchStack<D> st;
+  KdTracer<D> tr(sc);
   float t;
   int32_t best, id;
-  trace_ray<D, false>(sc, st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.tmin[i],
+  trace_ray(sc, tr, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.tmin[i],
                       r.tmax[i], skip, t, best, id);
   hit[i] = best;
   hit_t[i] = t;
@@ -68,19 +70,19 @@ __global__ __launch_bounds__(256) void k_trace_closest_plain(DevScene sc, DevRay
 // blocked the segment before it (occluded_by: exact, the walk would accept
 // that hit); the segments it does not decide are queued in LDS and walked
 // 64 at a time, so lanes stay busy whatever the hit pattern.
-template <int S, int D, int R>
+template <int S, int R>
 __global__ __launch_bounds__(64) void k_test_line_lds(DevScene sc, DevSegs s, int64_t n,
                                                       int32_t skip, uint8_t *__restrict__ vis,
                                                       uint8_t *__restrict__ sky, uint32_t xg) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   __shared__ int32_t s_q[R > 1 ? 64 * (R - 1) : 1];  // queued segments (offsets from base)
   const int lane = (int)threadIdx.x;
   const int64_t base = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, xg) * 64 * R;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, lane, spill);
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(sc, s_stk, lane, spill);
   auto walk = [&](int64_t i, uint32_t &occ) {
     bool hs;
-    const bool v = test_line_cached<D>(sc, st, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i],
+    const bool v = test_line_cached(sc, tr, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i],
                                        s.ez[i], skip, hs, occ);
     vis[i] = v ? 1 : 0;
     if (sky) sky[i] = hs ? 1 : 0;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(64) void k_test_line_lds(DevScene sc, DevSegs s, in
     const int64_t i = base + lane;
     if (i < n) {
       bool hs;
-      const bool v = test_line<D>(sc, st, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i],
+      const bool v = test_line(sc, tr, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i],
                                   skip, hs);
       vis[i] = v ? 1 : 0;
       if (sky) sky[i] = hs ? 1 : 0;
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(64) void k_test_line_lds(DevScene sc, DevSegs s, in
       const int64_t i = first + q;
       if (i >= n) break;
       if (occ != kNoRef &&
-          occluded_by<D>(sc, st, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i], skip, occ)) {
+          occluded_by(sc, tr, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i], skip, occ)) {
         vis[i] = 0;
         if (sky) sky[i] = 0;
       } else {
@@ -136,9 +138,9 @@ __global__ __launch_bounds__(256) void k_test_line_plain(DevScene sc, DevSegs s,
                                                          uint8_t *sky) {
   const int64_t i = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  ScratchStack<D> st;
+  KdTracer<D> tr(sc);
   bool hs;
-  bool v = test_line<D>(sc, st, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i], skip, hs);
+  bool v = test_line(sc, tr, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i], skip, hs);
   vis[i] = v ? 1 : 0;
   if (sky) sky[i] = hs ? 1 : 0;
 }
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(256) void k_test_line_plain(DevScene sc, DevSegs s,
 void launch_trace_closest(const DevScene &sc, const DevRays &r, int64_t n, int32_t skip,
                           int32_t *hit, float *hit_t, float *hit_n, int path, hipStream_t st) {
   if (n <= 0) return;
-  if (path == VR_PATH_PLAIN) {
+  if (path == VR_PATH_PLAIN || !sc.has_bvh) {
     hipLaunchKernelGGL(k_trace_closest_plain<kStackDepth>, dim3((unsigned)((n + 255) / 256)),
                        dim3(256), 0, st, sc, r, n, skip, hit, hit_t, hit_n);
     return;
@@ -163,7 +165,7 @@ void launch_trace_closest(const DevScene &sc, const DevRays &r, int64_t n, int32
   switch (tuning().trace_lds_entries * 8 + R) {
 #define X(S, RR)                                                                              \
   case S * 8 + RR:                                                                            \
-    hipLaunchKernelGGL((k_trace_closest_lds<S, kStackDepth, RR>), g, dim3(64), 0, st, sc, r, n, \
+    hipLaunchKernelGGL((k_trace_closest_lds<S, RR>), g, dim3(64), 0, st, sc, r, n, \
                        skip, hit, hit_t, hit_n, (uint32_t)tuning().trace_xcd_group);          \
     break;
     VR_LDS_VARIANTS(X)
@@ -174,7 +176,7 @@ void launch_trace_closest(const DevScene &sc, const DevRays &r, int64_t n, int32
 void launch_test_line(const DevScene &sc, const DevSegs &s, int64_t n, int32_t skip,
                       uint8_t *vis, uint8_t *sky, int path, hipStream_t st) {
   if (n <= 0) return;
-  if (path == VR_PATH_PLAIN) {
+  if (path == VR_PATH_PLAIN || !sc.has_bvh) {
     hipLaunchKernelGGL(k_test_line_plain<kStackDepth>, dim3((unsigned)((n + 255) / 256)),
                        dim3(256), 0, st, sc, s, n, skip, vis, sky);
     return;
@@ -184,7 +186,7 @@ void launch_test_line(const DevScene &sc, const DevSegs &s, int64_t n, int32_t s
   switch (tuning().trace_lds_entries * 8 + R) {
 #define X(S, RR)                                                                               \
   case S * 8 + RR:                                                                             \
-    hipLaunchKernelGGL((k_test_line_lds<S, kStackDepth, RR>), g, dim3(64), 0, st, sc, s, n, skip, \
+    hipLaunchKernelGGL((k_test_line_lds<S, RR>), g, dim3(64), 0, st, sc, s, n, skip, \
                        vis, sky, (uint32_t)tuning().trace_xcd_group);                          \
     break;
     VR_LDS_VARIANTS(X)

@@ -1,18 +1,22 @@
-// Device-side kd-tree traversal and triangle test shared by the visibility,
+// Device-side tree traversal and triangle test shared by the visibility,
 // transfer and direct-light kernels.  gfx950, wave64.
 //
 // Built with -ffp-contract=off: the triangle test below rounds once per
 // operation in the same association as the CPU restatement, so hit index and
-// hit t are bit-identical to it.  Traversal arithmetic only culls, with a
-// conservative slab margin, so its rounding never changes a result.
+// hit t are bit-identical to it.  Traversal arithmetic only culls, with
+// conservative bounds, so its rounding never changes a result.  The optimised
+// path walks a 4-wide bounding-volume hierarchy (BvhTracer, built by bvh.hip),
+// the plain path the kd-tree (KdTracer).
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace vr {
 
 struct DevScene {
+  // kd-tree (plain path)
   const uint2 *nodes;     // x = children ((index << 2) | type), y = split bits
   const float4 *refs;     // 3 float4 per leaf reference (leaf order)
   const float4 *planes;   // per triangle (nx, ny, nz, d), original order
@@ -24,7 +28,24 @@ struct DevScene {
   const uint2 *sky_nodes;
   const float4 *sky_refs;
   float sky_bmin[3], sky_bmax[3];
+  // 4-wide hierarchies over all triangles and over the sky triangles (null:
+  // no triangle of theirs can be hit): 8 float4 per node (the children's min x,
+  // max x, min y, max y, min z, max z, child words, unused) and 3 float4 per
+  // triangle, each triangle once
+  const float4 *bvh, *bvh_refs;
+  const float4 *sky_bvh, *sky_bvh_refs;
+  int has_bvh;            // 0: too large for 32-bit node offsets, walk the kd-tree
 };
+
+// Child words of the hierarchy: an inner node's index, or a leaf: kBvhLeaf, a
+// triangle count and the first triangle's record (a leaf of no triangles: no
+// child).
+constexpr uint32_t kBvhLeaf = 0x80000000u;
+constexpr int kBvhCntShift = 28;
+constexpr uint32_t kBvhFirstMask = (1u << kBvhCntShift) - 1u;
+// Stack entries of a walk: it leaves at most three children per level, and the
+// build keeps the tree within kBvhStack / 3 levels.
+constexpr int kBvhStack = 64;
 
 constexpr float kTiny = 1e-20f;
 
@@ -94,64 +115,33 @@ __device__ __forceinline__ void tri_test(const float4 *__restrict__ refs, uint32
 }
 constexpr uint32_t kNoRef = 0xffffffffu;
 
-// Per-lane traversal stack entries are 8-byte records: the node index in
-// the low 24 bits, then the entry's interval [a, b] as two 20-bit floats
-// (sign, exponent, the top 11 mantissa bits), a rounded toward -inf and b
-// toward +inf.  A popped interval can only be wider than the pushed one, so
-// a walk may visit a node more, never fewer, and its result is unchanged.
-// Trees hold fewer than 2^24 nodes (the scene build checks).
+// kd nodes a scene may hold (24-bit indices; the scene build checks)
 constexpr uint32_t kStackNodeBits = 24;
-__device__ __forceinline__ uint32_t f20_down(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u >> 12) + ((u >> 31) & ((u & 0xfffu) != 0u));  // negative: magnitude up
-}
-__device__ __forceinline__ uint32_t f20_up(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u >> 12) + ((~u >> 31) & ((u & 0xfffu) != 0u));  // positive: magnitude up
-}
-__device__ __forceinline__ uint2 stack_pack(uint32_t n, float a, float b) {
-  const uint32_t ka = f20_down(a), kb = f20_up(b);
-  return make_uint2(n | (ka << kStackNodeBits), (ka >> 8) | (kb << 12));
-}
-__device__ __forceinline__ void stack_unpack(uint2 w, uint32_t &n, float &a, float &b) {
-  n = w.x & ((1u << kStackNodeBits) - 1u);
-  a = __uint_as_float(((w.x >> kStackNodeBits) | ((w.y & 0xfffu) << 8)) << 12);
-  b = __uint_as_float((w.y >> 12) << 12);
-}
 
-// The first S entries of a lane's stack sit in LDS (entry e of lane l at
-// [e * 64 + l]: one ds_write_b64 / ds_read_b64 per push / pop, conflict
-// free), deeper entries in private scratch.  S = D keeps the whole stack in
-// LDS.  The deeper entries live in a separate object (StackSpill) the stack
+// Traversal stack of the hierarchy's walk: the first S entries of a lane in
+// LDS (entry k of lane l at [64 k + l]: conflict free), deeper ones in private
+// scratch.  The deeper entries live in a separate object (BvhSpill) the stack
 // points to: an array indexed at run time sits in private memory, and keeping
-// it out of this struct lets the LDS pointer stay in a register.
-template <int S, int D>
-struct StackSpill {
-  uint64_t v[D - S > 0 ? D - S : 1];
+// it out of this struct lets the LDS pointer stay in a register.  E: 4-byte
+// child words, or 8 bytes with the entry's key (BvhTracer::walk).
+template <int S, class E>
+struct BvhSpill {
+  E v[kBvhStack - S];
 };
 #define VR_PRIVATE __attribute__((address_space(5)))
-template <int S, int D>
-struct HybridStack {
-  uint2 *e;  // this lane's entry 0 in LDS; entry k at e + 64 k
-  VR_PRIVATE uint64_t *pv;  // private-memory pointer: scratch (not flat) accesses
-  __device__ HybridStack(uint2 *lds, int lane, StackSpill<S, D> &sp)
-      : e(lds + lane), pv((VR_PRIVATE uint64_t *)sp.v) {}
-  __device__ void push(int sp, uint32_t n, float a, float b) {
-    const uint2 w = stack_pack(n, a, b);
-    if (S == D || sp < S)
-      e[64 * sp] = w;
-    else
-      pv[sp - S] = (uint64_t)w.x | ((uint64_t)w.y << 32);
+template <int S, class E>
+struct BvhLaneStack {
+  E *e;              // this lane's entry 0 in LDS
+  VR_PRIVATE E *pv;  // private-memory pointer: scratch (not flat) accesses
+  __device__ BvhLaneStack(E *lds, int lane, BvhSpill<S, E> &sp)
+      : e(lds + lane), pv((VR_PRIVATE E *)sp.v) {}
+  __device__ void push(int sp, E v) {
+    if (sp < S) e[64 * sp] = v;
+    else pv[sp - S] = v;
   }
-  __device__ void get(int sp, uint32_t &n, float &a, float &b) const {
-    uint2 w;
-    if (S == D || sp < S) {
-      w = e[64 * sp];
-    } else {
-      const uint64_t v = pv[sp - S];
-      w = make_uint2((uint32_t)v, (uint32_t)(v >> 32));
-    }
-    stack_unpack(w, n, a, b);
+  __device__ E get(int sp) const {
+    if (sp < S) return e[64 * sp];
+    return pv[sp - S];
   }
 };
 
@@ -387,11 +377,265 @@ __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restr
   return best != best0;
 }
 
-// Closest hit in [tmin, tmax) (ANY: stop at the first hit).
-template <int D, bool ANY, class Stack>
-__device__ void trace_ray(const DevScene &sc, Stack &st, float ox, float oy, float oz, float dx,
-                          float dy, float dz, float tmin, float tmax, int32_t skip, float &t_out,
-                          int32_t &best_out, int32_t &id_out) {
+// ---- tracers: one ray against the scene's trees ---------------------------
+// A tracer is set up for a ray (begin) and then walks the full tree or the sky
+// tree for hits with tmin <= t that come before (tbest, best) in (t, triangle
+// index) order, updating them; ANY: it returns at the first accepted hit.
+// Returns whether a hit was accepted (ref = its record's index).
+
+template <int D>
+struct KdTracer {
+  const DevScene &sc;
+  ScratchStack<D> st;
+  RayPre rp;
+  float ox, oy, oz, dx, dy, dz;
+  __device__ explicit KdTracer(const DevScene &s) : sc(s) {}
+  __device__ __forceinline__ void begin(float ox_, float oy_, float oz_, float dx_, float dy_,
+                                        float dz_) {
+    ox = ox_;
+    oy = oy_;
+    oz = oz_;
+    dx = dx_;
+    dy = dy_;
+    dz = dz_;
+    rp = ray_pre(sc.M, ox, oy, oz, dx, dy, dz);
+  }
+  template <bool ANY, bool SKIPSKY>
+  __device__ __forceinline__ bool full(float tmin, int32_t skip, float &tbest, int32_t &best,
+                                       int32_t &id, uint32_t &ref) {
+    return walk_tree<D, ANY, SKIPSKY, !ANY>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, ox, oy,
+                                            oz, dx, dy, dz, tmin, tbest, skip, tbest, best, id,
+                                            ref);
+  }
+  template <bool ANY>
+  __device__ __forceinline__ bool sky(float tmin, int32_t skip, float &tbest, int32_t &best,
+                                      int32_t &id, uint32_t &ref) {
+    return walk_tree<D, ANY, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax,
+                                           rp, st, ox, oy, oz, dx, dy, dz, tmin, tbest, skip,
+                                           tbest, best, id, ref);
+  }
+};
+
+// The 4-wide hierarchy.  Bound by issue and by the vector cache: a node is
+// 112 bytes per lane (7 loads) and some 80 vector instructions.  On the
+// 8x8-room level a wave of 64 MakeTransfers segments takes 14-18 node steps
+// and 1-2 triangle tests (counted on the CPU; the kd-tree took 60-140 and
+// 40-110).
+//
+// A child's slab entry is fma(near plane, 1/d, a) with a = -o/d (and the exit
+// alike), the near plane picked by the direction's sign through the load's
+// offset.  The boxes hold every point an accepted hit can lie at for origins
+// within the scene's extent M, with the slab arithmetic's rounding
+// (k_bvh_bounds); an origin farther out widens the slabs by 96 u (|o| - M)
+// here.  A direction component of 0 counts as +-1e-20.
+//
+// While the wave's walking lanes are at the same node and share their signs
+// (most steps near the root for rays that start close together), the node
+// comes through scalar loads: a vector load of one address still takes the
+// vector cache 16 cycles, 112 per node, which was 81 % busy on the level's
+// TestLine batch.
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+typedef float f32v4 __attribute__((ext_vector_type(4)));
+struct Planes {
+  f32v4 ax, bx, ay, by, az, bz;  // the four children's near and far planes, by axis
+  u32v4 ch;                      // their words
+  template <class P>
+  __device__ __forceinline__ void load(P pax, P pbx, P pay, P pby, P paz, P pbz, P pch) {
+    auto f = [](P p) {
+      if constexpr (std::is_same<P, const char *>::value)
+        return *reinterpret_cast<const f32v4 *>(p);
+      else  // constant address space: scalar loads
+        return *(const __attribute__((address_space(4))) f32v4 *)p;
+    };
+    ax = f(pax);
+    bx = f(pbx);
+    ay = f(pay);
+    by = f(pby);
+    az = f(paz);
+    bz = f(pbz);
+    const f32v4 c = f(pch);
+    ch = u32v4{__float_as_uint(c.x), __float_as_uint(c.y), __float_as_uint(c.z),
+               __float_as_uint(c.w)};
+  }
+};
+template <int S, class E>
+struct BvhTracer {
+  static constexpr bool kKeyed = sizeof(E) == 8;  // stack entries with keys: closest hits
+  const DevScene &sc;
+  BvhLaneStack<S, E> st;
+  float ox, oy, oz, dx, dy, dz;
+  float ix, iy, iz, nx, ny, nz, fx, fy, fz;
+  uint32_t sx, sy, sz;  // byte offset of the near planes in a node, by axis
+  bool oct;             // the wave's rays (those set up together) share their signs
+  __device__ BvhTracer(const DevScene &s, E *lds, int lane, BvhSpill<S, E> &sp)
+      : sc(s), st(lds, lane, sp) {}
+  __device__ __forceinline__ void begin(float ox_, float oy_, float oz_, float dx_, float dy_,
+                                        float dz_) {
+    ox = ox_;
+    oy = oy_;
+    oz = oz_;
+    dx = dx_;
+    dy = dy_;
+    dz = dz_;
+    const float om = fmaxf(fabsf(ox), fmaxf(fabsf(oy), fabsf(oz)));
+    const float e = fmaxf(om - sc.M, 0.0f) * (96.0f * 0x1p-24f);
+    ix = 1.0f / (fabsf(dx) < kTiny ? copysignf(kTiny, dx) : dx);
+    iy = 1.0f / (fabsf(dy) < kTiny ? copysignf(kTiny, dy) : dy);
+    iz = 1.0f / (fabsf(dz) < kTiny ? copysignf(kTiny, dz) : dz);
+    nx = (-copysignf(e, ix) - ox) * ix;
+    ny = (-copysignf(e, iy) - oy) * iy;
+    nz = (-copysignf(e, iz) - oz) * iz;
+    fx = (copysignf(e, ix) - ox) * ix;
+    fy = (copysignf(e, iy) - oy) * iy;
+    fz = (copysignf(e, iz) - oz) * iz;
+    sx = (__float_as_uint(ix) >> 31) << 4;
+    sy = (__float_as_uint(iy) >> 31) << 4;
+    sz = (__float_as_uint(iz) >> 31) << 4;
+    const uint32_t o = sx | (sy << 1) | (sz << 2);
+    oct = __ballot(o != (uint32_t)__builtin_amdgcn_readfirstlane((int)o)) == 0;
+  }
+  template <bool ANY, bool SKIPSKY>
+  __device__ __forceinline__ bool full(float tmin, int32_t skip, float &tbest, int32_t &best,
+                                       int32_t &id, uint32_t &ref) {
+    return walk<ANY, SKIPSKY>(sc.bvh, sc.bvh_refs, tmin, skip, tbest, best, id, ref);
+  }
+  template <bool ANY>
+  __device__ __forceinline__ bool sky(float tmin, int32_t skip, float &tbest, int32_t &best,
+                                      int32_t &id, uint32_t &ref) {
+    return walk<ANY, false>(sc.sky_bvh, sc.sky_bvh_refs, tmin, skip, tbest, best, id, ref);
+  }
+
+  // Depth first.  Without keys (any hit; and the closest hit in the sky tree
+  // of a few dozen triangles) the children are taken in node order: sorting
+  // them changed an any-hit wave's steps by less than 5 % on six batches.
+  // With keys (closest hits) they are sorted by entry distance, which a popped
+  // entry is checked against again: 27 instead of 82 steps per wave of
+  // hemisphere rays.  A key is the entry distance with the child's number in
+  // its two low bits (rounded down; entries at or behind t = 0 have distance
+  // bits 0 and are never skipped).
+  template <bool ANY, bool SKIPSKY>
+  __device__ __forceinline__ bool walk(const float4 *__restrict__ nodes,
+                                       const float4 *__restrict__ refs, float tmin, int32_t skip,
+                                       float &tbest, int32_t &best, int32_t &best_id,
+                                       uint32_t &best_ref) {
+    // no t lies in an empty interval, and no hit has a NaN in its ray: without
+    // this such a ray would enter every box
+    if (!nodes || (best < 0 && !(tmin < tbest)) || __builtin_isunordered(ox, oy) ||
+        __builtin_isunordered(oz, dx) || __builtin_isunordered(dy, dz))
+      return false;
+    const int32_t best0 = best;
+    const char *const base = reinterpret_cast<const char *>(nodes);
+    constexpr uint32_t kDone = 0xffffffffu;  // no stacked entry is left
+    uint32_t cur = 0;
+    int sp = 0;
+    auto pop = [&]() -> uint32_t {
+      if constexpr (kKeyed) {
+        while (sp > 0) {
+          const uint64_t w = st.get(--sp);
+          const uint32_t key = (uint32_t)(w >> 32);
+          if (key < 4u || __uint_as_float(key & ~3u) <= tbest) return (uint32_t)w;
+        }
+        return kDone;
+      } else {
+        return sp > 0 ? st.get(--sp) : kDone;
+      }
+    };
+    // the children a ray enters: the next one to visit, the others stacked
+    auto step = [&](const Planes &n) -> uint32_t {
+      auto enter = [&](float a, float b, float c) {
+        return fmaxf(fmaxf(__builtin_fmaf(a, ix, nx), __builtin_fmaf(b, iy, ny)),
+                     fmaxf(__builtin_fmaf(c, iz, nz), tmin));
+      };
+      auto leave = [&](float a, float b, float c) {
+        return fminf(fminf(__builtin_fmaf(a, ix, fx), __builtin_fmaf(b, iy, fy)),
+                     fminf(__builtin_fmaf(c, iz, fz), tbest));
+      };
+      const float t0 = enter(n.ax.x, n.ay.x, n.az.x), t1 = enter(n.ax.y, n.ay.y, n.az.y),
+                  t2 = enter(n.ax.z, n.ay.z, n.az.z), t3 = enter(n.ax.w, n.ay.w, n.az.w);
+      const bool h0 = t0 <= leave(n.bx.x, n.by.x, n.bz.x),
+                 h1 = t1 <= leave(n.bx.y, n.by.y, n.bz.y),
+                 h2 = t2 <= leave(n.bx.z, n.by.z, n.bz.z),
+                 h3 = t3 <= leave(n.bx.w, n.by.w, n.bz.w);
+      if constexpr (kKeyed) {
+        constexpr uint32_t kMiss = 0xffffffffu;
+        auto key = [](bool h, float t, uint32_t k) {
+          return h ? (__float_as_uint(fmaxf(t, 0.0f)) & ~3u) | k : kMiss;
+        };
+        uint32_t k0 = key(h0, t0, 0u), k1 = key(h1, t1, 1u), k2 = key(h2, t2, 2u),
+                 k3 = key(h3, t3, 3u);
+        auto order = [](uint32_t &a, uint32_t &b) {
+          const uint32_t lo = min(a, b), hi = max(a, b);
+          a = lo;
+          b = hi;
+        };
+        order(k0, k1);
+        order(k2, k3);
+        order(k0, k2);
+        order(k1, k3);
+        order(k1, k2);
+        auto child = [&](uint32_t k) {
+          const uint32_t a = (k & 1u) ? n.ch.y : n.ch.x, b = (k & 1u) ? n.ch.w : n.ch.z;
+          return (k & 2u) ? b : a;
+        };
+        auto entry = [&](uint32_t k) { return ((uint64_t)k << 32) | child(k); };
+        if (k3 != kMiss) st.push(sp++, entry(k3));
+        if (k2 != kMiss) st.push(sp++, entry(k2));
+        if (k1 != kMiss) st.push(sp++, entry(k1));
+        return k0 != kMiss ? child(k0) : pop();
+      } else {
+        uint32_t next = kDone;
+        auto take = [&](bool h, uint32_t c) {
+          if (h) {
+            if (next != kDone) st.push(sp++, next);
+            next = c;
+          }
+        };
+        take(h0, n.ch.x);
+        take(h1, n.ch.y);
+        take(h2, n.ch.z);
+        take(h3, n.ch.w);
+        return next != kDone ? next : pop();
+      }
+    };
+    for (;;) {
+      while (!(cur & kBvhLeaf)) {
+        Planes n;
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)cur);
+        if (oct && __ballot(cur != u) == 0) {
+          const auto *q = (const __attribute__((address_space(4))) char *)(base + ((size_t)u << 7));
+          const uint32_t ux = (uint32_t)__builtin_amdgcn_readfirstlane((int)sx),
+                         uy = (uint32_t)__builtin_amdgcn_readfirstlane((int)sy),
+                         uz = (uint32_t)__builtin_amdgcn_readfirstlane((int)sz);
+          n.load(q + ux, q + (ux ^ 16u), q + 32 + uy, q + 32 + (uy ^ 16u), q + 64 + uz,
+                 q + 64 + (uz ^ 16u), q + 96);
+          cur = step(n);
+        } else {
+          const uint32_t at = cur << 7;
+          const uint32_t px = at | sx, py = at | sy, pz = at | sz;
+          n.load(base + px, base + (px ^ 16u), base + py + 32, base + (py ^ 16u) + 32,
+                 base + pz + 64, base + (pz ^ 16u) + 64, base + at + 96);
+          cur = step(n);
+        }
+      }
+      if (cur == kDone) break;
+      const uint32_t first = cur & kBvhFirstMask, cnt = (cur & ~kBvhLeaf) >> kBvhCntShift;
+      for (uint32_t k = first; k < first + cnt; ++k)
+        tri_test<SKIPSKY>(refs, k, ox, oy, oz, dx, dy, dz, tmin, skip, tbest, best, best_id,
+                          best_ref);
+      if (ANY && best != best0) return true;
+      cur = pop();
+      if (cur == kDone) break;
+    }
+    return best != best0;
+  }
+};
+
+// Closest hit in [tmin, tmax).
+template <class Tracer>
+__device__ __forceinline__ void trace_ray(const DevScene &sc, Tracer &tr, float ox, float oy,
+                                          float oz, float dx, float dy, float dz, float tmin,
+                                          float tmax, int32_t skip, float &t_out,
+                                          int32_t &best_out, int32_t &id_out) {
   float tbest = tmax;
   int32_t best = -1, best_id = 0;
   t_out = 0.0f;
@@ -399,13 +643,25 @@ __device__ void trace_ray(const DevScene &sc, Stack &st, float ox, float oy, flo
   id_out = 0;
   if (sc.empty) return;
   uint32_t ref = kNoRef;
-  const RayPre rp = ray_pre(sc.M, ox, oy, oz, dx, dy, dz);
-  if (walk_tree<D, ANY, false, !ANY>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, ox, oy, oz, dx,
-                                     dy, dz, tmin, tmax, skip, tbest, best, best_id, ref)) {
+  tr.begin(ox, oy, oz, dx, dy, dz);
+  if (tr.template full<false, false>(tmin, skip, tbest, best, best_id, ref)) {
     t_out = tbest;
     best_out = best;
     id_out = best_id;
   }
+}
+
+// Direction and length of a segment: dir = delta * (1/len).
+__device__ __forceinline__ float segment_dir(float sx, float sy, float sz, float ex, float ey,
+                                             float ez, float &dx, float &dy, float &dz) {
+  const float vx = ex - sx, vy = ey - sy, vz = ez - sz;
+  const float len2 = (vx * vx + vy * vy) + vz * vz;
+  const float len = __builtin_sqrtf(len2);
+  const float inv = 1.0f / len;
+  dx = vx * inv;
+  dy = vy * inv;
+  dz = vz * inv;
+  return len;
 }
 
 // TestLineDoesHitSky for one segment (raytracer/trace/testline.go:22-51):
@@ -416,41 +672,34 @@ __device__ void trace_ray(const DevScene &sc, Stack &st, float ox, float oy, flo
 // tree stops at the first non-sky hit before (ts, is) in (t, index) order;
 // the segment is occluded iff there is one.
 //
-// occluder (in/out): a leaf reference of the full tree to test first (kNoRef
+// occluder (in/out): a record of the full tree to test first (kNoRef
 // for none), typically the triangle that blocked the caller's previous,
 // nearby segment.  It is tested with the same arithmetic and bound as the
 // walk, so a hit there is exactly a hit the walk would accept and the result
 // does not depend on it.  On return it holds the blocking triangle found, if
 // any, else it is unchanged.
-template <int D, class Stack>
-__device__ __forceinline__ bool test_line_cached(const DevScene &sc, Stack &st, float sx,
+template <class Tracer>
+__device__ __forceinline__ bool test_line_cached(const DevScene &sc, Tracer &tr, float sx,
                                                  float sy, float sz, float ex, float ey, float ez,
                                                  int32_t skip, bool &sky, uint32_t &occluder) {
-  const float vx = ex - sx, vy = ey - sy, vz = ez - sz;
-  const float len2 = (vx * vx + vy * vy) + vz * vz;
-  const float len = __builtin_sqrtf(len2);
-  const float inv = 1.0f / len;
-  const float dx = vx * inv, dy = vy * inv, dz = vz * inv;
+  float dx, dy, dz;
+  const float len = segment_dir(sx, sy, sz, ex, ey, ez, dx, dy, dz);
   sky = false;
   if (sc.empty) return true;
   float t = len;
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
-  const RayPre rp = ray_pre(sc.M, sx, sy, sz, dx, dy, dz);
-  if (sc.has_sky)
-    walk_tree<D, false, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax, rp, st,
-                                      sx, sy, sz, dx, dy, dz, 0.0f, len, skip, t, best, id, ref);
+  tr.begin(sx, sy, sz, dx, dy, dz);
+  if (sc.has_sky) tr.template sky<false>(0.0f, skip, t, best, id, ref);
   const int32_t sky_best = best;
   bool occluded = false;
   if (occluder != kNoRef) {
-    tri_test<true>(sc.refs, occluder, sx, sy, sz, dx, dy, dz, 0.0f, skip, t, best, id, ref);
+    tri_test<true>(sc.bvh_refs, occluder, sx, sy, sz, dx, dy, dz, 0.0f, skip, t, best, id, ref);
     occluded = best != sky_best;
   }
   if (!occluded) {
     ref = kNoRef;
-    occluded = walk_tree<D, true, true, false>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, sx,
-                                               sy, sz, dx, dy, dz, 0.0f, len, skip, t, best, id,
-                                               ref);
+    occluded = tr.template full<true, true>(0.0f, skip, t, best, id, ref);
     if (occluded) occluder = ref;
   }
   sky = !occluded && sky_best >= 0;
@@ -464,36 +713,25 @@ __device__ __forceinline__ bool test_line_cached(const DevScene &sc, Stack &st, 
 // hit (test_line_cached's second walk) decide; a sky hit found that way is
 // the closest of all, since every sky hit it passed over lies after an
 // opaque one.  Same results as test_line_cached.
-template <int D, class Stack>
-__device__ __forceinline__ bool test_line(const DevScene &sc, Stack &st, float sx, float sy,
+template <class Tracer>
+__device__ __forceinline__ bool test_line(const DevScene &sc, Tracer &tr, float sx, float sy,
                                           float sz, float ex, float ey, float ez, int32_t skip,
                                           bool &sky) {
-  const float vx = ex - sx, vy = ey - sy, vz = ez - sz;
-  const float len2 = (vx * vx + vy * vy) + vz * vz;
-  const float len = __builtin_sqrtf(len2);
-  const float inv = 1.0f / len;
-  const float dx = vx * inv, dy = vy * inv, dz = vz * inv;
+  float dx, dy, dz;
+  const float len = segment_dir(sx, sy, sz, ex, ey, ez, dx, dy, dz);
   sky = false;
   if (sc.empty) return true;
-  const RayPre rp = ray_pre(sc.M, sx, sy, sz, dx, dy, dz);
   float t = len;
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
-  if (!walk_tree<D, true, true, false>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, sx, sy, sz,
-                                       dx, dy, dz, 0.0f, len, skip, t, best, id, ref)) {
-    if (sc.has_sky)
-      sky = walk_tree<D, true, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax,
-                                             rp, st, sx, sy, sz, dx, dy, dz, 0.0f, len, skip, t,
-                                             best, id, ref);
+  tr.begin(sx, sy, sz, dx, dy, dz);
+  if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) {
+    if (sc.has_sky) sky = tr.template sky<true>(0.0f, skip, t, best, id, ref);
     return true;
   }
   if (!sc.has_sky) return false;
-  const int32_t first = best;
-  walk_tree<D, false, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax, rp, st,
-                                    sx, sy, sz, dx, dy, dz, 0.0f, len, skip, t, best, id, ref);
-  if (best == first) return false;
-  sky = !walk_tree<D, true, true, false>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, sx, sy, sz,
-                                         dx, dy, dz, 0.0f, len, skip, t, best, id, ref);
+  if (!tr.template sky<false>(0.0f, skip, t, best, id, ref)) return false;
+  sky = !tr.template full<true, true>(0.0f, skip, t, best, id, ref);
   return sky;
 }
 
@@ -505,55 +743,43 @@ __device__ __forceinline__ bool test_line(const DevScene &sc, Stack &st, float s
 // hit.  The three steps decide what test_line decides: a sky hit found in
 // the second is the closest of all, since every sky hit it passed over lies
 // after a non-sky hit.
-template <int D, class Stack>
-__device__ __forceinline__ bool segment_visible(const DevScene &sc, Stack &st, float sx, float sy,
+template <class Tracer>
+__device__ __forceinline__ bool segment_visible(const DevScene &sc, Tracer &tr, float sx, float sy,
                                                 float sz, float ex, float ey, float ez,
                                                 int32_t skip) {
-  const float vx = ex - sx, vy = ey - sy, vz = ez - sz;
-  const float len2 = (vx * vx + vy * vy) + vz * vz;
-  const float len = __builtin_sqrtf(len2);
-  const float inv = 1.0f / len;
-  const float dx = vx * inv, dy = vy * inv, dz = vz * inv;
+  float dx, dy, dz;
+  const float len = segment_dir(sx, sy, sz, ex, ey, ez, dx, dy, dz);
   if (sc.empty) return true;
-  const RayPre rp = ray_pre(sc.M, sx, sy, sz, dx, dy, dz);
   float t = len;
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
-  if (!walk_tree<D, true, true, false>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, sx, sy, sz,
-                                       dx, dy, dz, 0.0f, len, skip, t, best, id, ref))
-    return true;
+  tr.begin(sx, sy, sz, dx, dy, dz);
+  if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) return true;
   if (!sc.has_sky) return false;
-  const int32_t first = best;
-  walk_tree<D, false, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax, rp, st,
-                                    sx, sy, sz, dx, dy, dz, 0.0f, len, skip, t, best, id, ref);
-  if (best == first) return false;
-  return !walk_tree<D, true, true, false>(sc.nodes, sc.refs, sc.bmin, sc.bmax, rp, st, sx, sy, sz,
-                                          dx, dy, dz, 0.0f, len, skip, t, best, id, ref);
+  if (!tr.template sky<false>(0.0f, skip, t, best, id, ref)) return false;
+  return !tr.template full<true, true>(0.0f, skip, t, best, id, ref);
 }
 
 // The first half of test_line_cached alone: whether the segment is occluded
-// by `occluder` (a full-tree leaf reference) as test_line would decide it
+// by `occluder` (a record of the full tree) as test_line would decide it
 // (the closest sky hit first, then the same hit test and bound).  False
 // means only that this triangle does not decide it.
-template <int D, class Stack>
-__device__ __forceinline__ bool occluded_by(const DevScene &sc, Stack &st, float sx, float sy,
+template <class Tracer>
+__device__ __forceinline__ bool occluded_by(const DevScene &sc, Tracer &tr, float sx, float sy,
                                             float sz, float ex, float ey, float ez, int32_t skip,
                                             uint32_t occluder) {
-  const float vx = ex - sx, vy = ey - sy, vz = ez - sz;
-  const float len2 = (vx * vx + vy * vy) + vz * vz;
-  const float len = __builtin_sqrtf(len2);
-  const float inv = 1.0f / len;
-  const float dx = vx * inv, dy = vy * inv, dz = vz * inv;
+  float dx, dy, dz;
+  const float len = segment_dir(sx, sy, sz, ex, ey, ez, dx, dy, dz);
   if (sc.empty) return false;
   float t = len;
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
-  if (sc.has_sky)
-    walk_tree<D, false, false, false>(sc.sky_nodes, sc.sky_refs, sc.sky_bmin, sc.sky_bmax,
-                                      ray_pre(sc.M, sx, sy, sz, dx, dy, dz), st, sx, sy, sz, dx,
-                                      dy, dz, 0.0f, len, skip, t, best, id, ref);
+  if (sc.has_sky) {
+    tr.begin(sx, sy, sz, dx, dy, dz);
+    tr.template sky<false>(0.0f, skip, t, best, id, ref);
+  }
   const int32_t sky_best = best;
-  tri_test<true>(sc.refs, occluder, sx, sy, sz, dx, dy, dz, 0.0f, skip, t, best, id, ref);
+  tri_test<true>(sc.bvh_refs, occluder, sx, sy, sz, dx, dy, dz, 0.0f, skip, t, best, id, ref);
   return best != sky_best;
 }
 

@@ -81,14 +81,14 @@ __device__ __forceinline__ void set_pair_bits(uint32_t *bits, int64_t words, int
   atomicOr(bits + (int64_t)j * words + (i >> 5), 1u << (i & 31));
 }
 
-template <int S, int D>
+template <int S>
 __global__ __launch_bounds__(64) void k_pair_trace_lds(DevScene sc, DevPatches p,
                                                        const int2 *__restrict__ pairs,
                                                        const uint32_t *__restrict__ count,
                                                        uint32_t cap, float eps, int32_t skip,
                                                        uint32_t *__restrict__ bits,
                                                        int64_t words, uint32_t xg) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   // The grid is sized for cap pairs; only the first ceil(n / 64) blocks have
   // work.  Blocks are dealt to the XCDs round-robin, so those blocks spread
   // over all of them, and the XCD-aware remap runs over just those.
@@ -99,9 +99,9 @@ __global__ __launch_bounds__(64) void k_pair_trace_lds(DevScene sc, DevPatches p
   if (k >= n) return;
   const int2 ij = pairs[k];
   const int i = ij.x, j = ij.y;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
-  const bool vis = segment_visible<D>(sc, st, p.ox[i] + eps * p.nx[i],
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
+  const bool vis = segment_visible(sc, tr, p.ox[i] + eps * p.nx[i],
                                       p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
                                       p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
                                       p.oz[j] + eps * p.nz[j], skip);
@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256) void k_pair_trace_plain(DevScene sc, DevPatche
   if (k >= n) return;
   const int2 ij = pairs[k];
   const int i = ij.x, j = ij.y;
-  ScratchStack<D> st;
-  const bool vis = segment_visible<D>(sc, st, p.ox[i] + eps * p.nx[i],
+  KdTracer<D> tr(sc);
+  const bool vis = segment_visible(sc, tr, p.ox[i] + eps * p.nx[i],
                                       p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
                                       p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
                                       p.oz[j] + eps * p.nz[j], skip);
@@ -134,13 +134,13 @@ void launch_pair_trace(const DevScene &sc, const DevPatches &p, const int2 *pair
                        const uint32_t *count, uint32_t cap, float eps, int32_t skip,
                        uint32_t *bits, int64_t words, int path, hipStream_t st) {
   if (cap == 0) return;
-  if (path == VR_PATH_PLAIN)
+  if (path == VR_PATH_PLAIN || !sc.has_bvh)
     hipLaunchKernelGGL(k_pair_trace_plain<kStackDepth>, dim3((cap + 255) / 256), dim3(256), 0, st,
                        sc, p, pairs, count, cap, eps, skip, bits, words);
   else {
     // the traversal-stack entries kept in LDS follow the autotuned knob
 #define VR_PAIR_TRACE(S)                                                                    \
-  hipLaunchKernelGGL((k_pair_trace_lds<S, kStackDepth>), dim3((cap + 63) / 64), dim3(64), 0, st, \
+  hipLaunchKernelGGL((k_pair_trace_lds<S>), dim3((cap + 63) / 64), dim3(64), 0, st, \
                      sc, p, pairs, count, cap, eps, skip, bits, words,                          \
                      (uint32_t)tuning().trace_xcd_group)
     switch (tuning().trace_lds_entries) {
@@ -162,10 +162,10 @@ void launch_pair_trace(const DevScene &sc, const DevPatches &p, const int2 *pair
 // jobs' first blocks; the job index is the same for the whole wave, so its
 // descriptor comes through scalar loads), and lane l traces that job's pair
 // (b - first block) * 64 + l on the job's scene.
-template <int S, int D>
+template <int S>
 __global__ __launch_bounds__(64) void k_pair_trace_jobs(const TraceJob *__restrict__ jobs,
                                                         int n_jobs, float eps, int32_t skip) {
-  __shared__ uint2 s_stk[S * 64];
+  __shared__ uint32_t s_stk[S * 64];
   const int64_t b = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
   int lo = 0, hi = n_jobs - 1;
   while (lo < hi) {  // last job with blk_begin <= b
@@ -180,9 +180,9 @@ __global__ __launch_bounds__(64) void k_pair_trace_jobs(const TraceJob *__restri
   const int2 ij = J.pairs[k];
   const int i = ij.x, j = ij.y;
   const DevPatches &p = J.p;
-  StackSpill<S, D> spill;
-  HybridStack<S, D> st(s_stk, (int)threadIdx.x, spill);
-  const bool vis = segment_visible<D>(J.sc, st, p.ox[i] + eps * p.nx[i],
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(J.sc, s_stk, (int)threadIdx.x, spill);
+  const bool vis = segment_visible(J.sc, tr, p.ox[i] + eps * p.nx[i],
                                       p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
                                       p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
                                       p.oz[j] + eps * p.nz[j], skip);
@@ -193,7 +193,7 @@ void launch_pair_trace_jobs(const TraceJob *jobs, int n_jobs, int64_t total_bloc
                             int32_t skip, int lds_entries, hipStream_t st) {
   if (n_jobs <= 0 || total_blocks <= 0) return;
 #define VR_PT_JOBS(S)                                                                          \
-  hipLaunchKernelGGL((k_pair_trace_jobs<S, kStackDepth>), dim3((unsigned)total_blocks), dim3(64), \
+  hipLaunchKernelGGL((k_pair_trace_jobs<S>), dim3((unsigned)total_blocks), dim3(64), \
                      0, st, jobs, n_jobs, eps, skip)
   switch (lds_entries) {
     case 2: VR_PT_JOBS(2); break;
