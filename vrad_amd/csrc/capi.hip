@@ -1303,9 +1303,10 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
   TRY(S.make({fb, fb, fb, fb, fb, fb, 3 * fb, sizeof(vr_light) * (size_t)std::max<int64_t>(nl_tot, 1),
               162 * 3 * 4, sizeof(GatherJob) * (size_t)n_scenes}));
   std::vector<GatherJob> jobs;
-  int64_t at = 0, lat = 0, blocks = 0;
+  int64_t at = 0, lat = 0, blocks = 0, walks = 0;
   for (int32_t k = 0; k < n_scenes; ++k) {
     const int64_t m = n[k];
+    if (m > 0) walks = std::max(walks, light_walks(lights ? lights[k] : nullptr, n_lights[k]));
     const float *src[6] = {samples[k].px, samples[k].py, samples[k].pz,
                            samples[k].nx, samples[k].ny, samples[k].nz};
     for (int q = 0; q < 6 && m > 0; ++q)
@@ -1336,7 +1337,7 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
                         hipMemcpyHostToDevice, st));
   {
     Prof p("gather_light", st);
-    launch_gather_jobs(S.ptr<GatherJob>(9), (int)jobs.size(), blocks, S.ptr<float>(8),
+    launch_gather_jobs(S.ptr<GatherJob>(9), (int)jobs.size(), blocks, walks, S.ptr<float>(8),
                        normal_offset, skip_id, tuning().trace_lds_entries, st);
   }
   TRY(check_launch());
@@ -1603,9 +1604,9 @@ int vr_gather_sample_light(vr_scene *s, const vr_samples *smp, int64_t n, const 
                 S.ptr<float>(3), S.ptr<float>(4), S.ptr<float>(5)};
   {
     Prof p("gather_light", g_stream);
-    launch_gather_light(s->dev, ds, n, S.ptr<vr_light>(7), n_lights, S.ptr<float>(8),
-                        normal_offset, skip_id, S.ptr<float>(6), g_path,
-                        tuning().trace_lds_entries, g_stream);
+    launch_gather_light(s->dev, ds, n, S.ptr<vr_light>(7), n_lights,
+                        light_walks(lights, n_lights), S.ptr<float>(8), normal_offset, skip_id,
+                        S.ptr<float>(6), g_path, tuning().trace_lds_entries, g_stream);
   }
   TRY(check_launch());
   VR_HIP(hipMemcpyAsync(rgb, S.ptr<float>(6), 3 * fb, hipMemcpyDeviceToHost, g_stream));
@@ -2216,8 +2217,10 @@ int serve_request_setup(vr_server *sv, ServeReq *r) {
   float *direct = reinterpret_cast<float *>(base + L.emit1);  // free until the first bounce
   const int path = sv->prm.mode == VR_SERVE_PLAIN ? VR_PATH_PLAIN : VR_PATH_OPT;
   launch_gather_light(sc.scene->dev, ds, n, reinterpret_cast<vr_light *>(base + L.lights),
-                      (int32_t)r->lights.size(), sv->sky.as<float>(), sv->prm.normal_offset, -1,
-                      direct, path, sv->tune.trace_lds_entries, st);
+                      (int32_t)r->lights.size(),
+                      light_walks(r->lights.data(), (int32_t)r->lights.size()),
+                      sv->sky.as<float>(), sv->prm.normal_offset, -1, direct, path,
+                      sv->tune.trace_lds_entries, st);
   launch_emit_init(n, direct, sc.refl.as<float>(), reinterpret_cast<float *>(base + L.emit0),
                    reinterpret_cast<float *>(base + L.total), st);
   VR_HIP(hipMemsetAsync(sv->states.as<BounceState>() + r->slot, 0, sizeof(BounceState), st));

@@ -280,11 +280,14 @@ void launch_read_probe(const void *in, int64_t bytes, float *out, int blocks, hi
 struct DevSamples {
   const float *px, *py, *pz, *nx, *ny, *nz;
 };
-// lds_entries: traversal-stack entries per lane in LDS (2/4/8/12/16/24)
+// Segments a sample's lights may trace: one each, 162 for sky ambient.
+int64_t light_walks(const vr_light *lights, int32_t n_lights);
+// lds_entries: traversal-stack entries per lane in LDS (2/4/8/12/16/24);
+// walks: light_walks of the lights
 void launch_gather_light(const DevScene &sc, const DevSamples &s, int64_t n,
-                         const vr_light *lights, int32_t n_lights, const float *sky_dirs,
-                         float eps, int32_t skip, float *rgb, int path, int lds_entries,
-                         hipStream_t st);
+                         const vr_light *lights, int32_t n_lights, int64_t walks,
+                         const float *sky_dirs, float eps, int32_t skip, float *rgb, int path,
+                         int lds_entries, hipStream_t st);
 // One scene's samples in a many-scene direct-light launch: blocks
 // [blk_begin, blk_begin + ceil(n / 64)) gather samples [0, n) of s on sc with
 // lights[0, n_lights), writing rgb (3 n).
@@ -297,7 +300,8 @@ struct GatherJob {
   int64_t n;
   int64_t blk_begin;
 };
-void launch_gather_jobs(const GatherJob *jobs, int n_jobs, int64_t total_blocks,
+// walks: the most of any job
+void launch_gather_jobs(const GatherJob *jobs, int n_jobs, int64_t total_blocks, int64_t walks,
                         const float *sky_dirs, float eps, int32_t skip, int lds_entries,
                         hipStream_t st);
 // CanLeafTraceToSky per leaf (n waves; n < 2^32): out[i] = 0 / 1

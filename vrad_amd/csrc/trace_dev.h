@@ -725,14 +725,15 @@ __device__ __forceinline__ bool test_line(const DevScene &sc, Tracer &tr, float 
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
   tr.begin(sx, sy, sz, dx, dy, dz);
-  if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) {
-    if (sc.has_sky) sky = tr.template sky<true>(0.0f, skip, t, best, id, ref);
-    return true;
+  for (int pass = 0;; ++pass) {  // one copy of the walk's code
+    if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) {
+      sky = pass != 0 ||
+            (sc.has_sky && tr.template sky<false>(0.0f, skip, t, best, id, ref));
+      return true;
+    }
+    if (pass != 0 || !sc.has_sky || !tr.template sky<false>(0.0f, skip, t, best, id, ref))
+      return false;
   }
-  if (!sc.has_sky) return false;
-  if (!tr.template sky<false>(0.0f, skip, t, best, id, ref)) return false;
-  sky = !tr.template full<true, true>(0.0f, skip, t, best, id, ref);
-  return sky;
 }
 
 // test_line's visibility without its sky output, with the walks in the
@@ -754,10 +755,11 @@ __device__ __forceinline__ bool segment_visible(const DevScene &sc, Tracer &tr, 
   int32_t best = -1, id = 0;
   uint32_t ref = kNoRef;
   tr.begin(sx, sy, sz, dx, dy, dz);
-  if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) return true;
-  if (!sc.has_sky) return false;
-  if (!tr.template sky<false>(0.0f, skip, t, best, id, ref)) return false;
-  return !tr.template full<true, true>(0.0f, skip, t, best, id, ref);
+  for (int pass = 0;; ++pass) {  // one copy of the walk's code
+    if (!tr.template full<true, true>(0.0f, skip, t, best, id, ref)) return true;
+    if (pass != 0 || !sc.has_sky || !tr.template sky<false>(0.0f, skip, t, best, id, ref))
+      return false;
+  }
 }
 
 // The first half of test_line_cached alone: whether the segment is occluded
