@@ -599,7 +599,7 @@ int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, 
   struct Temp {
     char *p = nullptr;
     ~Temp() {
-      if (p) (void)hipFree(p);
+      dev_free(p);
     }
   } tmp;
   size_t off = 0;
@@ -617,7 +617,7 @@ int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, 
   const size_t o_choice = carve(4 * (size_t)cap), o_queue = carve(4 * (size_t)cap);
   const size_t o_wide = carve(128 * (size_t)cap), o_refs = carve(48 * (size_t)cap);
   const size_t o_state = carve(2 * sizeof(PlocState) + 4), o_lv = carve(4 * 128);
-  BVH_HIP(hipMalloc(reinterpret_cast<void **>(&tmp.p), off));
+  BVH_HIP((hipError_t)dev_alloc(reinterpret_cast<void **>(&tmp.p), off));
   auto at = [&](size_t o) { return tmp.p + o; };
   Box *box = reinterpret_cast<Box *>(at(o_box));
   uint8_t *live = reinterpret_cast<uint8_t *>(at(o_live));
@@ -688,8 +688,8 @@ int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, 
     if (pass == 1) return fail(VR_E_CAPACITY, "BVH deeper than the traversal stack");
   }
   if (out->n_nodes == 0) return VR_OK;  // no triangle can be hit
-  BVH_HIP(hipMalloc(&out->nodes, 128 * (size_t)out->n_nodes));
-  BVH_HIP(hipMalloc(&out->refs, 48 * (size_t)out->n_refs));
+  BVH_HIP((hipError_t)dev_alloc(&out->nodes, 128 * (size_t)out->n_nodes));
+  BVH_HIP((hipError_t)dev_alloc(&out->refs, 48 * (size_t)out->n_refs));
   BVH_HIP(hipMemcpyAsync(out->nodes, wide, 128 * (size_t)out->n_nodes, hipMemcpyDeviceToDevice, st));
   BVH_HIP(hipMemcpyAsync(out->refs, refs, 48 * (size_t)out->n_refs, hipMemcpyDeviceToDevice, st));
   BVH_HIP(hipStreamSynchronize(st));

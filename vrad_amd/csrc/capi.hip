@@ -147,6 +147,44 @@ int check_launch() {
   return VR_OK;
 }
 
+// Pinned host memory of the host-pointer calls, one block until the process
+// ends, used under the library lock by one call at a time (every such call
+// leaves its stream drained).  A copy from or to pageable memory costs some 25
+// us whatever its size; small calls pack their arrays here and pay one copy
+// each way, or let the kernel read and write this block itself.
+struct Pinned {
+  static constexpr size_t kBytes = (size_t)4 << 20;
+  char *host = nullptr, *dev = nullptr;
+  size_t used = 0;
+  bool tried = false;
+  void begin() {
+    used = 0;
+    if (tried) return;
+    tried = true;
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, kBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    host = static_cast<char *>(h);
+    dev = static_cast<char *>(d);
+  }
+  // n bytes of the block, or null (then the caller copies to its own memory)
+  char *take(size_t n) {
+    n = (n + 255) & ~(size_t)255;
+    if (!host || n > kBytes - used) return nullptr;
+    char *p = host + used;
+    used += n;
+    return p;
+  }
+  template <class T>
+  T *device(const void *p) const {
+    return reinterpret_cast<T *>(dev + (static_cast<const char *>(p) - host));
+  }
+};
+Pinned g_pin;
+
 // device buffer
 struct DBuf {
   void *p = nullptr;
@@ -156,18 +194,18 @@ struct DBuf {
   DBuf &operator=(const DBuf &) = delete;
   ~DBuf() { release(); }
   void release() {
-    if (p) (void)hipFree(p);
+    dev_free(p);
     p = nullptr;
     bytes = 0;
   }
   int alloc(size_t n) {
     release();
     if (n == 0) n = 16;
-    hipError_t e = hipMalloc(&p, n);
-    if (e != hipSuccess) {
+    const int e = dev_alloc(&p, n);
+    if (e) {
       p = nullptr;
-      (void)hipGetLastError();
-      return fail(VR_E_NOMEM, "hipMalloc(" + std::to_string(n) + "): " + hipGetErrorString(e));
+      return fail(VR_E_NOMEM,
+                  "hipMalloc(" + std::to_string(n) + "): " + hipGetErrorString((hipError_t)e));
     }
     bytes = n;
     return VR_OK;
@@ -175,7 +213,10 @@ struct DBuf {
   int upload(const void *h, size_t n, hipStream_t st) {
     int rc = alloc(n);
     if (rc) return rc;
-    if (n && h) VR_HIP(hipMemcpyAsync(p, h, n, hipMemcpyHostToDevice, st));
+    if (!n || !h) return VR_OK;
+    char *pin = n <= ((size_t)256 << 10) ? g_pin.take(n) : nullptr;
+    if (pin) std::memcpy(pin, h, n);
+    VR_HIP(hipMemcpyAsync(p, pin ? pin : h, n, hipMemcpyHostToDevice, st));
     return VR_OK;
   }
   template <class T>
@@ -196,6 +237,7 @@ using namespace vr;
 
 // ---------------------------------------------------------------------------
 struct vr_scene {
+  DevHolder holder;
   int64_t n_tri = 0;
   std::vector<float> v9;
   std::vector<int32_t> ids;
@@ -213,6 +255,7 @@ struct vr_scene {
 };
 
 struct vr_xfers {
+  DevHolder holder;
   int64_t n = 0, nnz = 0, stored = 0;
   int32_t precision = VR_COEF_F32;
   int64_t pairs = 0, segments = 0;
@@ -391,6 +434,19 @@ std::vector<float> sky_dirs() {
   return std::vector<float>(&kAnorms[0][0], &kAnorms[0][0] + 162 * 3);
 }
 
+constexpr size_t kPackMost = (size_t)1 << 20;  // bytes of one packed copy
+
+struct HostPart {  // part k of a staging block, in host memory (null or 0: skipped)
+  int k;
+  void *p;
+  size_t bytes;
+};
+struct HostCopyBack {  // pinned bytes to hand to the caller once the stream is drained
+  void *to;
+  const void *from;
+  size_t bytes;
+};
+
 // staging for host-pointer calls: one device block carved into arrays
 struct Staging {
   DBuf buf;
@@ -408,7 +464,66 @@ struct Staging {
   T *ptr(int k) const {
     return reinterpret_cast<T *>(buf.as<char>() + parts[(size_t)k].first);
   }
+  // the bytes the listed parts span in the block
+  bool span(const std::vector<HostPart> &v, size_t &lo, size_t &hi) const {
+    lo = ~(size_t)0;
+    hi = 0;
+    for (const HostPart &h : v) {
+      if (!h.p || !h.bytes) continue;
+      lo = std::min(lo, parts[(size_t)h.k].first);
+      hi = std::max(hi, parts[(size_t)h.k].first + h.bytes);
+    }
+    return hi > lo;
+  }
+  // host arrays to their parts: one copy through pinned memory when their span
+  // is small (it must hold nothing the device has written), else one each
+  int upload(const std::vector<HostPart> &v, hipStream_t st) const {
+    size_t lo, hi;
+    if (!span(v, lo, hi)) return VR_OK;
+    char *p = hi - lo <= kPackMost ? g_pin.take(hi - lo) : nullptr;
+    for (const HostPart &h : v) {
+      if (!h.p || !h.bytes) continue;
+      if (p)
+        std::memcpy(p + (parts[(size_t)h.k].first - lo), h.p, h.bytes);
+      else
+        VR_HIP(hipMemcpyAsync(ptr<char>(h.k), h.p, h.bytes, hipMemcpyHostToDevice, st));
+    }
+    if (p) VR_HIP(hipMemcpyAsync(buf.as<char>() + lo, p, hi - lo, hipMemcpyHostToDevice, st));
+    return VR_OK;
+  }
+  // parts to host arrays, likewise; a packed copy leaves its hand-over in `back`
+  int download(const std::vector<HostPart> &v, std::vector<HostCopyBack> &back,
+               hipStream_t st) const {
+    size_t lo, hi;
+    if (!span(v, lo, hi)) return VR_OK;
+    char *p = hi - lo <= kPackMost ? g_pin.take(hi - lo) : nullptr;
+    if (p) VR_HIP(hipMemcpyAsync(p, buf.as<char>() + lo, hi - lo, hipMemcpyDeviceToHost, st));
+    for (const HostPart &h : v) {
+      if (!h.p || !h.bytes) continue;
+      if (p)
+        back.push_back({h.p, p + (parts[(size_t)h.k].first - lo), h.bytes});
+      else
+        VR_HIP(hipMemcpyAsync(h.p, ptr<char>(h.k), h.bytes, hipMemcpyDeviceToHost, st));
+    }
+    return VR_OK;
+  }
 };
+void copy_back(const std::vector<HostCopyBack> &back) {
+  for (const HostCopyBack &c : back) std::memcpy(c.to, c.from, c.bytes);
+}
+
+// the sky directions on the device, until the process ends
+float *g_sky_dirs = nullptr;
+int resident_sky_dirs(const float **out) {
+  if (!g_sky_dirs) {
+    void *p = nullptr;
+    VR_HIP(hipMalloc(&p, sizeof kAnorms));
+    VR_HIP(hipMemcpy(p, kAnorms, sizeof kAnorms, hipMemcpyHostToDevice));
+    g_sky_dirs = static_cast<float *>(p);
+  }
+  *out = g_sky_dirs;
+  return VR_OK;
+}
 
 }  // namespace
 }  // namespace vr
@@ -651,6 +766,7 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
   LOCK;
   if (!s) return fail(VR_E_INVALID, "scene is NULL");
   TRY(ensure_init());
+  g_pin.begin();
   const int kb = tuning().kd_build;
   const bool device = kb == 1 || (kb == 2 && s->n_tri >= tuning().kd_build_device_min);
   TRY(build_scene_trees(s, n_threads, device));
@@ -772,6 +888,9 @@ int vr_scene_destroy(vr_scene *s) {
 }
 
 // ---- visibility ---------------------------------------------------------
+// Items of a host batch that the kernel reads from pinned memory itself.
+constexpr int64_t kDirectItems = 2048;
+
 int vr_trace_closest_dev(vr_scene *s, const vr_rays *r, int64_t n, int32_t skip_id,
                          int32_t *hit, float *hit_t, float *hit_n, void *stream) {
   LOCK;
@@ -818,19 +937,44 @@ int vr_trace_closest(vr_scene *s, const vr_rays *r, int64_t n, int32_t skip_id, 
     return fail(VR_E_INVALID, "NULL ray array or output");
   TRY(ensure_init());
   const size_t fb = 4 * (size_t)n;
+  const float *src[8] = {r->ox, r->oy, r->oz, r->dx, r->dy, r->dz, r->tmin, r->tmax};
+  g_pin.begin();
+  // every ray and result is read or written once: a small batch stays in
+  // pinned host memory, which the kernel reads and writes over the link
+  if (n <= kDirectItems) {
+    char *p = g_pin.take(13 * (fb + 256));
+    if (p) {
+      const size_t step = (fb + 255) & ~(size_t)255;
+      const float *d[8];
+      for (int k = 0; k < 8; ++k) {
+        std::memcpy(p + k * step, src[k], fb);
+        d[k] = g_pin.device<float>(p + k * step);
+      }
+      char *o = p + 8 * step;
+      vr_rays dr{d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7]};
+      TRY(vr_trace_closest_dev(s, &dr, n, skip_id, g_pin.device<int32_t>(o),
+                               g_pin.device<float>(o + step),
+                               hit_n ? g_pin.device<float>(o + 2 * step) : nullptr, nullptr));
+      VR_HIP(hipStreamSynchronize(g_stream));
+      std::memcpy(hit, o, fb);
+      std::memcpy(hit_t, o + step, fb);
+      if (hit_n) std::memcpy(hit_n, o + 2 * step, 3 * fb);
+      return VR_OK;
+    }
+  }
   Staging S;
   TRY(S.make({fb, fb, fb, fb, fb, fb, fb, fb, fb, fb, hit_n ? 3 * fb : 0}));
-  const float *src[8] = {r->ox, r->oy, r->oz, r->dx, r->dy, r->dz, r->tmin, r->tmax};
-  for (int k = 0; k < 8; ++k)
-    VR_HIP(hipMemcpyAsync(S.ptr<float>(k), src[k], fb, hipMemcpyHostToDevice, g_stream));
+  std::vector<HostPart> in;
+  for (int k = 0; k < 8; ++k) in.push_back({k, const_cast<float *>(src[k]), fb});
+  TRY(S.upload(in, g_stream));
   vr_rays dr{S.ptr<float>(0), S.ptr<float>(1), S.ptr<float>(2), S.ptr<float>(3),
              S.ptr<float>(4), S.ptr<float>(5), S.ptr<float>(6), S.ptr<float>(7)};
   TRY(vr_trace_closest_dev(s, &dr, n, skip_id, S.ptr<int32_t>(8), S.ptr<float>(9),
                            hit_n ? S.ptr<float>(10) : nullptr, nullptr));
-  VR_HIP(hipMemcpyAsync(hit, S.ptr<int32_t>(8), fb, hipMemcpyDeviceToHost, g_stream));
-  VR_HIP(hipMemcpyAsync(hit_t, S.ptr<float>(9), fb, hipMemcpyDeviceToHost, g_stream));
-  if (hit_n) VR_HIP(hipMemcpyAsync(hit_n, S.ptr<float>(10), 3 * fb, hipMemcpyDeviceToHost, g_stream));
+  std::vector<HostCopyBack> back;
+  TRY(S.download({{8, hit, fb}, {9, hit_t, fb}, {10, hit_n, 3 * fb}}, back, g_stream));
   VR_HIP(hipStreamSynchronize(g_stream));
+  copy_back(back);
   return VR_OK;
 }
 
@@ -845,18 +989,40 @@ int vr_test_line(vr_scene *s, const vr_segs *g, int64_t n, int32_t skip_id, uint
     return fail(VR_E_INVALID, "NULL segment array or output");
   TRY(ensure_init());
   const size_t fb = 4 * (size_t)n;
+  const float *src[6] = {g->sx, g->sy, g->sz, g->ex, g->ey, g->ez};
+  g_pin.begin();
+  if (n <= kDirectItems) {  // as in vr_trace_closest
+    const size_t step = (fb + 255) & ~(size_t)255;
+    char *p = g_pin.take(8 * step);
+    if (p) {
+      const float *d[6];
+      for (int k = 0; k < 6; ++k) {
+        std::memcpy(p + k * step, src[k], fb);
+        d[k] = g_pin.device<float>(p + k * step);
+      }
+      char *o = p + 6 * step;
+      vr_segs ds{d[0], d[1], d[2], d[3], d[4], d[5]};
+      TRY(vr_test_line_dev(s, &ds, n, skip_id, g_pin.device<uint8_t>(o),
+                           sky ? g_pin.device<uint8_t>(o + step) : nullptr, nullptr));
+      VR_HIP(hipStreamSynchronize(g_stream));
+      std::memcpy(vis, o, (size_t)n);
+      if (sky) std::memcpy(sky, o + step, (size_t)n);
+      return VR_OK;
+    }
+  }
   Staging S;
   TRY(S.make({fb, fb, fb, fb, fb, fb, (size_t)n, (size_t)n}));
-  const float *src[6] = {g->sx, g->sy, g->sz, g->ex, g->ey, g->ez};
-  for (int k = 0; k < 6; ++k)
-    VR_HIP(hipMemcpyAsync(S.ptr<float>(k), src[k], fb, hipMemcpyHostToDevice, g_stream));
+  std::vector<HostPart> in;
+  for (int k = 0; k < 6; ++k) in.push_back({k, const_cast<float *>(src[k]), fb});
+  TRY(S.upload(in, g_stream));
   vr_segs ds{S.ptr<float>(0), S.ptr<float>(1), S.ptr<float>(2),
              S.ptr<float>(3), S.ptr<float>(4), S.ptr<float>(5)};
   TRY(vr_test_line_dev(s, &ds, n, skip_id, S.ptr<uint8_t>(6), sky ? S.ptr<uint8_t>(7) : nullptr,
                        nullptr));
-  VR_HIP(hipMemcpyAsync(vis, S.ptr<uint8_t>(6), (size_t)n, hipMemcpyDeviceToHost, g_stream));
-  if (sky) VR_HIP(hipMemcpyAsync(sky, S.ptr<uint8_t>(7), (size_t)n, hipMemcpyDeviceToHost, g_stream));
+  std::vector<HostCopyBack> back;
+  TRY(S.download({{6, vis, (size_t)n}, {7, sky, (size_t)n}}, back, g_stream));
   VR_HIP(hipStreamSynchronize(g_stream));
+  copy_back(back);
   return VR_OK;
 }
 
@@ -969,8 +1135,10 @@ static int make_transfers_impl(vr_scene *s, const vr_patches *p, int64_t np,
   Staging S;
   TRY(S.make({fb, fb, fb, fb, fb, fb, fb}));
   const float *src[7] = {p->ox, p->oy, p->oz, p->nx, p->ny, p->nz, p->area};
-  for (int k = 0; k < 7 && np > 0; ++k)
-    VR_HIP(hipMemcpyAsync(S.ptr<float>(k), src[k], 4 * (size_t)np, hipMemcpyHostToDevice, st));
+  g_pin.begin();
+  std::vector<HostPart> in;
+  for (int k = 0; k < 7; ++k) in.push_back({k, const_cast<float *>(src[k]), 4 * (size_t)np});
+  TRY(S.upload(in, st));
   DevPatches dp{S.ptr<float>(0), S.ptr<float>(1), S.ptr<float>(2), S.ptr<float>(3),
                 S.ptr<float>(4), S.ptr<float>(5), S.ptr<float>(6)};
   const int64_t words = (np + 31) / 32;
@@ -1300,8 +1468,10 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
   hipStream_t st = g_stream;
   Staging S;
   const size_t fb = 4 * (size_t)ns_tot;
+  const float *dirs = nullptr;
+  TRY(resident_sky_dirs(&dirs));
   TRY(S.make({fb, fb, fb, fb, fb, fb, 3 * fb, sizeof(vr_light) * (size_t)std::max<int64_t>(nl_tot, 1),
-              162 * 3 * 4, sizeof(GatherJob) * (size_t)n_scenes}));
+              sizeof(GatherJob) * (size_t)n_scenes}));
   std::vector<GatherJob> jobs;
   int64_t at = 0, lat = 0, blocks = 0, walks = 0;
   for (int32_t k = 0; k < n_scenes; ++k) {
@@ -1331,13 +1501,11 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
     lat += n_lights[k];
   }
   if (blocks >= ((int64_t)1 << 32)) return fail(VR_E_CAPACITY, "too many samples per launch");
-  std::vector<float> dirs = sky_dirs();
-  VR_HIP(hipMemcpyAsync(S.ptr<float>(8), dirs.data(), dirs.size() * 4, hipMemcpyHostToDevice, st));
-  VR_HIP(hipMemcpyAsync(S.ptr<GatherJob>(9), jobs.data(), sizeof(GatherJob) * jobs.size(),
+  VR_HIP(hipMemcpyAsync(S.ptr<GatherJob>(8), jobs.data(), sizeof(GatherJob) * jobs.size(),
                         hipMemcpyHostToDevice, st));
   {
     Prof p("gather_light", st);
-    launch_gather_jobs(S.ptr<GatherJob>(9), (int)jobs.size(), blocks, walks, S.ptr<float>(8),
+    launch_gather_jobs(S.ptr<GatherJob>(8), (int)jobs.size(), blocks, walks, dirs,
                        normal_offset, skip_id, tuning().trace_lds_entries, st);
   }
   TRY(check_launch());
@@ -1586,31 +1754,32 @@ int vr_gather_sample_light(vr_scene *s, const vr_samples *smp, int64_t n, const 
   if (!rgb || (n_lights > 0 && !lights)) return fail(VR_E_INVALID, "NULL lights/output");
   TRY(ensure_init());
   const size_t fb = 4 * (size_t)n;
-  Staging S;
-  TRY(S.make({fb, fb, fb, fb, fb, fb, 3 * fb, sizeof(vr_light) * (size_t)std::max(n_lights, 1),
-              162 * 3 * 4}));
   const float *src[6] = {smp->px, smp->py, smp->pz, smp->nx, smp->ny, smp->nz};
-  for (int k = 0; k < 6; ++k) {
+  for (int k = 0; k < 6; ++k)
     if (!src[k]) return fail(VR_E_INVALID, "NULL sample array");
-    VR_HIP(hipMemcpyAsync(S.ptr<float>(k), src[k], fb, hipMemcpyHostToDevice, g_stream));
-  }
-  if (n_lights > 0)
-    VR_HIP(hipMemcpyAsync(S.ptr<vr_light>(7), lights, sizeof(vr_light) * (size_t)n_lights,
-                          hipMemcpyHostToDevice, g_stream));
-  std::vector<float> dirs = sky_dirs();
-  VR_HIP(hipMemcpyAsync(S.ptr<float>(8), dirs.data(), dirs.size() * 4, hipMemcpyHostToDevice,
-                        g_stream));
+  const float *dirs = nullptr;
+  TRY(resident_sky_dirs(&dirs));
+  g_pin.begin();
+  Staging S;
+  const size_t lb = sizeof(vr_light) * (size_t)n_lights;
+  TRY(S.make({fb, fb, fb, fb, fb, fb, lb, 3 * fb}));
+  std::vector<HostPart> in;
+  for (int k = 0; k < 6; ++k) in.push_back({k, const_cast<float *>(src[k]), fb});
+  in.push_back({6, const_cast<vr_light *>(lights), lb});
+  TRY(S.upload(in, g_stream));
   DevSamples ds{S.ptr<float>(0), S.ptr<float>(1), S.ptr<float>(2),
                 S.ptr<float>(3), S.ptr<float>(4), S.ptr<float>(5)};
   {
     Prof p("gather_light", g_stream);
-    launch_gather_light(s->dev, ds, n, S.ptr<vr_light>(7), n_lights,
-                        light_walks(lights, n_lights), S.ptr<float>(8), normal_offset, skip_id,
-                        S.ptr<float>(6), g_path, tuning().trace_lds_entries, g_stream);
+    launch_gather_light(s->dev, ds, n, S.ptr<vr_light>(6), n_lights,
+                        light_walks(lights, n_lights), dirs, normal_offset, skip_id,
+                        S.ptr<float>(7), g_path, tuning().trace_lds_entries, g_stream);
   }
   TRY(check_launch());
-  VR_HIP(hipMemcpyAsync(rgb, S.ptr<float>(6), 3 * fb, hipMemcpyDeviceToHost, g_stream));
+  std::vector<HostCopyBack> back;
+  TRY(S.download({{7, rgb, 3 * fb}}, back, g_stream));
   VR_HIP(hipStreamSynchronize(g_stream));
+  copy_back(back);
   return VR_OK;
 }
 
@@ -1625,22 +1794,23 @@ int vr_can_leaf_trace_to_sky(vr_scene *s, const int16_t *mins, const int16_t *ma
   if (n > (int64_t)UINT32_MAX) return fail(VR_E_CAPACITY, "more than 2^32 - 1 leaves per call");
   TRY(ensure_init());
   const size_t bb = 6 * (size_t)n;
+  const float *dirs = nullptr;
+  TRY(resident_sky_dirs(&dirs));
+  g_pin.begin();
   Staging S;
-  TRY(S.make({bb, bb, (size_t)n, 162 * 3 * 4}));
-  VR_HIP(hipMemcpyAsync(S.ptr<int16_t>(0), mins, bb, hipMemcpyHostToDevice, g_stream));
-  VR_HIP(hipMemcpyAsync(S.ptr<int16_t>(1), maxs, bb, hipMemcpyHostToDevice, g_stream));
-  std::vector<float> dirs = sky_dirs();
-  VR_HIP(hipMemcpyAsync(S.ptr<float>(3), dirs.data(), dirs.size() * 4, hipMemcpyHostToDevice,
-                        g_stream));
+  TRY(S.make({bb, bb, (size_t)n}));
+  TRY(S.upload({{0, const_cast<int16_t *>(mins), bb}, {1, const_cast<int16_t *>(maxs), bb}},
+               g_stream));
   {
     Prof p("leaf_sky", g_stream);
-    launch_leaf_sky(s->dev, S.ptr<int16_t>(0), S.ptr<int16_t>(1), n, S.ptr<float>(3),
-                    S.ptr<uint8_t>(2), g_stream);
+    launch_leaf_sky(s->dev, S.ptr<int16_t>(0), S.ptr<int16_t>(1), n, dirs, S.ptr<uint8_t>(2),
+                    g_stream);
   }
   TRY(check_launch());
-  VR_HIP(hipMemcpyAsync(can_see_sky, S.ptr<uint8_t>(2), (size_t)n, hipMemcpyDeviceToHost,
-                        g_stream));
+  std::vector<HostCopyBack> back;
+  TRY(S.download({{2, can_see_sky, (size_t)n}}, back, g_stream));
   VR_HIP(hipStreamSynchronize(g_stream));
+  copy_back(back);
   return VR_OK;
 }
 
@@ -1760,14 +1930,15 @@ int prepare_tiles(vr_xfers *x, const TiledShape &sh, DevTiles &tl, hipStream_t s
   return VR_OK;
 }
 
-// Device buffers of one job of a tiled bounce (emit x2, total, refl, area,
-// e_row, energy scratch, energy); the state lives in a shared array.
+// Device buffers of one job of a tiled bounce (emit, total, refl, area, the
+// other emit, e_row, energy scratch, energy: inputs, then the rest); the state
+// lives in a shared array.
 struct JobBuffers {
   Staging S;
   int make(int64_t n, int K) {
     const size_t vb = 12 * (size_t)std::max<int64_t>(n, 1);
     const int64_t eb = (n + 2047) / 2048;
-    return S.make({vb, vb, vb, vb, 4 * (size_t)std::max<int64_t>(n, 1),
+    return S.make({vb, vb, vb, 4 * (size_t)std::max<int64_t>(n, 1), vb,
                    8 * (size_t)std::max<int64_t>(n, 1), 8 * (size_t)(eb + 2),
                    8 * (size_t)std::max(K, 1)});
   }
@@ -1778,10 +1949,10 @@ void fill_job(BounceJob &jb, const vr_xfers *x, const DevTiles &tl, JobBuffers &
   jb.x = x->dev();
   jb.tl = tl;
   jb.emit[0] = b.S.ptr<float>(0);
-  jb.emit[1] = b.S.ptr<float>(1);
-  jb.total = b.S.ptr<float>(2);
-  jb.refl = b.S.ptr<float>(3);
-  jb.area = b.S.ptr<float>(4);
+  jb.total = b.S.ptr<float>(1);
+  jb.refl = b.S.ptr<float>(2);
+  jb.area = b.S.ptr<float>(3);
+  jb.emit[1] = b.S.ptr<float>(4);
   jb.e_row = b.S.ptr<double>(5);
   jb.scratch = b.S.ptr<double>(6);
   jb.energy = b.S.ptr<double>(7);
@@ -1793,11 +1964,19 @@ void fill_job(BounceJob &jb, const vr_xfers *x, const DevTiles &tl, JobBuffers &
 
 // Runs the bounces of a set of prepared jobs (device table `d_jobs`, states
 // `d_states`) in chunks of 8, optionally as a captured graph of one chunk
-// replayed until every job has stopped.
+// replayed until every job has stopped.  k_done: each job's bounces.
 int run_jobs(const TiledShape &sh, int kind, const BounceJob *d_jobs, int n_jobs,
              int64_t total_chunks, int64_t total_eblocks, BounceState *d_states, int K,
-             bool use_graph, hipStream_t st) {
-  std::vector<BounceState> hs((size_t)n_jobs);
+             bool use_graph, hipStream_t st, std::vector<int32_t> &k_done) {
+  k_done.assign((size_t)n_jobs, 0);
+  // the states are read into pinned memory when there is room
+  std::vector<BounceState> own;
+  BounceState *hs =
+      reinterpret_cast<BounceState *>(g_pin.take(sizeof(BounceState) * (size_t)n_jobs));
+  if (!hs) {
+    own.resize((size_t)n_jobs);
+    hs = own.data();
+  }
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   int rc = VR_OK;
@@ -1836,7 +2015,7 @@ int run_jobs(const TiledShape &sh, int kind, const BounceJob *d_jobs, int n_jobs
       if ((rc = check_launch())) break;
     }
     done += 8;
-    hipError_t e = hipMemcpyAsync(hs.data(), d_states, sizeof(BounceState) * (size_t)n_jobs,
+    hipError_t e = hipMemcpyAsync(hs, d_states, sizeof(BounceState) * (size_t)n_jobs,
                                   hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
@@ -1844,7 +2023,10 @@ int run_jobs(const TiledShape &sh, int kind, const BounceJob *d_jobs, int n_jobs
       break;
     }
     bool all = true;
-    for (const BounceState &b : hs) all = all && (b.converged || b.k_done >= K);
+    for (int j = 0; j < n_jobs; ++j) {
+      k_done[(size_t)j] = hs[j].k_done;
+      all = all && (hs[j].converged || hs[j].k_done >= K);
+    }
     if (all) break;
   }
   if (exec) (void)hipGraphExecDestroy(exec);
@@ -1960,46 +2142,47 @@ int vr_bounce_light_batch(vr_bounce_job *jobs, int32_t n_jobs, const vr_bounce_p
                                   ": transfers are held by a server with another gather layout");
   std::vector<BounceJob> hj((size_t)n_jobs);
   std::vector<JobBuffers> bufs((size_t)n_jobs);
-  DBuf d_states, d_jobs;
-  TRY(d_states.alloc(sizeof(BounceState) * (size_t)n_jobs));
-  VR_HIP(hipMemsetAsync(d_states.p, 0, sizeof(BounceState) * (size_t)n_jobs, st));
+  Staging T;  // the job table and the states
+  const size_t jbytes = sizeof(BounceJob) * (size_t)n_jobs,
+               sbytes = sizeof(BounceState) * (size_t)n_jobs;
+  TRY(T.make({jbytes, sbytes}));
+  std::vector<BounceState> zero((size_t)n_jobs, BounceState{0.0, 0, 0});
+  g_pin.begin();
   int64_t chunks = 0, eblocks = 0;
   for (int j = 0; j < n_jobs; ++j) {
     vr_xfers *x = jobs[j].xfers;
     const int64_t n = x->n;
     DevTiles tl;
     TRY(prepare_tiles(x, sh, tl, st));
-    TRY(bufs[(size_t)j].make(n, K));
+    JobBuffers &b = bufs[(size_t)j];
+    TRY(b.make(n, K));
     BounceJob &jb = hj[(size_t)j];
-    fill_job(jb, x, tl, bufs[(size_t)j], d_states.as<BounceState>() + j, K, prm->stop_frac);
+    fill_job(jb, x, tl, b, T.ptr<BounceState>(1) + j, K, prm->stop_frac);
     jb.chunk_begin = chunks;
     jb.eblk_begin = eblocks;
     chunks += tl.n_chunks;
     eblocks += jb.e_blocks;
-    if (n > 0) {
-      VR_HIP(hipMemcpyAsync(jb.emit[0], jobs[j].emit0, 12 * (size_t)n, hipMemcpyHostToDevice, st));
-      VR_HIP(hipMemcpyAsync(jb.total, jobs[j].total, 12 * (size_t)n, hipMemcpyHostToDevice, st));
-      VR_HIP(hipMemcpyAsync((void *)jb.refl, jobs[j].refl, 12 * (size_t)n, hipMemcpyHostToDevice, st));
-      VR_HIP(hipMemcpyAsync((void *)jb.area, jobs[j].area, 4 * (size_t)n, hipMemcpyHostToDevice, st));
-    }
+    TRY(b.S.upload({{0, const_cast<float *>(jobs[j].emit0), 12 * (size_t)n},
+                    {1, jobs[j].total, 12 * (size_t)n},
+                    {2, const_cast<float *>(jobs[j].refl), 12 * (size_t)n},
+                    {3, const_cast<float *>(jobs[j].area), 4 * (size_t)n}},
+                   st));
   }
-  TRY(d_jobs.upload(hj.data(), sizeof(BounceJob) * (size_t)n_jobs, st));
-  TRY(run_jobs(sh, kind, d_jobs.as<BounceJob>(), n_jobs, chunks, eblocks,
-               d_states.as<BounceState>(), K, use_graph != 0, st));
-  std::vector<BounceState> hs((size_t)n_jobs);
-  VR_HIP(hipMemcpyAsync(hs.data(), d_states.p, sizeof(BounceState) * (size_t)n_jobs,
-                        hipMemcpyDeviceToHost, st));
-  VR_HIP(hipStreamSynchronize(st));
+  TRY(T.upload({{0, hj.data(), jbytes}, {1, zero.data(), sbytes}}, st));
+  std::vector<int32_t> k_done;
+  TRY(run_jobs(sh, kind, T.ptr<BounceJob>(0), n_jobs, chunks, eblocks, T.ptr<BounceState>(1), K,
+               use_graph != 0, st, k_done));
+  std::vector<HostCopyBack> back;
   for (int j = 0; j < n_jobs; ++j) {
-    const BounceJob &jb = hj[(size_t)j];
-    const int done = hs[(size_t)j].k_done;
+    JobBuffers &b = bufs[(size_t)j];
+    const int done = k_done[(size_t)j];
     const int64_t n = jobs[j].xfers->n;
-    if (done > 0)
-      VR_HIP(hipMemcpyAsync(jobs[j].energy, jb.energy, 8 * (size_t)done, hipMemcpyDeviceToHost, st));
-    if (n > 0) VR_HIP(hipMemcpyAsync(jobs[j].total, jb.total, 12 * (size_t)n, hipMemcpyDeviceToHost, st));
+    if (done > 0) TRY(b.S.download({{7, jobs[j].energy, 8 * (size_t)done}}, back, st));
+    TRY(b.S.download({{1, jobs[j].total, 12 * (size_t)n}}, back, st));
     jobs[j].n_bounces = done;
   }
   VR_HIP(hipStreamSynchronize(st));
+  copy_back(back);
   return VR_OK;
 }
 
@@ -2177,6 +2360,7 @@ struct ServeReq {
 }  // namespace vr
 
 struct vr_server {
+  DevHolder holder;
   vr_server_params prm{};
   std::vector<std::unique_ptr<vr::ServeScene>> scenes;
   vr::Arena arena;
@@ -2741,6 +2925,7 @@ int vr_calc_face_extents(const vr_face *faces, int64_t n, const float *lux_ofs,
   TRY(ensure_init());
   static_assert(sizeof(vr_face_lightmap) == 32, "vr_face_lightmap layout");
   hipStream_t st = g_stream;
+  g_pin.begin();
   DBuf df, dofs, dout;
   TRY(df.upload(faces, sizeof(vr_face) * (size_t)n, st));
   if (lux_ofs) TRY(dofs.upload(lux_ofs, 8 * (size_t)n, st));
@@ -2857,6 +3042,7 @@ int vr_face_luxels(const vr_face *faces, int64_t n_faces, const float *lux_ofs,
   if (total == 0) return VR_OK;
   TRY(ensure_init());
   hipStream_t st = g_stream;
+  g_pin.begin();
   DBuf df, dofs, dlm, dblk, dlo, dli, dp, dv, opos, onrm, opat, oval;
   TRY(df.upload(faces, sizeof(vr_face) * (size_t)n_faces, st));
   if (lux_ofs) TRY(dofs.upload(lux_ofs, 8 * (size_t)n_faces, st));

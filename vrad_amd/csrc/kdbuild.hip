@@ -691,7 +691,7 @@ struct Arena {
   std::vector<size_t> sizes;
   size_t cur = 0, used = 0;
   ~Arena() {
-    for (void *p : blocks) (void)hipFree(p);
+    for (void *p : blocks) dev_free(p);
   }
   void reset() {
     cur = 0;
@@ -707,8 +707,7 @@ struct Arena {
     if (cur == blocks.size()) {
       const size_t sz = std::max(bytes, (size_t)64 << 20);
       void *p = nullptr;
-      if (hipMalloc(&p, sz) != hipSuccess) {
-        (void)hipGetLastError();
+      if (dev_alloc(&p, sz) != 0) {
         return fail(VR_E_NOMEM, "kd-tree build: hipMalloc(" + std::to_string(sz) + ")");
       }
       blocks.push_back(p);

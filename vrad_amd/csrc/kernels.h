@@ -56,7 +56,7 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
 // order; a triangle listed several times counts once) and, with `all`, every
 // triangle not listed; tris: n intersection records (48 bytes) in device
 // memory, M the scene's largest coordinate (at least 1).  Allocates nodes and
-// refs with hipMalloc; none when no triangle can be hit.
+// refs with dev_alloc; none when no triangle can be hit.
 struct BvhBuild {
   void *nodes = nullptr, *refs = nullptr;
   int64_t n_nodes = 0, n_refs = 0;

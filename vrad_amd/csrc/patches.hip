@@ -560,9 +560,7 @@ static int make_patches_levels(const vr_face *faces, int64_t n_faces, float max_
     Buf(const Buf &) = delete;
     Buf &operator=(const Buf &) = delete;
     Buf(Buf &&o) noexcept : p(o.p) { o.p = nullptr; }
-    ~Buf() {
-      if (p) (void)hipFree(p);
-    }
+    ~Buf() { dev_free(p); }
   };
   struct Level {
     Buf lv, par, split, cbase, desc, fin, pair;  // par: parent in the level above
@@ -579,7 +577,7 @@ static int make_patches_levels(const vr_face *faces, int64_t n_faces, float max_
     return fail(e == hipErrorOutOfMemory ? VR_E_NOMEM : VR_E_HIP,
                 std::string("make patches: ") + what + ": " + hipGetErrorString(e));
   };
-  auto M = [&](Buf &b, size_t bytes) { return H(hipMalloc(&b.p, bytes ? bytes : 16), "hipMalloc"); };
+  auto M = [&](Buf &b, size_t bytes) { return H((hipError_t)dev_alloc(&b.p, bytes ? bytes : 16), "hipMalloc"); };
   const unsigned gf = (unsigned)((n_faces + 63) / 64);
   if ((rc = M(d_faces, sizeof(vr_face) * n_faces)) || (rc = M(d_tmp, sizeof(vr_patch) * n_faces)) ||
       (rc = M(d_has, n_faces)) || (rc = M(d_fb, 36 * n_faces)) || (rc = M(d_err, 4)) ||
@@ -737,7 +735,7 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
   auto release = [&]() {
     (void)hipStreamSynchronize(st);
     for (void *p : {d_faces, d_base, d_cnt, d_ofs, d_out, d_stk, d_vn})
-      if (p) (void)hipFree(p);
+      dev_free(p);
   };
   auto H = [&](hipError_t e, const char *what) {
     if (e == hipSuccess) return VR_OK;
@@ -746,16 +744,16 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
   };
   const size_t fb = sizeof(vr_face) * (size_t)n_faces;
   const size_t sb = sizeof(Pending) * kMaxDepth * (size_t)n_faces;
-  if ((rc = H(hipMalloc(&d_faces, fb), "hipMalloc")) || (rc = H(hipMalloc(&d_base, 4 * n_faces), "hipMalloc")) ||
-      (rc = H(hipMalloc(&d_cnt, 8 * n_faces), "hipMalloc")) ||
-      (rc = H(hipMalloc(&d_ofs, 16 * n_faces), "hipMalloc")) ||
-      (rc = H(hipMalloc(&d_stk, sb), "hipMalloc")) ||
+  if ((rc = H((hipError_t)dev_alloc(&d_faces, fb), "hipMalloc")) || (rc = H((hipError_t)dev_alloc(&d_base, 4 * n_faces), "hipMalloc")) ||
+      (rc = H((hipError_t)dev_alloc(&d_cnt, 8 * n_faces), "hipMalloc")) ||
+      (rc = H((hipError_t)dev_alloc(&d_ofs, 16 * n_faces), "hipMalloc")) ||
+      (rc = H((hipError_t)dev_alloc(&d_stk, sb), "hipMalloc")) ||
       (rc = H(hipMemcpyAsync(d_faces, faces, fb, hipMemcpyHostToDevice, st), "upload"))) {
     release();
     return rc == VR_E_HIP ? VR_E_NOMEM : rc;
   }
   const size_t vnb = sizeof(float) * kMaxPts * 3 * (size_t)n_faces;
-  if (vnorm && ((rc = H(hipMalloc(&d_vn, vnb), "hipMalloc")) ||
+  if (vnorm && ((rc = H((hipError_t)dev_alloc(&d_vn, vnb), "hipMalloc")) ||
                 (rc = H(hipMemcpyAsync(d_vn, vnorm, vnb, hipMemcpyHostToDevice, st), "upload")))) {
     release();
     return rc;
@@ -801,7 +799,7 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
                                    std::to_string(total) + " patches");
   }
   const size_t ob = sizeof(vr_patch) * (size_t)std::max<int64_t>(total, 1);
-  if ((rc = H(hipMalloc(&d_out, ob), "hipMalloc")) ||
+  if ((rc = H((hipError_t)dev_alloc(&d_out, ob), "hipMalloc")) ||
       (rc = H(hipMemcpyAsync(d_ofs, ofs.data(), 16 * n_faces, hipMemcpyHostToDevice, st), "upload"))) {
     release();
     return rc;

@@ -15,6 +15,18 @@ namespace vr {
 void set_error(const std::string &msg);
 int fail(int code, const std::string &msg);
 
+// ---- device memory (devmem.cpp) ---------------------------------------------
+// Blocks are kept and handed out again; dev_alloc returns 0 or the hipError_t.
+int dev_alloc(void **out, size_t n);
+void dev_free(void *p);  // work in flight may still use the block
+void dev_holder(int delta);  // scenes, transfer sets and servers alive
+struct DevHolder {
+  DevHolder() { dev_holder(1); }
+  ~DevHolder() { dev_holder(-1); }
+  DevHolder(const DevHolder &) = delete;
+  DevHolder &operator=(const DevHolder &) = delete;
+};
+
 // ---- host geometry ---------------------------------------------------------
 // TriIntersectData, raytracer/cache/triangle/triintersectdata.go:3-22 (48 B)
 struct TriIntersect {

@@ -177,9 +177,29 @@ def MakePatches(faces, max_chop=MAX_CHOP, min_chop=MIN_CHOP, vertex_normals=None
             raise ValueError(f"vertex_normals: shape {vn.shape}, want "
                              f"({len(f)}, {_lib.VR_FACE_MAX_POINTS}, 3)")
     n = C.c_int64()
-    check(lib.vr_make_patches_phong(ptr(f), len(f), float(max_chop), float(min_chop), ptr(vn),
-                                    None, 0, C.byref(n)))
-    out = np.zeros(n.value, _lib.PATCH_DTYPE)
-    check(lib.vr_make_patches_phong(ptr(f), len(f), float(max_chop), float(min_chop), ptr(vn),
-                                    ptr(out), len(out), C.byref(n)))
-    return out
+    # room for the patches a face of these lightmap extents usually gives (pages
+    # that are not written cost nothing); a count that exceeds it comes back
+    # with the capacity error and is asked for again
+    out = np.empty(_patch_room(f, float(max_chop)), _lib.PATCH_DTYPE)
+    for _ in range(2):
+        rc = lib.vr_make_patches_phong(ptr(f), len(f), float(max_chop), float(min_chop), ptr(vn),
+                                       ptr(out), len(out), C.byref(n))
+        if rc != _lib.VR_E_CAPACITY or n.value <= len(out):
+            break
+        out = np.empty(n.value, _lib.PATCH_DTYPE)
+    check(rc)
+    return out[:n.value]
+
+
+def _patch_room(faces, max_chop):
+    """Patches the faces may give: leaves of at least half a chop a side, and
+    as many inner patches again."""
+    if len(faces) == 0:
+        return 0
+    used = np.arange(_lib.VR_FACE_MAX_POINTS)[None, :, None] < faces["n_points"][:, None, None]
+    lux = np.stack([faces["lux_s"], faces["lux_t"]], 2)
+    with np.errstate(all="ignore"):
+        uv = np.where(used, faces["points"] @ lux, np.nan)
+        side = np.nan_to_num(np.fmax.reduce(uv, 1) - np.fmin.reduce(uv, 1), posinf=0.0)
+        leaves = np.prod(np.minimum(2.0 * side / max_chop, 4096.0) + 1.0, 1)
+    return int(min(2.0 * leaves.sum() + 16.0 * len(faces), 2.0 ** 23))
