@@ -717,10 +717,16 @@ __host__ __device__ inline int stream_pass_slot(int c, int nc) {
 // loaded into registers when a tile starts and written to the other LDS
 // buffer when it ends (no LDS DMA: the compiler waits for every pending load
 // before an LDS read while a DMA to LDS is in flight).
-template <int KIND, int C, int D>
-__global__ __launch_bounds__(1024) void k_bounce_stream(const BounceJob *__restrict__ jobs,
-                                                        int n_jobs) {
-  const int jid = find_job<&BounceJob::chunk_begin>(jobs, n_jobs, blockIdx.x);
+//
+// SP > 1: a chunk's 16 waves are shared among SP workgroups of 16 / SP waves,
+// each staging the emit tiles for itself.  A wave's sums depend only on its own
+// stream, so the results are the same; what changes is that a transfer set of
+// few chunks uses SP times the CUs (rule: stream_split).
+template <int KIND, int C, int D, int SP>
+__global__ __launch_bounds__(1024 / SP) void k_bounce_stream(const BounceJob *__restrict__ jobs,
+                                                             int n_jobs) {
+  const int64_t chunk = (int64_t)(blockIdx.x / SP);
+  const int jid = find_job<&BounceJob::chunk_begin>(jobs, n_jobs, chunk);
   const BounceJob &jb = jobs[jid];
   if (job_done(jb)) return;
   const int kb = jb.state->k_done;
@@ -730,21 +736,24 @@ __global__ __launch_bounds__(1024) void k_bounce_stream(const BounceJob *__restr
   float *__restrict__ emit_out = jb.emit[(kb + 1) & 1];
   constexpr int G = 4;                 // entries per chunk, every precision
   constexpr int PW = 128 * G;          // entries per pass of a wave
-  constexpr int T = 1024;              // threads
+  constexpr int T = 1024 / SP;         // threads
+  constexpr int NW = 16 / SP;          // waves
   constexpr int RS = 1028;             // stride of a block's segment offsets
   constexpr int EPT = C / T;           // emit records copied per thread and tile
   constexpr int cbytes = KIND == VR_COEF_F32 ? 4 : 2;
   static_assert(C % T == 0 && 16 * C <= 65536, "16-byte LDS records with 16-bit offsets");
   __shared__ __attribute__((aligned(16))) float s_e[2][4 * C];  // (r, g, b, -) per patch
-  __shared__ __attribute__((aligned(16))) float s_acc[16 * 64 * 4];  // slot sums per wave
-  __shared__ int64_t s_bs[kMaxTilesPerJob];  // this chunk's block starts
-  __shared__ int s_tn[kMaxTilesPerJob];      // this chunk's tiles holding entries, in order
-  __shared__ int s_wn[16];
+  __shared__ __attribute__((aligned(16))) float s_acc[NW * 64 * 4];  // slot sums per wave
+  constexpr int kTiles = kMaxTilesPerJob / SP;  // stream_split: fewer tiles than threads
+  __shared__ int64_t s_bs[kTiles];  // this chunk's block starts
+  __shared__ int s_tn[kTiles];      // this chunk's tiles holding entries, in order
+  __shared__ int s_wn[NW];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t c = (int64_t)blockIdx.x - jb.chunk_begin;
+  const int own = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in the workgroup
+  const int wave = (int)(blockIdx.x % SP) * NW + own;                       // in the chunk
+  const int64_t c = chunk - jb.chunk_begin;
   const int nt = tl.nt;
-  static_assert(kMaxTilesPerJob <= T, "one thread per tile lists the tiles");
+  static_assert(kTiles <= T, "one thread per tile lists the tiles");
   // Tiles where no row of the chunk has entries add nothing to any sum: the
   // chunk walks only the others (block totals are boff[block][1024]), in
   // tile order, so the sums do not change.
@@ -752,13 +761,13 @@ __global__ __launch_bounds__(1024) void k_bounce_stream(const BounceJob *__restr
   const bool tile_live = tt < nt && tl.boff[(c * nt + tt) * (int64_t)RS + 1024] > 0;
   const uint64_t live_bits = __ballot(tile_live);
   if (tt < nt) s_bs[tt] = tl.bstart[c * nt + tt];
-  if (lane == 0) s_wn[wave] = __builtin_popcountll(live_bits);
-  f32x3 *const acc = reinterpret_cast<f32x3 *>(s_acc) + 64 * wave;
+  if (lane == 0) s_wn[own] = __builtin_popcountll(live_bits);
+  f32x3 *const acc = reinterpret_cast<f32x3 *>(s_acc) + 64 * own;
   acc[lane] = f32x3{0.0f, 0.0f, 0.0f};
   __syncthreads();
   int live_before = 0, n_live = 0;
-  for (int w2 = 0; w2 < 16; ++w2) {
-    live_before += w2 < wave ? s_wn[w2] : 0;
+  for (int w2 = 0; w2 < NW; ++w2) {
+    live_before += w2 < own ? s_wn[w2] : 0;
     n_live += s_wn[w2];
   }
   if (tile_live)
@@ -1129,12 +1138,43 @@ bool bounce_gather_variant(const GatherShape &sh) {
   return false;
 }
 
+// Workgroups per chunk: the most of 1, 2, 4, 8 that still run at once (a
+// workgroup's LDS takes a whole CU).  Above 1 the launch holds at most 128
+// chunks, so no set of it has more than 32,768 rows or 8 column tiles.  20,011
+// rows of 30 M FP16 transfers (79 chunks): 62.7 us per bounce with one, 55.7
+// with two; 5,970 rows (24 chunks): 16.5 with one, 12.4 with eight.  What is
+// left is the longest wave: rows are not cut, and the slowest wave of a
+// workgroup sets its tile.  Loads running three passes ahead (57.3, 13.7) and
+// two passes side by side (62.6, 14.4) did not help.
+static int stream_split(int64_t chunks) {
+  int sp = 1;
+  while (sp < 8 && chunks * sp * 2 <= kChunkTarget) sp *= 2;
+  return sp;
+}
+
 void launch_gather_jobs(int kind, const GatherShape &sh, const BounceJob *jobs, int n_jobs,
                         int64_t total_chunks, hipStream_t st) {
   if (n_jobs <= 0 || total_chunks <= 0) return;
   const dim3 g((unsigned)total_chunks);
 #define VR_GO(KER, K, ...) \
   hipLaunchKernelGGL((KER<K, __VA_ARGS__>), g, dim3(1024), 0, st, jobs, n_jobs)
+#define VR_GO_SPLIT(K, SP)                                                                 \
+  hipLaunchKernelGGL((k_bounce_stream<K, 4096, 1, SP>), dim3((unsigned)total_chunks * SP), \
+                     dim3(1024 / SP), 0, st, jobs, n_jobs)
+#define VR_SPLIT(SP)                                                  \
+  {                                                                   \
+    if (kind == VR_COEF_F32) VR_GO_SPLIT(VR_COEF_F32, SP);            \
+    else if (kind == VR_COEF_F16) VR_GO_SPLIT(VR_COEF_F16, SP);       \
+    else VR_GO_SPLIT(VR_COEF_BF16, SP);                               \
+    return;                                                           \
+  }
+  if (sh.kernel == 2 && sh.cols == 4096 && sh.prefetch == 1) switch (stream_split(total_chunks)) {
+      case 8: VR_SPLIT(8)
+      case 4: VR_SPLIT(4)
+      case 2: VR_SPLIT(2)
+    }
+#undef VR_SPLIT
+#undef VR_GO_SPLIT
 #define VR_KINDS(KER, ...)                                   \
   {                                                          \
     if (kind == VR_COEF_F32) VR_GO(KER, VR_COEF_F32, __VA_ARGS__);  \
@@ -1146,7 +1186,7 @@ void launch_gather_jobs(int kind, const GatherShape &sh, const BounceJob *jobs, 
   if (sh.cols == CC && sh.group == GG && sh.passes == PP && sh.prefetch == DD)            \
     VR_KINDS(k_bounce_tiled, CC, GG, PP, DD)
 #define VR_SHAPE_S(CC, DD) \
-  if (sh.cols == CC && sh.prefetch == DD) VR_KINDS(k_bounce_stream, CC, DD)
+  if (sh.cols == CC && sh.prefetch == DD) VR_KINDS(k_bounce_stream, CC, DD, 1)
   if (sh.kernel == 0) {
     VR_TILED_SHAPES(VR_SHAPE)
   } else if (sh.kernel == 2) {
@@ -1216,7 +1256,8 @@ void launch_energy(const double *e_row, int64_t n, double *scratch, double *ener
 
 // ---- FP64 energy of batched jobs: the same tree as launch_energy for
 // n <= 2048^2 (stage 1: blocks of 2048 over e_row; stage 2: one block over
-// the stage-1 partials when there is more than one), then the stop test.
+// the stage-1 partials when there is more than one), then the stop test.  A
+// job without rows has one workgroup, which sums nothing.
 __device__ __forceinline__ double reduce_block2048(const double *__restrict__ in, int64_t m,
                                                    int64_t blk, double *v) {
   const int t = threadIdx.x;
@@ -1236,34 +1277,32 @@ __device__ __forceinline__ double reduce_block2048(const double *__restrict__ in
   return v[0];
 }
 
-__global__ __launch_bounds__(256) void k_energy_jobs1(const BounceJob *__restrict__ jobs,
-                                                      int n_jobs) {
+// One launch per bounce: a job's stage-1 workgroups leave their partials, and
+// the last of them to arrive reduces those and does the stop test.  The three
+// launches before it took 13.8 us of a 20,011-row set's bounce, this one 7.4.
+__global__ __launch_bounds__(256) void k_energy_jobs(const BounceJob *__restrict__ jobs,
+                                                     int n_jobs) {
   __shared__ double v[256];
+  __shared__ int s_last;
   const int jid = find_job<&BounceJob::eblk_begin>(jobs, n_jobs, blockIdx.x);
   const BounceJob &jb = jobs[jid];
-  if (job_done(jb)) return;
-  const int64_t lb = (int64_t)blockIdx.x - jb.eblk_begin;
-  const double r = reduce_block2048(jb.e_row, jb.x.n, lb, v);
-  if (threadIdx.x == 0) jb.scratch[lb] = r;
-}
-
-__global__ __launch_bounds__(256) void k_energy_jobs2(const BounceJob *__restrict__ jobs) {
-  __shared__ double v[256];
-  const BounceJob &jb = jobs[blockIdx.x];
-  if (job_done(jb) || jb.e_blocks <= 1) return;
-  const double r = reduce_block2048(jb.scratch, jb.e_blocks, 0, v);
-  if (threadIdx.x == 0) jb.scratch[jb.e_blocks] = r;
-}
-
-__global__ __launch_bounds__(64) void k_energy_jobs_final(const BounceJob *__restrict__ jobs,
-                                                          int n_jobs) {
-  const int j = blockIdx.x * 64 + threadIdx.x;
-  if (j >= n_jobs) return;
-  const BounceJob &jb = jobs[j];
-  if (job_done(jb)) return;
-  const double ek = jb.e_blocks > 1 ? jb.scratch[jb.e_blocks]
-                    : jb.e_blocks == 1 ? jb.scratch[0] : 0.0;
+  if (job_done(jb)) return;  // the state changes only once every workgroup has arrived
   BounceState *stt = jb.state;
+  const int64_t lb = (int64_t)blockIdx.x - jb.eblk_begin;
+  double ek = reduce_block2048(jb.e_row, jb.x.n, lb, v);
+  if (jb.e_blocks > 1) {
+    if (threadIdx.x == 0) {
+      jb.scratch[lb] = ek;
+      __threadfence();
+      s_last = atomicAdd(&stt->arrived, 1u) + 1u == (uint32_t)jb.e_blocks;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    ek = reduce_block2048(jb.scratch, jb.e_blocks, 0, v);
+  }
+  if (threadIdx.x != 0) return;
+  stt->arrived = 0u;
   const int k = stt->k_done;
   jb.energy[k] = ek;
   const double cum = stt->cum + ek;
@@ -1273,13 +1312,8 @@ __global__ __launch_bounds__(64) void k_energy_jobs_final(const BounceJob *__res
 }
 
 void launch_energy_jobs(const BounceJob *jobs, int n_jobs, int64_t total_eblocks, hipStream_t st) {
-  if (n_jobs <= 0) return;
-  if (total_eblocks > 0)
-    hipLaunchKernelGGL(k_energy_jobs1, dim3((unsigned)total_eblocks), dim3(256), 0, st, jobs,
-                       n_jobs);
-  hipLaunchKernelGGL(k_energy_jobs2, dim3((unsigned)n_jobs), dim3(256), 0, st, jobs);
-  hipLaunchKernelGGL(k_energy_jobs_final, dim3((unsigned)((n_jobs + 63) / 64)), dim3(64), 0, st,
-                     jobs, n_jobs);
+  if (n_jobs <= 0 || total_eblocks <= 0) return;
+  hipLaunchKernelGGL(k_energy_jobs, dim3((unsigned)total_eblocks), dim3(256), 0, st, jobs, n_jobs);
 }
 
 void launch_bounce_jobs(int kind, const GatherShape &sh, const BounceJob *jobs, int n_jobs,

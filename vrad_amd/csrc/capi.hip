@@ -1957,7 +1957,7 @@ void fill_job(BounceJob &jb, const vr_xfers *x, const DevTiles &tl, JobBuffers &
   jb.scratch = b.S.ptr<double>(6);
   jb.energy = b.S.ptr<double>(7);
   jb.state = state;
-  jb.e_blocks = (x->n + 2047) / 2048;
+  jb.e_blocks = std::max<int64_t>(1, (x->n + 2047) / 2048);
   jb.max_bounces = K;
   jb.stop_frac = stop_frac;
 }
@@ -2080,7 +2080,7 @@ int vr_bounce_light(vr_xfers *x, const float *emit0, const float *refl, const fl
   VR_HIP(hipMemsetAsync(counters, 0, 4 * (size_t)std::max(K, 1), st));
   VR_HIP(hipMemsetAsync(state, 0, sizeof(BounceState), st));
   const DevXfers dx = x->dev();
-  BounceState hs{0.0, 0, 0};
+  BounceState hs{};
   const int chunk = g_path == VR_PATH_PLAIN ? 1 : 8;
   int k = 0;
   while (k < K) {
@@ -2146,7 +2146,7 @@ int vr_bounce_light_batch(vr_bounce_job *jobs, int32_t n_jobs, const vr_bounce_p
   const size_t jbytes = sizeof(BounceJob) * (size_t)n_jobs,
                sbytes = sizeof(BounceState) * (size_t)n_jobs;
   TRY(T.make({jbytes, sbytes}));
-  std::vector<BounceState> zero((size_t)n_jobs, BounceState{0.0, 0, 0});
+  std::vector<BounceState> zero((size_t)n_jobs, BounceState{});
   g_pin.begin();
   int64_t chunks = 0, eblocks = 0;
   for (int j = 0; j < n_jobs; ++j) {
@@ -2228,7 +2228,7 @@ int vr_bounce_light_noalloc(vr_xfers *x, const float *emit0, const float *refl,
   jb.scratch = reinterpret_cast<double *>(base + kNaEScr);
   jb.energy = reinterpret_cast<double *>(base + kNaEnergy);
   jb.state = reinterpret_cast<BounceState *>(base + kNaState);
-  jb.e_blocks = (n + 2047) / 2048;
+  jb.e_blocks = std::max<int64_t>(1, (n + 2047) / 2048);
   jb.max_bounces = K;
   jb.stop_frac = prm->stop_frac;
   jb.chunk_begin = 0;
@@ -2244,7 +2244,7 @@ int vr_bounce_light_noalloc(vr_xfers *x, const float *emit0, const float *refl,
   VR_HIP(hipMemsetAsync(jb.state, 0, sizeof(BounceState), st));
   VR_HIP(hipMemcpyAsync(d_job, &jb, sizeof jb, hipMemcpyHostToDevice, st));
   const int kind = x->precision;
-  BounceState hs{0.0, 0, 0};
+  BounceState hs{};
   for (int done = 0; done < K; done += 8) {
     for (int i = 0; i < std::min(8, K - done); ++i) {
       launch_gather_jobs(kind, sh, d_job, 1, tl.n_chunks, st);
@@ -2426,7 +2426,7 @@ void serve_job(vr_server *sv, ServeReq *r, BounceJob &jb) {
   jb.scratch = reinterpret_cast<double *>(base + L.scratch);
   jb.energy = reinterpret_cast<double *>(base + L.energy);
   jb.state = sv->states.as<BounceState>() + r->slot;
-  jb.e_blocks = (sc.n + 2047) / 2048;
+  jb.e_blocks = std::max<int64_t>(1, (sc.n + 2047) / 2048);
   jb.max_bounces = sv->prm.bounces;
   jb.stop_frac = 0.0;
 }

@@ -191,6 +191,8 @@ struct BounceState {       // device-resident bounce bookkeeping
   double cum;
   int32_t converged;
   int32_t k_done;
+  uint32_t arrived;        // energy workgroups of the current bounce (0 between launches)
+  uint32_t pad;
 };
 // One transfer set's bounce in a batched launch of the LDS-tiled gather and
 // the FP64 energy.  The bounce index is state->k_done: the gather reads
@@ -206,7 +208,7 @@ struct BounceJob {
   BounceState *state;
   int64_t chunk_begin;     // first gather workgroup of the job
   int64_t eblk_begin;      // first stage-1 energy block of the job
-  int64_t e_blocks;        // ceil(n / 2048) stage-1 blocks (n <= 2048^2)
+  int64_t e_blocks;        // stage-1 blocks: ceil(n / 2048), at least 1 (n <= 2048^2)
   int32_t max_bounces;
   double stop_frac;
 };
