@@ -219,7 +219,7 @@ typedef struct {
   float normal_offset;  /* segment end offset along each normal (0.1) */
   int32_t skip_id;
   int32_t normalize;    /* scale rows with FP64 sum > 1 by 1/sum */
-  int64_t batch_pairs;  /* candidate pairs per visibility batch (<=0: 32M) */
+  int64_t batch_pairs;  /* candidate pairs per visibility batch (<=0: 32M); no effect on results */
 } vr_xfer_params;
 typedef struct vr_xfers vr_xfers;
 typedef struct {
@@ -237,13 +237,11 @@ int vr_make_transfers(vr_scene *s, const vr_patches *p, int64_t n_patches,
                       const vr_xfer_params *params, vr_xfers **out);
 /* MakeTransfers for many scenes at once (no reference counterpart): scene
  * k's patches[k] (n_patches[k] of them) give out[k],
- * equal bit for bit to vr_make_transfers(scenes[k], ...).  Every round, each
- * unfinished scene culls its next candidate rows into its own region of one
- * pair buffer (params->batch_pairs pairs per round, default 32M, shared
- * among the scenes still culling, at least a row each), and one visibility
- * launch walks all regions through a table of scene descriptors.  A scene
- * with params->batch_pairs candidate pairs or more fills a round alone and
- * runs as vr_make_transfers would.  The plain path runs the scenes one by
+ * equal bit for bit to vr_make_transfers(scenes[k], ...).  One visibility
+ * launch culls and traces the scenes' candidate pairs through a table of
+ * scene descriptors.  A scene with params->batch_pairs candidate pairs
+ * (default 32M) or more fills the GPU alone and runs as vr_make_transfers
+ * would.  The plain path runs the scenes one by
  * one.
  * On failure no out[k] is set. */
 int vr_make_transfers_batch(vr_scene *const *scenes, const vr_patches *patches,

@@ -40,9 +40,6 @@ std::recursive_mutex g_mu;
 bool g_init = false;
 int g_device = 0;
 hipStream_t g_stream = nullptr;
-// a second stream, on which MakeTransfers runs every other round of its
-// visibility batches (default priority, like g_stream)
-hipStream_t g_stream2 = nullptr;
 int g_path = VR_PATH_OPT;
 bool g_prof = false;
 
@@ -132,7 +129,6 @@ int ensure_init() {
     return fail(VR_E_INVALID, "no such device");
   VR_HIP(hipSetDevice(g_device));
   VR_HIP(hipStreamCreate(&g_stream));
-  VR_HIP(hipStreamCreate(&g_stream2));
   // this device's copy of the allocation-free bounce's working set
   void *sp = nullptr;
   VR_HIP(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
@@ -1038,9 +1034,12 @@ struct PvsPlan {
   std::vector<vr::PvsEntry> tab;
   std::vector<int64_t> blk_pre;
   int64_t pairs = 0;
+  int32_t chunk = 0;
 };
 
-static int pvs_plan(const int32_t *cl, int64_t np, const uint8_t *rows, int32_t nc, PvsPlan *P) {
+// Blocks take chunk(total candidate pairs) columns.
+static int pvs_plan(const int32_t *cl, int64_t np, const uint8_t *rows, int32_t nc,
+                    int (*chunk)(int64_t), PvsPlan *P) {
   const int32_t ng = nc + 1;  // group nc: patches with a negative cluster
   std::vector<int64_t> goff((size_t)ng + 1, 0);
   for (int64_t i = 0; i < np; ++i) {
@@ -1055,7 +1054,6 @@ static int pvs_plan(const int32_t *cl, int64_t np, const uint8_t *rows, int32_t 
   }
   const int64_t row = ((int64_t)nc + 7) >> 3;
   auto bit = [&](int32_t a, int32_t b) { return (rows[(int64_t)a * row + (b >> 3)] >> (b & 7)) & 1; };
-  const int64_t bc = vr::pvs_block_cols();
   P->tab.clear();
   P->blk_pre.assign(1, 0);
   P->pairs = 0;
@@ -1071,20 +1069,56 @@ static int pvs_plan(const int32_t *cl, int64_t np, const uint8_t *rows, int32_t 
       e.a_n = (int32_t)na;
       e.b_off = (int32_t)goff[(size_t)b];
       e.b_n = (int32_t)nb;
-      e.cpr = (int32_t)((nb + bc - 1) / bc);
       e.diag = a == b;
       P->tab.push_back(e);
-      P->blk_pre.push_back(P->blk_pre.back() + na * e.cpr);
       P->pairs += a == b ? na * (na - 1) / 2 : na * nb;
     }
+  }
+  P->chunk = chunk(P->pairs);
+  for (vr::PvsEntry &e : P->tab) {
+    e.cpr = (int32_t)(((int64_t)e.b_n + P->chunk - 1) / P->chunk);
+    P->blk_pre.push_back(P->blk_pre.back() + (int64_t)e.a_n * e.cpr);
   }
   return VR_OK;
 }
 
-// The CSR of a finished visibility bit matrix: row counts, padded layout,
+// The plan of all pairs (i, j > i): one group, in patch order.
+static PvsPlan one_group(int64_t np) {
+  PvsPlan P;
+  P.pairs = np * (np - 1) / 2;
+  P.chunk = vr::pair_chunk(P.pairs);
+  P.blk_pre.assign(1, 0);
+  if (np > 0) {
+    const int32_t n = (int32_t)np, cpr = (int32_t)((np + P.chunk - 1) / P.chunk);
+    P.tab.push_back(vr::PvsEntry{0, n, 0, n, cpr, 1});
+    P.blk_pre.push_back(np * cpr);
+  }
+  return P;
+}
+
+// S: patches (0-6), the plan's members, table and block prefix (7-9) and the
+// segment counters (10).
+static vr::PairJob pair_job(const DevScene &sc, const DevPatches &dp, const PvsPlan &plan,
+                            const Staging &S, uint32_t *bits, int64_t words) {
+  vr::PairJob j{};
+  j.sc = sc;
+  j.p = dp;
+  j.mem = plan.mem.empty() ? nullptr : S.ptr<int32_t>(7);
+  j.tab = S.ptr<vr::PvsEntry>(8);
+  j.blk_pre = S.ptr<int64_t>(9);
+  j.bits = bits;
+  j.segs = S.ptr<unsigned long long>(10);
+  j.words = words;
+  j.n_tab = (int32_t)plan.tab.size();
+  j.chunk = plan.chunk;
+  return j;
+}
+
+// The CSR of a finished visibility bit matrix (and its segment counters): row counts, padded layout,
 // columns and form factors, then the optional row normalisation.
 static int transfers_from_bits(vr_xfers *x, const DBuf &bits, int64_t words,
-                               const DevPatches &dp, int32_t normalize, hipStream_t st) {
+                               const DevPatches &dp, const unsigned long long *segs,
+                               int32_t normalize, hipStream_t st) {
   const int64_t np = x->n;
   TRY(x->cnt.alloc(4 * (size_t)std::max<int64_t>(np, 1)));
   launch_row_count(bits.as<uint32_t>(), np, words, x->cnt.as<int32_t>(), st);
@@ -1092,7 +1126,11 @@ static int transfers_from_bits(vr_xfers *x, const DBuf &bits, int64_t words,
   x->cnt_host.assign((size_t)np, 0);
   if (np > 0)
     VR_HIP(hipMemcpyAsync(x->cnt_host.data(), x->cnt.p, 4 * (size_t)np, hipMemcpyDeviceToHost, st));
+  unsigned long long seg[vr::kSegCounters];
+  VR_HIP(hipMemcpyAsync(seg, segs, sizeof seg, hipMemcpyDeviceToHost, st));
   VR_HIP(hipStreamSynchronize(st));
+  x->segments = 0;
+  for (unsigned long long v : seg) x->segments += (int64_t)v;
   x->nnz = 0;
   for (int32_t c : x->cnt_host) x->nnz += c;
   TRY(finish_layout(x, st));
@@ -1126,128 +1164,86 @@ static int make_transfers_impl(vr_scene *s, const vr_patches *p, int64_t np,
   const int64_t all_pairs = np * (np - 1) / 2;
   const int64_t cap = std::max<int64_t>(
       std::min<int64_t>(P.batch_pairs > 0 ? P.batch_pairs : (int64_t)32 << 20, all_pairs),
-      std::max<int64_t>(np - 1, nc > 0 ? (int64_t)vr::pvs_block_cols() : 1));
+      std::max<int64_t>(np - 1, nc > 0 ? (int64_t)vr::pvs_chunk(0) : 1));
   if (cap >= (1ll << 31)) return fail(VR_E_INVALID, "batch_pairs too large");
   hipStream_t st = g_stream;
   std::unique_ptr<vr_xfers> x(new vr_xfers);
   x->n = np;
-  const size_t fb = 4 * (size_t)std::max<int64_t>(np, 1);
-  Staging S;
-  TRY(S.make({fb, fb, fb, fb, fb, fb, fb}));
+  const size_t n4 = 4 * (size_t)np, fb = std::max<size_t>(n4, 4);
   const float *src[7] = {p->ox, p->oy, p->oz, p->nx, p->ny, p->nz, p->area};
+  const bool fused = g_path != VR_PATH_PLAIN && s->dev.has_bvh;
+  // the candidate pairs, as blocks of a table's rows (pair_rows)
+  PvsPlan plan;
+  if (nc > 0) {
+    TRY(pvs_plan(cl, np, pvs, nc, fused ? vr::pair_chunk : vr::pvs_chunk, &plan));
+  } else {
+    plan = one_group(np);
+  }
+  x->pairs = plan.pairs;
+  Staging S;
+  const size_t mem_b = 4 * plan.mem.size(), tab_b = sizeof(vr::PvsEntry) * plan.tab.size(),
+               pre_b = 8 * plan.blk_pre.size(), seg_b = 8 * vr::kSegCounters;
+  TRY(S.make({fb, fb, fb, fb, fb, fb, fb, std::max<size_t>(mem_b, 4), std::max<size_t>(tab_b, 4),
+              pre_b, seg_b}));
   g_pin.begin();
   std::vector<HostPart> in;
-  for (int k = 0; k < 7; ++k) in.push_back({k, const_cast<float *>(src[k]), 4 * (size_t)np});
+  for (int k = 0; k < 7; ++k) in.push_back({k, const_cast<float *>(src[k]), n4});
+  in.push_back({7, plan.mem.data(), mem_b});
+  in.push_back({8, plan.tab.data(), tab_b});
+  in.push_back({9, plan.blk_pre.data(), pre_b});
   TRY(S.upload(in, st));
   DevPatches dp{S.ptr<float>(0), S.ptr<float>(1), S.ptr<float>(2), S.ptr<float>(3),
                 S.ptr<float>(4), S.ptr<float>(5), S.ptr<float>(6)};
   const int64_t words = (np + 31) / 32;
-  // The optimised path alternates rounds between two streams, each with its
-  // own pair buffer and count: a round's cull and the start of its trace
-  // run beside the end of the previous round's trace (the launch's tail).
-  // Both set bits of one matrix (atomicOr) and add to one segment total.
-  const int n_sides = g_path == VR_PATH_PLAIN ? 1 : 2;
-  DBuf bits, pairs[2], count[2], segtot;
+  DBuf bits, pairs, count;
   TRY(bits.alloc((size_t)np * (size_t)words * 4));
   VR_HIP(hipMemsetAsync(bits.p, 0, bits.bytes, st));
-  for (int q = 0; q < n_sides; ++q) {
-    TRY(pairs[q].alloc((size_t)cap * sizeof(int2)));
-    TRY(count[q].alloc(4));
+  unsigned long long *const segs = S.ptr<unsigned long long>(10);
+  VR_HIP(hipMemsetAsync(segs, 0, seg_b, st));
+  if (!fused) {
+    TRY(pairs.alloc((size_t)cap * sizeof(int2)));
+    TRY(count.alloc(4));
   }
-  TRY(segtot.alloc(8));
-  VR_HIP(hipMemsetAsync(segtot.p, 0, 8, st));
-  hipStream_t side_st[2] = {st, g_stream2};
-  hipEvent_t ev_start = nullptr, ev_end = nullptr;
-  if (n_sides == 2) {
-    // the second stream starts after the clears on the first, and the first
-    // goes on (CSR build, segment total) after everything on the second
-    VR_HIP(hipEventCreateWithFlags(&ev_start, hipEventDisableTiming));
-    if (hipEventCreateWithFlags(&ev_end, hipEventDisableTiming) != hipSuccess) {
-      (void)hipEventDestroy(ev_start);
-      return fail(VR_E_HIP, "hipEventCreate failed");
-    }
-  }
-  struct Events {
-    hipEvent_t a, b;
-    ~Events() {
-      if (a) (void)hipEventDestroy(a);
-      if (b) (void)hipEventDestroy(b);
-    }
-  } events{ev_start, ev_end};
-  // the second stream waits for everything queued on the first so far (the
-  // clears, the patch and PVS uploads); called before the first round
-  auto start_second = [&]() -> int {
-    if (n_sides == 2) {
-      VR_HIP(hipEventRecord(ev_start, st));
-      VR_HIP(hipStreamWaitEvent(g_stream2, ev_start, 0));
-    }
-    return VR_OK;
-  };
-  int round = 0;
   {
     Prof pr(nc > 0 ? "make_transfers_pvs" : "make_transfers", st);
-    // the buffers and stream of the current round
-    auto side = [&]() { return round % n_sides; };
+    const int64_t n_blk = plan.blk_pre.back();
     auto trace_batch = [&]() {
-      const int q = side();
-      launch_pair_trace(s->dev, dp, pairs[q].as<int2>(), count[q].as<uint32_t>(),
-                        (uint32_t)cap, P.normal_offset, P.skip_id, bits.as<uint32_t>(), words,
-                        g_path, side_st[q]);
-      hipLaunchKernelGGL(k_add_count, dim3(1), dim3(1), 0, side_st[q], count[q].as<uint32_t>(),
-                         (uint32_t)cap, segtot.as<unsigned long long>());
-      ++round;
+      launch_pair_trace(s->dev, dp, pairs.as<int2>(), count.as<uint32_t>(), (uint32_t)cap,
+                        P.normal_offset, P.skip_id, bits.as<uint32_t>(), words, st);
+      hipLaunchKernelGGL(k_add_count, dim3(1), dim3(1), 0, st, count.as<uint32_t>(),
+                         (uint32_t)cap, segs);
       return check_launch();
     };
-    if (nc > 0) {
-      PvsPlan plan;
-      TRY(pvs_plan(cl, np, pvs, nc, &plan));
-      x->pairs = plan.pairs;
-      const int64_t n_blk = plan.blk_pre.back();
-      if (n_blk > 0) {
-        DBuf mem, tab, pre;
-        TRY(mem.upload(plan.mem.data(), 4 * plan.mem.size(), st));
-        TRY(tab.upload(plan.tab.data(), sizeof(vr::PvsEntry) * plan.tab.size(), st));
-        TRY(pre.upload(plan.blk_pre.data(), 8 * plan.blk_pre.size(), st));
-        // a block keeps at most pvs_block_cols() pairs
-        const int64_t per = std::max<int64_t>(1, cap / vr::pvs_block_cols());
-        TRY(start_second());
-        for (int64_t b0 = 0; b0 < n_blk; b0 += per) {
-          const int q = side();
-          VR_HIP(hipMemsetAsync(count[q].p, 0, 4, side_st[q]));
-          launch_pair_cull_pvs(dp, mem.as<int32_t>(), tab.as<vr::PvsEntry>(), pre.as<int64_t>(),
-                               (int32_t)plan.tab.size(), b0, std::min(per, n_blk - b0),
-                               pairs[q].as<int2>(), count[q].as<uint32_t>(), (uint32_t)cap,
-                               side_st[q]);
-          TRY(trace_batch());
-        }
-        // mem / tab / pre are freed on return
-        for (int q = 0; q < n_sides; ++q) VR_HIP(hipStreamSynchronize(side_st[q]));
+    if (fused) {
+      vr::PairJob j = pair_job(s->dev, dp, plan, S, bits.as<uint32_t>(), words);
+      launch_pair_rows(j, n_blk, P.normal_offset, P.skip_id, tuning().trace_lds_entries,
+                       tuning().trace_xcd_group, st);
+      launch_bits_mirror(bits.as<uint32_t>(), np, words, st);
+      TRY(check_launch());
+    } else if (nc > 0) {
+      // a block keeps at most pvs_chunk(0) pairs
+      const int64_t per = std::max<int64_t>(1, cap / vr::pvs_chunk(0));
+      for (int64_t b0 = 0; b0 < n_blk; b0 += per) {
+        VR_HIP(hipMemsetAsync(count.p, 0, 4, st));
+        launch_pair_cull_pvs(dp, S.ptr<int32_t>(7), S.ptr<vr::PvsEntry>(8), S.ptr<int64_t>(9),
+                             (int32_t)plan.tab.size(), b0, std::min(per, n_blk - b0),
+                             pairs.as<int2>(), count.as<uint32_t>(), (uint32_t)cap, st);
+        TRY(trace_batch());
       }
     } else {
-      TRY(start_second());
       int64_t i0 = 0;
       while (i0 + 1 < np) {
         const int64_t rowlen = np - 1 - i0;
         int64_t rows = std::max<int64_t>(1, cap / rowlen);
         const int64_t i1 = std::min<int64_t>(np - 1, i0 + rows);
-        x->pairs += (2 * np - i0 - i1 - 1) * (i1 - i0) / 2;
-        const int q = side();
-        VR_HIP(hipMemsetAsync(count[q].p, 0, 4, side_st[q]));
-        launch_pair_cull(dp, np, i0, i1, pairs[q].as<int2>(), count[q].as<uint32_t>(),
-                         (uint32_t)cap, side_st[q]);
+        VR_HIP(hipMemsetAsync(count.p, 0, 4, st));
+        launch_pair_cull(dp, np, i0, i1, pairs.as<int2>(), count.as<uint32_t>(), (uint32_t)cap,
+                         st);
         TRY(trace_batch());
         i0 = i1;
       }
     }
-    if (n_sides == 2) {
-      VR_HIP(hipEventRecord(ev_end, g_stream2));
-      VR_HIP(hipStreamWaitEvent(st, ev_end, 0));
-    }
-    unsigned long long segs = 0;
-    VR_HIP(hipMemcpyAsync(&segs, segtot.p, 8, hipMemcpyDeviceToHost, st));
-    VR_HIP(hipStreamSynchronize(st));
-    x->segments = (int64_t)segs;
-    TRY(transfers_from_bits(x.get(), bits, words, dp, P.normalize, st));
+    TRY(transfers_from_bits(x.get(), bits, words, dp, segs, P.normalize, st));
   }
   *out = x.release();
   return VR_OK;
@@ -1307,7 +1303,7 @@ int vr_make_transfers_batch(vr_scene *const *scenes, const vr_patches *patches,
   int rc = VR_OK;
   for (int32_t k = 0; k < n_scenes && rc == VR_OK; ++k) {
     const int64_t np = n_patches[k];
-    if (np * (np - 1) / 2 >= budget)
+    if (np * (np - 1) / 2 >= budget || !scenes[k]->dev.has_bvh)
       rc = make_transfers_impl(scenes[k], &patches[k], np, &P, nullptr, nullptr, 0, &out[k]);
     else
       shared.push_back(k);
@@ -1329,106 +1325,61 @@ static int make_transfers_shared(vr_scene *const *scenes, const vr_patches *patc
   hipStream_t st = g_stream;
   const int32_t n_scenes = (int32_t)which.size();
   if (n_scenes == 0) return VR_OK;
-  // every round, each unfinished scene culls its next rows into its own
-  // region of one pair buffer, and the regions' pairs are traced in one
-  // launch.  The round's budget is shared among the scenes still culling
-  // (at least one whole row each), so the rounds do not outlast the small
-  // scenes with small shares.
+  // every scene's rows in one launch, the scenes one after the other
   struct One {
     std::unique_ptr<vr_xfers> x;
     Staging S;
+    PvsPlan plan;
     DevPatches dp{};
     DBuf bits;
-    int64_t np = 0, words = 0, cap = 0, off = 0, i0 = 0;
+    int64_t words = 0;
   };
   std::vector<One> sc((size_t)n_scenes);
-  int64_t total_cap = budget;  // a round's shares plus one row per scene
+  std::vector<vr::PairJob> jobs;
+  int64_t blocks = 0;
+  if (budget >= (1ll << 31)) return fail(VR_E_INVALID, "batch_pairs too large");
   for (int32_t k = 0; k < n_scenes; ++k) {
     One &o = sc[(size_t)k];
     const vr_patches *p = &patches[which[(size_t)k]];
-    o.np = n_patches[which[(size_t)k]];
+    const int64_t np = n_patches[which[(size_t)k]];
     o.x.reset(new vr_xfers);
-    o.x->n = o.np;
-    const size_t fb = 4 * (size_t)std::max<int64_t>(o.np, 1);
-    TRY(o.S.make({fb, fb, fb, fb, fb, fb, fb}));
+    o.x->n = np;
+    o.plan = one_group(np);
+    o.x->pairs = o.plan.pairs;
+    const size_t n4 = 4 * (size_t)np, fb = std::max<size_t>(n4, 4);
+    const size_t tab_b = sizeof(vr::PvsEntry) * o.plan.tab.size(),
+                 pre_b = 8 * o.plan.blk_pre.size(), seg_b = 8 * vr::kSegCounters;
+    TRY(o.S.make({fb, fb, fb, fb, fb, fb, fb, 4, std::max<size_t>(tab_b, 4), pre_b, seg_b}));
     const float *src[7] = {p->ox, p->oy, p->oz, p->nx, p->ny, p->nz, p->area};
-    for (int q = 0; q < 7 && o.np > 0; ++q)
-      VR_HIP(hipMemcpyAsync(o.S.ptr<float>(q), src[q], 4 * (size_t)o.np, hipMemcpyHostToDevice, st));
+    for (int q = 0; q < 7 && np > 0; ++q)
+      VR_HIP(hipMemcpyAsync(o.S.ptr<float>(q), src[q], n4, hipMemcpyHostToDevice, st));
+    if (tab_b)
+      VR_HIP(hipMemcpyAsync(o.S.ptr<char>(8), o.plan.tab.data(), tab_b, hipMemcpyHostToDevice, st));
+    VR_HIP(hipMemcpyAsync(o.S.ptr<char>(9), o.plan.blk_pre.data(), pre_b, hipMemcpyHostToDevice, st));
+    VR_HIP(hipMemsetAsync(o.S.ptr<char>(10), 0, seg_b, st));
     o.dp = DevPatches{o.S.ptr<float>(0), o.S.ptr<float>(1), o.S.ptr<float>(2), o.S.ptr<float>(3),
                       o.S.ptr<float>(4), o.S.ptr<float>(5), o.S.ptr<float>(6)};
-    o.words = (o.np + 31) / 32;
-    TRY(o.bits.alloc((size_t)std::max<int64_t>(o.np, 1) * (size_t)std::max<int64_t>(o.words, 1) * 4));
+    o.words = (np + 31) / 32;
+    TRY(o.bits.alloc((size_t)std::max<int64_t>(np, 1) * (size_t)std::max<int64_t>(o.words, 1) * 4));
     VR_HIP(hipMemsetAsync(o.bits.p, 0, o.bits.bytes, st));
-    if (budget >= (1ll << 31) || o.np - 1 >= (1ll << 31))
-      return fail(VR_E_INVALID, "batch_pairs too large");
-    total_cap += std::max<int64_t>(o.np - 1, 0);
+    if (o.plan.blk_pre.back() == 0) continue;
+    jobs.push_back(pair_job(scenes[which[(size_t)k]]->dev, o.dp, o.plan, o.S,
+                            o.bits.as<uint32_t>(), o.words));
+    jobs.back().blk_begin = blocks;
+    blocks += o.plan.blk_pre.back();
   }
-  DBuf pairs, counts, d_jobs;
-  TRY(pairs.alloc((size_t)std::max<int64_t>(total_cap, 1) * sizeof(int2)));
-  TRY(counts.alloc(4 * (size_t)n_scenes));
-  TRY(d_jobs.alloc(sizeof(TraceJob) * (size_t)n_scenes));
-  std::vector<uint32_t> hc((size_t)n_scenes);
-  std::vector<TraceJob> jobs;
-  const int lds = tuning().trace_lds_entries;
+  DBuf d_jobs;
+  TRY(upload_vec(d_jobs, jobs, st));
   {
     Prof pr("make_transfers", st);
-    for (;;) {
-      bool any = false;
-      int64_t active = 0, off = 0;
-      for (int32_t k = 0; k < n_scenes; ++k) active += sc[(size_t)k].i0 + 1 < sc[(size_t)k].np;
-      const int64_t share = std::max<int64_t>(1, budget / std::max<int64_t>(active, 1));
-      VR_HIP(hipMemsetAsync(counts.p, 0, 4 * (size_t)n_scenes, st));
-      for (int32_t k = 0; k < n_scenes; ++k) {
-        One &o = sc[(size_t)k];
-        if (o.i0 + 1 >= o.np) continue;
-        any = true;
-        const int64_t rowlen = o.np - 1 - o.i0;
-        // share <= budget / active and rowlen <= np - 1, so the regions fit
-        o.cap = std::max<int64_t>(rowlen, share);
-        o.off = off;
-        off += o.cap;
-        const int64_t rows = std::max<int64_t>(1, o.cap / rowlen);
-        const int64_t i1 = std::min<int64_t>(o.np - 1, o.i0 + rows);
-        o.x->pairs += (2 * o.np - o.i0 - i1 - 1) * (i1 - o.i0) / 2;
-        launch_pair_cull(o.dp, o.np, o.i0, i1, pairs.as<int2>() + o.off,
-                         counts.as<uint32_t>() + k, (uint32_t)o.cap, st);
-        o.i0 = i1;
-      }
-      if (!any) break;
-      TRY(check_launch());
-      VR_HIP(hipMemcpyAsync(hc.data(), counts.p, 4 * (size_t)n_scenes, hipMemcpyDeviceToHost, st));
-      VR_HIP(hipStreamSynchronize(st));
-      jobs.clear();
-      int64_t blocks = 0;
-      for (int32_t k = 0; k < n_scenes; ++k) {
-        One &o = sc[(size_t)k];
-        const int64_t c = std::min<int64_t>(hc[(size_t)k], o.cap);
-        if (c <= 0) continue;
-        o.x->segments += c;
-        TraceJob j;
-        j.sc = scenes[which[(size_t)k]]->dev;
-        j.p = o.dp;
-        j.pairs = pairs.as<int2>() + o.off;
-        j.bits = o.bits.as<uint32_t>();
-        j.words = o.words;
-        j.count = c;
-        j.blk_begin = blocks;
-        blocks += (c + 63) / 64;
-        jobs.push_back(j);
-      }
-      if (jobs.empty()) continue;
-      if (blocks >= ((int64_t)1 << 32)) return fail(VR_E_CAPACITY, "too many pairs per launch");
-      VR_HIP(hipMemcpyAsync(d_jobs.p, jobs.data(), sizeof(TraceJob) * jobs.size(),
-                            hipMemcpyHostToDevice, st));
-      launch_pair_trace_jobs(d_jobs.as<TraceJob>(), (int)jobs.size(), blocks, P.normal_offset,
-                             P.skip_id, lds, st);
-      TRY(check_launch());
-      // the job table is rewritten next round: wait for this launch
-      VR_HIP(hipStreamSynchronize(st));
-    }
+    launch_pair_rows_jobs(d_jobs.as<vr::PairJob>(), (int)jobs.size(), blocks, P.normal_offset,
+                          P.skip_id, tuning().trace_lds_entries, st);
+    TRY(check_launch());
     for (int32_t k = 0; k < n_scenes; ++k) {
       One &o = sc[(size_t)k];
-      TRY(transfers_from_bits(o.x.get(), o.bits, o.words, o.dp, P.normalize, st));
+      launch_bits_mirror(o.bits.as<uint32_t>(), o.x->n, o.words, st);
+      TRY(transfers_from_bits(o.x.get(), o.bits, o.words, o.dp, o.S.ptr<unsigned long long>(10),
+                              P.normalize, st));
       o.bits.release();
     }
   }

@@ -98,21 +98,37 @@ void launch_pair_cull(const DevPatches &p, int64_t np, int64_t i0, int64_t i1, i
                       uint32_t *count, uint32_t cap, hipStream_t st);
 void launch_pair_trace(const DevScene &sc, const DevPatches &p, const int2 *pairs,
                        const uint32_t *count, uint32_t cap, float eps, int32_t skip,
-                       uint32_t *bits, int64_t words, int path, hipStream_t st);
-// One scene's candidate pairs in a many-scene visibility launch: blocks
-// [blk_begin, blk_begin + ceil(count / 64)) of the launch trace pairs[0, count)
-// on sc with patches p, setting bits of the scene's N x N matrix (words per row).
-struct TraceJob {
+                       uint32_t *bits, int64_t words, hipStream_t st);
+// A pair of patch groups that see each other: |a| virtual rows of |b|
+// columns, cpr blocks per row; diag = the same group (columns > row only).
+struct PvsEntry {
+  int32_t a_off, a_n, b_off, b_n, cpr, diag;
+};
+// One scene's candidate pairs: table entry k's blocks are [blk_pre[k],
+// blk_pre[k + 1]), a block is one wave and up to `chunk` columns of one row.
+// mem: the patches by group (null: one group, in patch order).  Sets bits of
+// the N x N matrix (words per row) in the table's row direction only, and adds
+// the traced segments to the 64 counters at segs, 8 apart.
+struct PairJob {
   DevScene sc;
   DevPatches p;
-  const int2 *pairs;
+  const int32_t *mem;
+  const PvsEntry *tab;
+  const int64_t *blk_pre;
   uint32_t *bits;
+  unsigned long long *segs;
   int64_t words;
-  int64_t count;
-  int64_t blk_begin;
+  int64_t blk_begin;  // the scene's first block in a launch of many
+  int32_t n_tab, chunk;
 };
-void launch_pair_trace_jobs(const TraceJob *jobs, int n_jobs, int64_t total_blocks, float eps,
-                            int32_t skip, int lds_entries, hipStream_t st);
+constexpr int kSegCounters = 64 * 8;
+int pair_chunk(int64_t pairs);  // columns per block for a total of candidate pairs
+void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip, int lds_entries,
+                      int xcd_group, hipStream_t st);
+void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float eps, int32_t skip,
+                           int lds_entries, hipStream_t st);
+// bits |= transpose(bits)
+void launch_bits_mirror(uint32_t *bits, int64_t np, int64_t words, hipStream_t st);
 void launch_row_count(const uint32_t *bits, int64_t np, int64_t words, int32_t *cnt,
                       hipStream_t st);
 // exclusive scan of padded lengths (multiple of 8) into rp[0..n]
@@ -145,11 +161,6 @@ struct DevBsp {
   const int *nodes;             // planenum, children[0], children[1]
   const int16_t *leaf_cluster;
 };
-// A pair of patch groups that see each other: |a| virtual rows of |b|
-// columns, cpr blocks per row; diag = the same group (columns > row only).
-struct PvsEntry {
-  int32_t a_off, a_n, b_off, b_n, cpr, diag;
-};
 void launch_point_cluster(const DevBsp &b, const float *xyz, int64_t n, int16_t *out,
                           hipStream_t st);
 void launch_patch_cluster(const DevBsp &b, const vr_patch *p, int64_t n, int32_t *out,
@@ -157,7 +168,7 @@ void launch_patch_cluster(const DevBsp &b, const vr_patch *p, int64_t n, int32_t
 void launch_decompress_vis(const uint8_t *vis, int64_t vis_len, const int32_t *ofs, int32_t nc,
                            uint8_t *rows, unsigned long long *overrun, uint32_t *err,
                            hipStream_t st);
-int pvs_block_cols();  // columns one block of the PVS pair cull covers
+int pvs_chunk(int64_t pairs);  // columns per block of the PVS pair cull, whatever the total
 void launch_pair_cull_pvs(const DevPatches &p, const int32_t *mem, const PvsEntry *tab,
                           const int64_t *blk_pre, int32_t n_tab, int64_t blk0, int64_t n_blk,
                           int2 *pairs, uint32_t *count, uint32_t cap, hipStream_t st);

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void k_pair_cull_pvs(DevPatches p, const int32
   }
 }
 
-int pvs_block_cols() { return 256 * kPvsIt; }
+int pvs_chunk(int64_t) { return 256 * kPvsIt; }
 
 void launch_pair_cull_pvs(const DevPatches &p, const int32_t *mem, const PvsEntry *tab,
                           const int64_t *blk_pre, int32_t n_tab, int64_t blk0, int64_t n_blk,

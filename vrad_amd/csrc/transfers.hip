@@ -1,15 +1,18 @@
-// MakeTransfers: patch-pair visibility batches and CSR construction.
+// MakeTransfers: patch-pair visibility and CSR construction.
 //
-//  1. k_pair_cull   candidate pairs (i, j > i) of a row range that pass the
-//                   facing cull, compacted with a wave ballot + one atomic.
-//  2. k_pair_trace  TestLine(o_i + eps n_i -> o_j + eps n_j) per candidate;
-//                   visible pairs set bits (i,j) and (j,i) of an N x N
-//                   bit matrix (N^2/8 bytes: 10 GB at 280k patches, which an
-//                   MI355X holds with room to spare).
+//  1. k_pair_rows   candidate pairs that pass the facing cull, a wave per patch
+//                   and run of columns; TestLine(o_i + eps n_i -> o_j + eps n_j)
+//                   per survivor; visible pairs set bit (i, j) of an N x N bit
+//                   matrix (N^2/8 bytes: 15 GB at 341k patches, which an MI355X
+//                   holds with room to spare).  The plain path lists the pairs
+//                   (k_pair_cull) and traces the list (k_pair_trace_plain).
+//  2. k_bits_mirror makes the matrix symmetric.
 //  3. k_row_count   popcount per row; k_row_scan pads lengths to 8 and scans.
 //  4. k_row_fill    columns in ascending order, F_ij in FP32.
 //  5. k_row_norm    FP64 row sum in the bounce-kernel wave order (G = 4);
 //                   rows with sum > 1 are scaled by 1/sum.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace vr {
@@ -81,33 +84,6 @@ __device__ __forceinline__ void set_pair_bits(uint32_t *bits, int64_t words, int
   atomicOr(bits + (int64_t)j * words + (i >> 5), 1u << (i & 31));
 }
 
-template <int S>
-__global__ __launch_bounds__(64) void k_pair_trace_lds(DevScene sc, DevPatches p,
-                                                       const int2 *__restrict__ pairs,
-                                                       const uint32_t *__restrict__ count,
-                                                       uint32_t cap, float eps, int32_t skip,
-                                                       uint32_t *__restrict__ bits,
-                                                       int64_t words, uint32_t xg) {
-  __shared__ uint32_t s_stk[S * 64];
-  // The grid is sized for cap pairs; only the first ceil(n / 64) blocks have
-  // work.  Blocks are dealt to the XCDs round-robin, so those blocks spread
-  // over all of them, and the XCD-aware remap runs over just those.
-  const uint32_t n = min(*count, cap);
-  const uint32_t nb = (n + 63u) / 64u;
-  if (blockIdx.x >= nb) return;
-  const uint32_t k = xcd_group_chunk(blockIdx.x, nb, xg) * 64 + threadIdx.x;
-  if (k >= n) return;
-  const int2 ij = pairs[k];
-  const int i = ij.x, j = ij.y;
-  BvhSpill<S, uint32_t> spill;
-  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
-  const bool vis = segment_visible(sc, tr, p.ox[i] + eps * p.nx[i],
-                                      p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
-                                      p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
-                                      p.oz[j] + eps * p.nz[j], skip);
-  if (vis) set_pair_bits(bits, words, i, j);
-}
-
 template <int D>
 __global__ __launch_bounds__(256) void k_pair_trace_plain(DevScene sc, DevPatches p,
                                                           const int2 *__restrict__ pairs,
@@ -116,7 +92,9 @@ __global__ __launch_bounds__(256) void k_pair_trace_plain(DevScene sc, DevPatche
                                                           uint32_t *__restrict__ bits,
                                                           int64_t words) {
   const uint32_t n = min(*count, cap);
-  const uint32_t nb = (n + 255u) / 256u;  // blocks with work (see k_pair_trace_lds)
+  // the grid is sized for cap pairs; only the first ceil(n / 256) blocks have
+  // work, and the XCD-aware remap runs over just those
+  const uint32_t nb = (n + 255u) / 256u;
   if (blockIdx.x >= nb) return;
   const uint32_t k = xcd_chunk(blockIdx.x, nb) * 256 + threadIdx.x;
   if (k >= n) return;
@@ -132,80 +110,269 @@ __global__ __launch_bounds__(256) void k_pair_trace_plain(DevScene sc, DevPatche
 
 void launch_pair_trace(const DevScene &sc, const DevPatches &p, const int2 *pairs,
                        const uint32_t *count, uint32_t cap, float eps, int32_t skip,
-                       uint32_t *bits, int64_t words, int path, hipStream_t st) {
+                       uint32_t *bits, int64_t words, hipStream_t st) {
   if (cap == 0) return;
-  if (path == VR_PATH_PLAIN || !sc.has_bvh)
-    hipLaunchKernelGGL(k_pair_trace_plain<kStackDepth>, dim3((cap + 255) / 256), dim3(256), 0, st,
-                       sc, p, pairs, count, cap, eps, skip, bits, words);
-  else {
-    // the traversal-stack entries kept in LDS follow the autotuned knob
-#define VR_PAIR_TRACE(S)                                                                    \
-  hipLaunchKernelGGL((k_pair_trace_lds<S>), dim3((cap + 63) / 64), dim3(64), 0, st, \
-                     sc, p, pairs, count, cap, eps, skip, bits, words,                          \
-                     (uint32_t)tuning().trace_xcd_group)
-    switch (tuning().trace_lds_entries) {
-      case 2: VR_PAIR_TRACE(2); break;
-      case 4: VR_PAIR_TRACE(4); break;
-      case 6: VR_PAIR_TRACE(6); break;
-      case 10: VR_PAIR_TRACE(10); break;
-      case 12: VR_PAIR_TRACE(12); break;
-      case 16: VR_PAIR_TRACE(16); break;
-      case 24: VR_PAIR_TRACE(24); break;
-      default: VR_PAIR_TRACE(8); break;
-    }
-#undef VR_PAIR_TRACE
-  }
+  hipLaunchKernelGGL(k_pair_trace_plain<kStackDepth>, dim3((cap + 255) / 256), dim3(256), 0, st,
+                     sc, p, pairs, count, cap, eps, skip, bits, words);
 }
 
-// Many scenes' candidate pairs in one launch: block b (after the XCD remap)
-// belongs to the job whose block range holds it (binary search over the
-// jobs' first blocks; the job index is the same for the whole wave, so its
-// descriptor comes through scalar loads), and lane l traces that job's pair
-// (b - first block) * 64 + l on the job's scene.
+// Candidate pairs of one or many scenes, culled and traced in one launch.  A
+// wave takes one patch i and up to `chunk` columns j of its row (one group of
+// patches against another, or all patches against all): 64 columns at a time
+// pass the facing cull, the survivors' end points queue up in LDS, and 64 of
+// them are traced together once they are there.  Bound by the walk: vector
+// issue and the vector cache are each some 70 % busy.  The 8x8-room level's
+// 2.57 G segments take 166 ms, 250 as rounds of list, trace and two atomics
+// per visible pair.
+//  - Segments of one wave share an end point and run to neighbouring patches.
+//  - No pair list: it took 41 GB of traffic, 512 MB, and a hundred launches,
+//    each with a tail.
+//  - A wave sets its bits in row i alone, one atomic per word of 32 columns and
+//    64 segments (two waves can meet in a word); k_bits_mirror then makes the
+//    matrix symmetric.  An atomic per visible pair and direction was 3.2 G
+//    atomics, half of them one per cache line.
 template <int S>
-__global__ __launch_bounds__(64) void k_pair_trace_jobs(const TraceJob *__restrict__ jobs,
-                                                        int n_jobs, float eps, int32_t skip) {
+__device__ __forceinline__ void pair_rows(const PairJob &J, int64_t gb, float eps, int32_t skip,
+                                          uint32_t *s_stk, float4 *s_q, uint32_t *s_w) {
+  int lo = 0, hi = J.n_tab - 1;
+  while (lo < hi) {  // the entry whose blocks hold gb
+    const int mid = (lo + hi + 1) >> 1;
+    if (J.blk_pre[mid] <= gb) lo = mid;
+    else hi = mid - 1;
+  }
+  const PvsEntry e = J.tab[lo];
+  const int64_t local = gb - J.blk_pre[lo];
+  const int ia = (int)(local / e.cpr);
+  int col = (int)(local - (int64_t)ia * e.cpr) * J.chunk + (e.diag ? ia + 1 : 0);
+  const int end = min(e.b_n, col + J.chunk);
+  if (col >= end) return;
+  const DevPatches &p = J.p;
+  const int lane = (int)threadIdx.x;
+  const int32_t *const mem = J.mem ? J.mem + e.b_off : nullptr;
+  const int i = J.mem ? J.mem[e.a_off + ia] : ia;
+  const float ix = p.ox[i], iy = p.oy[i], iz = p.oz[i];
+  const float inx = p.nx[i], iny = p.ny[i], inz = p.nz[i];
+  const float px = ix + eps * inx, py = iy + eps * iny, pz = iz + eps * inz;
+  // the next 64 columns, loaded ahead of their use
+  int j = -1;
+  float jx = 0, jy = 0, jz = 0, jnx = 0, jny = 0, jnz = 0;
+  auto fetch = [&](int at) {
+    const int c = at + lane;
+    j = c < end ? (mem ? mem[c] : c) : -1;
+    if (j >= 0) {
+      jx = p.ox[j], jy = p.oy[j], jz = p.oz[j];
+      jnx = p.nx[j], jny = p.ny[j], jnz = p.nz[j];
+    }
+  };
+  fetch(col);
+  const uint64_t below = (1ull << lane) - 1ull;
+  uint32_t head = 0, qn = 0, total = 0;  // survivors queued at [head, head + qn) mod 128
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(J.sc, s_stk, lane, spill);
+  uint32_t *const row = J.bits + (int64_t)i * J.words;
+  for (;;) {
+    while (qn < 64u && col < end) {
+      // the segment runs from the smaller patch index to the larger
+      const bool ij = i < j;
+      const float rx = ij ? ix : jx, ry = ij ? iy : jy, rz = ij ? iz : jz;
+      const float qx = ij ? inx : jnx, qy = ij ? iny : jny, qz = ij ? inz : jnz;
+      const float sx = ij ? jx : ix, sy = ij ? jy : iy, sz = ij ? jz : iz;
+      const float tx = ij ? jnx : inx, ty = ij ? jny : iny, tz = ij ? jnz : inz;
+      const float dx = sx - rx, dy = sy - ry, dz = sz - rz;
+      const float di = (qx * dx + qy * dy) + qz * dz;
+      const float dj = -((tx * dx + ty * dy) + tz * dz);
+      const bool keep = j >= 0 && di > 0.0f && dj > 0.0f;
+      const uint64_t m = __ballot(keep);
+      if (keep)
+        s_q[(head + qn + (uint32_t)__popcll(m & below)) & 127u] =
+            make_float4(jx + eps * jnx, jy + eps * jny, jz + eps * jnz, __int_as_float(j));
+      qn += (uint32_t)__popcll(m);
+      col += 64;
+      fetch(col);
+    }
+    const uint32_t n = min(qn, 64u);
+    if (n == 0) break;
+    __syncthreads();  // one wave: the queue is written before it is read
+    const bool ray = (uint32_t)lane < n;
+    const float4 q = s_q[(head + (uint32_t)lane) & 127u];
+    const int jj = __float_as_int(q.w);
+    const bool ij = i < jj;
+    const bool vis =
+        ray && segment_visible(J.sc, tr, ij ? px : q.x, ij ? py : q.y, ij ? pz : q.z,
+                               ij ? q.x : px, ij ? q.y : py, ij ? q.z : pz, skip);
+    head = (head + n) & 127u;
+    qn -= n;
+    total += n;
+    // columns ascend, so a word's lanes are neighbours: they meet in the LDS
+    // word of their run, which the run's first lane adds to the matrix
+    const int w = jj >> 5;
+    const int wl = __shfl_up(w, 1);
+    const uint64_t heads = __ballot(ray && (lane == 0 || w != wl));
+    const int run = __popcll(heads & (below | (1ull << lane))) - 1;
+    s_w[lane] = 0u;
+    __syncthreads();
+    if (vis) atomicOr(&s_w[run], 1u << (jj & 31));
+    __syncthreads();
+    if ((heads >> lane) & 1ull) {
+      const uint32_t v = s_w[run];
+      if (v) atomicOr(row + w, v);
+    }
+  }
+  // 64 counters, 64 bytes apart
+  if (lane == 0 && total)
+    atomicAdd(J.segs + 8 * (blockIdx.x & 63u), (unsigned long long)total);
+}
+
+// 6 waves per SIMD: 186 ms on the level, 189 with 5, 198 with 8 (and spills)
+template <int S>
+__global__ __launch_bounds__(64, 6) void k_pair_rows(PairJob job, int64_t blk0, float eps,
+                                                  int32_t skip, uint32_t xg) {
   __shared__ uint32_t s_stk[S * 64];
-  const int64_t b = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
+  __shared__ float4 s_q[128];
+  __shared__ uint32_t s_w[64];
+  pair_rows<S>(job, blk0 + xcd_group_chunk(blockIdx.x, gridDim.x, xg), eps, skip, s_stk, s_q,
+               s_w);
+}
+
+// Block b (after the XCD remap) belongs to the job whose block range holds it
+// (binary search over the jobs' first blocks; the index is the same for the
+// whole wave, so the descriptor comes through scalar loads).
+template <int S>
+__global__ __launch_bounds__(64, 6) void k_pair_rows_jobs(const PairJob *__restrict__ jobs,
+                                                       int n_jobs, int64_t blk0, float eps,
+                                                       int32_t skip) {
+  __shared__ uint32_t s_stk[S * 64];
+  __shared__ float4 s_q[128];
+  __shared__ uint32_t s_w[64];
+  const int64_t b = blk0 + xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
   int lo = 0, hi = n_jobs - 1;
   while (lo < hi) {  // last job with blk_begin <= b
     const int mid = (lo + hi + 1) >> 1;
     if (jobs[mid].blk_begin <= b) lo = mid;
     else hi = mid - 1;
   }
-  const int jx = __builtin_amdgcn_readfirstlane(lo);
-  const TraceJob &J = jobs[jx];
-  const int64_t k = (b - J.blk_begin) * 64 + threadIdx.x;
-  if (k >= (int64_t)J.count) return;
-  const int2 ij = J.pairs[k];
-  const int i = ij.x, j = ij.y;
-  const DevPatches &p = J.p;
-  BvhSpill<S, uint32_t> spill;
-  BvhTracer<S, uint32_t> tr(J.sc, s_stk, (int)threadIdx.x, spill);
-  const bool vis = segment_visible(J.sc, tr, p.ox[i] + eps * p.nx[i],
-                                      p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
-                                      p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
-                                      p.oz[j] + eps * p.nz[j], skip);
-  if (vis) set_pair_bits(J.bits, J.words, i, j);
+  const PairJob &J = jobs[__builtin_amdgcn_readfirstlane(lo)];
+  pair_rows<S>(J, b - J.blk_begin, eps, skip, s_stk, s_q, s_w);
 }
 
-void launch_pair_trace_jobs(const TraceJob *jobs, int n_jobs, int64_t total_blocks, float eps,
-                            int32_t skip, int lds_entries, hipStream_t st) {
-  if (n_jobs <= 0 || total_blocks <= 0) return;
-#define VR_PT_JOBS(S)                                                                          \
-  hipLaunchKernelGGL((k_pair_trace_jobs<S>), dim3((unsigned)total_blocks), dim3(64), \
-                     0, st, jobs, n_jobs, eps, skip)
-  switch (lds_entries) {
-    case 2: VR_PT_JOBS(2); break;
-    case 4: VR_PT_JOBS(4); break;
-    case 6: VR_PT_JOBS(6); break;
-    case 10: VR_PT_JOBS(10); break;
-    case 12: VR_PT_JOBS(12); break;
-    case 16: VR_PT_JOBS(16); break;
-    case 24: VR_PT_JOBS(24); break;
-    default: VR_PT_JOBS(8); break;
+// Columns per wave.  Long rows waste less of their last 64 segments, short
+// ones fill the chip: 16 K waves or more, of 256 to 8192 columns.
+int pair_chunk(int64_t pairs) {
+  const int64_t c = (pairs / 16384 + 63) / 64 * 64;
+  return (int)std::min<int64_t>(8192, std::max<int64_t>(256, c));
+}
+
+// the traversal-stack entries kept in LDS follow the autotuned knob
+#define VR_BY_LDS(X)                                                                       \
+  switch (lds_entries) {                                                                   \
+    case 2: X(2); break;                                                                   \
+    case 4: X(4); break;                                                                   \
+    case 6: X(6); break;                                                                   \
+    case 10: X(10); break;                                                                 \
+    case 12: X(12); break;                                                                 \
+    case 16: X(16); break;                                                                 \
+    case 24: X(24); break;                                                                 \
+    default: X(8); break;                                                                  \
   }
-#undef VR_PT_JOBS
+constexpr int64_t kGridMax = (int64_t)1 << 24;  // workgroups per launch
+
+void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip, int lds_entries,
+                      int xcd_group, hipStream_t st) {
+  for (int64_t b = 0; b < n_blk; b += kGridMax) {
+    const dim3 grid((unsigned)std::min(kGridMax, n_blk - b));
+#define VR_ROWS(S)                                                                        \
+  hipLaunchKernelGGL((k_pair_rows<S>), grid, dim3(64), 0, st, job, b, eps, skip, (uint32_t)xcd_group)
+    VR_BY_LDS(VR_ROWS)
+#undef VR_ROWS
+  }
+}
+
+void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float eps, int32_t skip,
+                           int lds_entries, hipStream_t st) {
+  for (int64_t b = 0; n_jobs > 0 && b < n_blk; b += kGridMax) {
+    const dim3 grid((unsigned)std::min(kGridMax, n_blk - b));
+#define VR_ROWS(S) \
+  hipLaunchKernelGGL((k_pair_rows_jobs<S>), grid, dim3(64), 0, st, jobs, n_jobs, b, eps, skip)
+    VR_BY_LDS(VR_ROWS)
+#undef VR_ROWS
+  }
+}
+
+// bits |= transpose(bits), in place.  A workgroup takes a tile of 512 x 512
+// bits and its mirror image (64-byte row pieces, so whole memory accesses):
+// both go to LDS (rows 17 words apart: a column of words lies in 32 banks),
+// half-waves exchange 32 x 32 bit blocks, transposed in 5 steps of the half a
+// lane pairs up with, and the tiles go back if any bit is set.  Bound by
+// reading the matrix once.
+constexpr int kMirror = 512, kMirrorW = kMirror / 32, kMirrorS = kMirrorW + 1;
+
+__device__ __forceinline__ uint32_t transpose32(uint32_t x, int l) {
+  // rows and columns whose numbers differ in bit s change places, for each s
+  uint32_t m = 0x0000ffffu;
+#pragma unroll
+  for (int s = 16; s >= 1; s >>= 1, m ^= m << s) {
+    const uint32_t y = __shfl_xor(x, s);
+    x = (l & s) ? (x & ~m) | ((y >> s) & m) : (x & m) | ((y & m) << s);
+  }
+  return x;
+}
+
+__global__ __launch_bounds__(256) void k_bits_mirror(uint32_t *__restrict__ bits, int64_t np,
+                                                     int64_t words, uint32_t nt) {
+  __shared__ uint32_t s_a[kMirror * kMirrorS], s_b[kMirror * kMirrorS];
+  // tile (r, c), r <= c, of the upper triangle's row-by-row enumeration
+  // folded in two: row r of the fold holds tiles (r, r..) and (nt-1-r, ..)
+  const uint32_t w = nt + 1, f = blockIdx.x / w, x = blockIdx.x % w;
+  uint32_t r = f, c = f + x;
+  if (c >= nt) {
+    r = nt - 1 - f;
+    c = r + (x - (nt - f));
+    if (r == f) return;  // the middle row of an odd count stands alone
+  }
+  const int64_t ra = (int64_t)r * kMirror, rb = (int64_t)c * kMirror;
+  const int64_t wa = (int64_t)c * kMirrorW, wb = (int64_t)r * kMirrorW;
+  const int t = (int)threadIdx.x, col = t & (kMirrorW - 1);
+  const bool diag = r == c;
+  uint32_t any = 0;
+#pragma unroll 8
+  for (int k = t / kMirrorW; k < kMirror; k += 256 / kMirrorW) {
+    const uint32_t a = ra + k < np && wa + col < words ? bits[(ra + k) * words + wa + col] : 0u;
+    const uint32_t b =
+        !diag && rb + k < np && wb + col < words ? bits[(rb + k) * words + wb + col] : 0u;
+    s_a[k * kMirrorS + col] = a;
+    s_b[k * kMirrorS + col] = b;
+    any |= a | b;
+  }
+  if (!__syncthreads_or((int)any)) return;
+  uint32_t *const s_m = diag ? s_a : s_b;
+  const int half = t >> 5, l = t & 31;
+  for (int q = half; q < kMirrorW * kMirrorW; q += 8) {
+    const int br = q / kMirrorW, bc = q % kMirrorW;
+    // both halves of a wave run the shuffles; of a diagonal tile's block pair
+    // only one writes
+    uint32_t *const pa = s_a + (32 * br + l) * kMirrorS + bc;
+    uint32_t *const pb = s_m + (32 * bc + l) * kMirrorS + br;
+    const uint32_t a = *pa | transpose32(*pb, l);
+    const uint32_t b = transpose32(a, l);
+    if (!diag || br <= bc) {
+      *pb = b;
+      *pa = a;
+    }
+  }
+  __syncthreads();
+#pragma unroll 8
+  for (int k = t / kMirrorW; k < kMirror; k += 256 / kMirrorW) {
+    if (ra + k < np && wa + col < words) bits[(ra + k) * words + wa + col] = s_a[k * kMirrorS + col];
+    if (!diag && rb + k < np && wb + col < words)
+      bits[(rb + k) * words + wb + col] = s_b[k * kMirrorS + col];
+  }
+}
+
+void launch_bits_mirror(uint32_t *bits, int64_t np, int64_t words, hipStream_t st) {
+  if (np <= 0) return;
+  const uint32_t nt = (uint32_t)((np + kMirror - 1) / kMirror);
+  const uint32_t grid = (nt + 1) / 2 * (nt + 1);
+  hipLaunchKernelGGL(k_bits_mirror, dim3(grid), dim3(256), 0, st, bits, np, words, nt);
 }
 
 // one wave per row
