@@ -164,7 +164,7 @@ __device__ void gather_group(const DevScene &sc, Tracer &tr, int wave, bool live
 }
 
 template <int S, int W>
-__global__ __launch_bounds__(64 * W) void k_gather_lds(DevScene sc, DevSamples s, int64_t n,
+__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_lds(DevScene sc, DevSamples s, int64_t n,
                                                        const vr_light *__restrict__ lights,
                                                        int32_t n_lights,
                                                        const float *__restrict__ dirs, float eps,
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void k_gather_plain(DevScene sc, DevSamples s,
 // uniform per wave), and lane l gathers that job's sample
 // (b - first block) * 64 + l from the job's scene and lights.
 template <int S, int W>
-__global__ __launch_bounds__(64 * W) void k_gather_jobs(const GatherJob *__restrict__ jobs,
+__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_jobs(const GatherJob *__restrict__ jobs,
                                                         int n_jobs,
                                                         const float *__restrict__ dirs, float eps,
                                                         int32_t skip) {

@@ -429,11 +429,17 @@ struct KdTracer {
 // (k_bvh_bounds); an origin farther out widens the slabs by 96 u (|o| - M)
 // here.  A direction component of 0 counts as +-1e-20.
 //
-// While the wave's walking lanes are at the same node and share their signs
-// (most steps near the root for rays that start close together), the node
-// comes through scalar loads: a vector load of one address still takes the
-// vector cache 16 cycles, 112 per node, which was 81 % busy on the level's
-// TestLine batch.
+// While the wave's walking lanes are at the same node (most steps near the
+// root for rays that start close together), the node comes through scalar
+// loads: a vector load of one address still takes the vector cache 16 cycles,
+// 112 per node, which was 81 % busy on the level's TestLine batch.  Lanes of
+// several octants then sort each axis's two times, 24 instructions more: with
+// one octant alone (about half of MakeTransfers' waves) the level's pair trace
+// took 186 ms against 166, the closest hits 205 us against 188.
+//
+// A wave that walks as one (a node visited when any of its rays enters it,
+// nothing but scalar loads, the stack in a register) was slower: 28 steps for
+// 64 pair segments and 3100 instead of 1250 vector instructions, 300 ms.
 typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
 typedef float f32v4 __attribute__((ext_vector_type(4)));
 struct Planes {
@@ -466,7 +472,9 @@ struct BvhTracer {
   float ox, oy, oz, dx, dy, dz;
   float ix, iy, iz, nx, ny, nz, fx, fy, fz;
   uint32_t sx, sy, sz;  // byte offset of the near planes in a node, by axis
-  bool oct;             // the wave's rays (those set up together) share their signs
+  bool uni;             // scalar node loads will do (all rays set up together): one
+                        // octant, or no origin beyond M (nx == fx, so that either
+                        // plane of an axis can be the near one)
   __device__ BvhTracer(const DevScene &s, E *lds, int lane, BvhSpill<S, E> &sp)
       : sc(s), st(lds, lane, sp) {}
   __device__ __forceinline__ void begin(float ox_, float oy_, float oz_, float dx_, float dy_,
@@ -492,7 +500,8 @@ struct BvhTracer {
     sy = (__float_as_uint(iy) >> 31) << 4;
     sz = (__float_as_uint(iz) >> 31) << 4;
     const uint32_t o = sx | (sy << 1) | (sz << 2);
-    oct = __ballot(o != (uint32_t)__builtin_amdgcn_readfirstlane((int)o)) == 0;
+    uni = __ballot(o != (uint32_t)__builtin_amdgcn_readfirstlane((int)o)) == 0 ||
+          __ballot(e != 0.0f) == 0;
   }
   template <bool ANY, bool SKIPSKY>
   __device__ __forceinline__ bool full(float tmin, int32_t skip, float &tbest, int32_t &best,
@@ -537,25 +546,15 @@ struct BvhTracer {
         }
         return kDone;
       } else {
-        return sp > 0 ? st.get(--sp) : kDone;
+        --sp;
+        if (__ballot(sp >= S) == 0) return st.e[64 * sp];
+        return st.get(sp);
       }
     };
+    if constexpr (!kKeyed) st.push(sp++, kDone);  // the last entry popped
     // the children a ray enters: the next one to visit, the others stacked
-    auto step = [&](const Planes &n) -> uint32_t {
-      auto enter = [&](float a, float b, float c) {
-        return fmaxf(fmaxf(__builtin_fmaf(a, ix, nx), __builtin_fmaf(b, iy, ny)),
-                     fmaxf(__builtin_fmaf(c, iz, nz), tmin));
-      };
-      auto leave = [&](float a, float b, float c) {
-        return fminf(fminf(__builtin_fmaf(a, ix, fx), __builtin_fmaf(b, iy, fy)),
-                     fminf(__builtin_fmaf(c, iz, fz), tbest));
-      };
-      const float t0 = enter(n.ax.x, n.ay.x, n.az.x), t1 = enter(n.ax.y, n.ay.y, n.az.y),
-                  t2 = enter(n.ax.z, n.ay.z, n.az.z), t3 = enter(n.ax.w, n.ay.w, n.az.w);
-      const bool h0 = t0 <= leave(n.bx.x, n.by.x, n.bz.x),
-                 h1 = t1 <= leave(n.bx.y, n.by.y, n.bz.y),
-                 h2 = t2 <= leave(n.bx.z, n.by.z, n.bz.z),
-                 h3 = t3 <= leave(n.bx.w, n.by.w, n.bz.w);
+    auto take = [&](bool h0, bool h1, bool h2, bool h3, float t0, float t1, float t2, float t3,
+                    const u32v4 &ch) -> uint32_t {
       if constexpr (kKeyed) {
         constexpr uint32_t kMiss = 0xffffffffu;
         auto key = [](bool h, float t, uint32_t k) {
@@ -574,7 +573,7 @@ struct BvhTracer {
         order(k1, k3);
         order(k1, k2);
         auto child = [&](uint32_t k) {
-          const uint32_t a = (k & 1u) ? n.ch.y : n.ch.x, b = (k & 1u) ? n.ch.w : n.ch.z;
+          const uint32_t a = (k & 1u) ? ch.y : ch.x, b = (k & 1u) ? ch.w : ch.z;
           return (k & 2u) ? b : a;
         };
         auto entry = [&](uint32_t k) { return ((uint64_t)k << 32) | child(k); };
@@ -583,39 +582,70 @@ struct BvhTracer {
         if (k1 != kMiss) st.push(sp++, entry(k1));
         return k0 != kMiss ? child(k0) : pop();
       } else {
-        uint32_t next = kDone;
-        auto take = [&](bool h, uint32_t c) {
-          if (h) {
-            if (next != kDone) st.push(sp++, next);
-            next = c;
-          }
-        };
-        take(h0, n.ch.x);
-        take(h1, n.ch.y);
-        take(h2, n.ch.z);
-        take(h3, n.ch.w);
-        return next != kDone ? next : pop();
+        // the last child entered is next, the ones before it are stacked; with
+        // room for three more in LDS in every lane, without a look at each
+        const bool p0 = h0 && (h1 || h2 || h3), p1 = h1 && (h2 || h3), p2 = h2 && h3;
+        const uint32_t next = h3 ? ch.w : h2 ? ch.z : h1 ? ch.y : ch.x;
+        if (__ballot(sp > S - 3) == 0) {
+          if (p0) st.e[64 * sp++] = ch.x;
+          if (p1) st.e[64 * sp++] = ch.y;
+          if (p2) st.e[64 * sp++] = ch.z;
+        } else {
+          if (p0) st.push(sp++, ch.x);
+          if (p1) st.push(sp++, ch.y);
+          if (p2) st.push(sp++, ch.z);
+        }
+        return h0 || h1 || h2 || h3 ? next : pop();
+      }
+    };
+    float t[4];
+    bool h[4];
+    auto box = [&](int k, float xn, float xf, float yn, float yf, float zn, float zf) {
+      t[k] = fmaxf(fmaxf(xn, yn), fmaxf(zn, tmin));
+      h[k] = t[k] <= fminf(fminf(xf, yf), fminf(zf, tbest));
+    };
+    auto boxes = [&](const Planes &n) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        box(k, __builtin_fmaf(n.ax[k], ix, nx), __builtin_fmaf(n.bx[k], ix, fx),
+            __builtin_fmaf(n.ay[k], iy, ny), __builtin_fmaf(n.by[k], iy, fy),
+            __builtin_fmaf(n.az[k], iz, nz), __builtin_fmaf(n.bz[k], iz, fz));
+    };
+    // lanes of several octants (nx == fx and so on): each takes the nearer
+    // plane's time per axis; a missing child's planes are swapped, so that its
+    // box would be all of space
+    auto boxes_mixed = [&](const Planes &n) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float xa = __builtin_fmaf(n.ax[k], ix, nx), xb = __builtin_fmaf(n.bx[k], ix, nx),
+                    ya = __builtin_fmaf(n.ay[k], iy, ny), yb = __builtin_fmaf(n.by[k], iy, ny),
+                    za = __builtin_fmaf(n.az[k], iz, nz), zb = __builtin_fmaf(n.bz[k], iz, nz);
+        box(k, fminf(xa, xb), fmaxf(xa, xb), fminf(ya, yb), fmaxf(ya, yb), fminf(za, zb),
+            fmaxf(za, zb));
+        h[k] = h[k] && n.ch[k] != kBvhLeaf;
       }
     };
     for (;;) {
       while (!(cur & kBvhLeaf)) {
         Planes n;
         const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)cur);
-        if (oct && __ballot(cur != u) == 0) {
+        if (uni && __ballot(cur != u) == 0) {
           const auto *q = (const __attribute__((address_space(4))) char *)(base + ((size_t)u << 7));
           const uint32_t ux = (uint32_t)__builtin_amdgcn_readfirstlane((int)sx),
                          uy = (uint32_t)__builtin_amdgcn_readfirstlane((int)sy),
                          uz = (uint32_t)__builtin_amdgcn_readfirstlane((int)sz);
           n.load(q + ux, q + (ux ^ 16u), q + 32 + uy, q + 32 + (uy ^ 16u), q + 64 + uz,
                  q + 64 + (uz ^ 16u), q + 96);
-          cur = step(n);
+          if (__ballot(sx != ux || sy != uy || sz != uz) == 0) boxes(n);
+          else boxes_mixed(n);
         } else {
           const uint32_t at = cur << 7;
           const uint32_t px = at | sx, py = at | sy, pz = at | sz;
           n.load(base + px, base + (px ^ 16u), base + py + 32, base + (py ^ 16u) + 32,
                  base + pz + 64, base + (pz ^ 16u) + 64, base + at + 96);
-          cur = step(n);
+          boxes(n);
         }
+        cur = take(h[0], h[1], h[2], h[3], t[0], t[1], t[2], t[3], n.ch);
       }
       if (cur == kDone) break;
       const uint32_t first = cur & kBvhFirstMask, cnt = (cur & ~kBvhLeaf) >> kBvhCntShift;
