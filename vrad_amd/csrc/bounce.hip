@@ -992,67 +992,94 @@ __global__ __launch_bounds__(1024) void k_block_offsets(DevXfers x, DevTiles tl,
 // Blocked layout, pass 2: copy each owner's segment with its columns turned
 // into LDS byte offsets ostride (col - t C) (stream layout: 16 emit_slot(col
 // - t C)), bit 0 set on the segment's first entry; pad with (offset 0,
-// coef 0).  One wave per (block, gather wave w): it copies the segments of
-// w's 64 owner slots one after another, each with all 64 lanes.
-__global__ __launch_bounds__(256) void k_block_fill(DevXfers x, DevTiles tl, int G,
+// coef 0).  One wave per `slots` (4 or 16) of a block's owner slots: its lanes
+// look up the segments side by side, then all 64 copy them one after another,
+// in the stream layout a chunk of 4 entries per lane with one store of
+// offsets and one of coefficients.  Bound by latency and, before chunks per
+// lane, by index arithmetic: entry by entry with a wave per 64 slots 5,970
+// rows of 3.2 M transfers took 116 us (now 45), 341,299 rows of 1.56 G 10.4 ms
+// (now 8.4).
+__global__ __launch_bounds__(256) void k_block_fill(DevXfers x, DevTiles tl, int slots,
                                                     int coef_bytes, uint16_t *__restrict__ bidx,
                                                     void *__restrict__ bcoef) {
   const int lane = threadIdx.x & 63;
-  const int R = 1024, RS = R + 4;
+  const int R = 1024, RS = R + 4, nw = R / slots;
   const int64_t gw = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t nblk = tl.n_chunks * (int64_t)tl.nt;
-  if (gw >= nblk * 16) return;
-  const int64_t blk = gw / 16;
-  const int w = (int)(gw % 16);
+  if (gw >= nblk * nw) return;
+  const int64_t blk = gw / nw;
+  const int u0 = (int)(gw % nw) * slots, w = u0 / 64;
   const int64_t c = blk / tl.nt;
   const int t = (int)(blk % tl.nt);
-  for (int j = 0; j < 64; ++j) {
-    const int u = 64 * w + j;
-    const int64_t oi = c + slot_rank(w, j) * tl.n_chunks;
-    if (oi >= x.n) continue;
-    const int64_t row = x.order[oi];
-    const int32_t *tp = tl.tp + row * (int64_t)(tl.nt + 1);
-    const int64_t src = x.rp[row] + tp[t];
-    const int len = tp[t + 1] - tp[t];
-    const int32_t *bo = tl.boff + blk * RS;
-    const int64_t dst = tl.bstart[blk] + bo[u];
-    const int plen = bo[u + 1] - bo[u];
-    const int p0 = t * tl.cols;
-    const int ss = bo[u] - bo[64 * w];  // the segment's start in the wave's stream
-    const int wlen = bo[64 * w + 64] - bo[64 * w];
-    const int nch = plen / G;
-    for (int q = lane; q < plen; q += 64) {
+  const int32_t *bo = tl.boff + blk * RS;
+  const int w0 = bo[64 * w], wlen = bo[64 * w + 64] - w0;
+  const int64_t bstart = tl.bstart[blk];
+  const int p0 = t * tl.cols;
+  int64_t l_src = 0;
+  int l_len = 0, l_bo = 0, l_plen = 0;
+  if (lane < slots) {
+    const int u = u0 + lane;
+    const int64_t oi = c + slot_rank(w, u & 63) * tl.n_chunks;
+    if (oi < x.n) {
+      const int64_t row = x.order[oi];
+      const int32_t *tp = tl.tp + row * (int64_t)(tl.nt + 1);
+      l_src = x.rp[row] + tp[t];
+      l_len = tp[t + 1] - tp[t];
+      l_bo = bo[u];
+      l_plen = bo[u + 1] - l_bo;
+    }
+  }
+  for (uint64_t m = __ballot(l_plen != 0); m; m &= m - 1ull) {
+    const int k = __ffsll((unsigned long long)m) - 1;
+    const int j = (u0 + k) & 63;
+    const int64_t src = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(l_src >> 32), k) << 32) |
+                                  (uint32_t)__builtin_amdgcn_readlane((int)l_src, k));
+    const int len = __builtin_amdgcn_readlane(l_len, k);
+    const int bu = __builtin_amdgcn_readlane(l_bo, k);
+    const int plen = __builtin_amdgcn_readlane(l_plen, k);
+    const int64_t dst = bstart + bu;
+    if (tl.ostride == 16) {  // stream layout (G = 4): chunk metadata, A/B chunk order per pass
+      const int s0 = (bu - w0) >> 2, nch = plen >> 2;  // the segment in the wave's chunks
+      for (int q = lane; q < nch; q += 64) {
+        const int pos = s0 + q, ps = pos & ~127;  // the pass's first chunk
+        const int sl = s0 >= ps ? (s0 - ps) >> 1 : 0;
+        const int nc = min(128, (wlen >> 2) - ps);
+        const int64_t at = bstart + w0 + 4 * (int64_t)(ps + stream_pass_slot(pos - ps, nc));
+        uint32_t off[4], cf[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool real = 4 * q + e < len;
+          const int cp = real ? x.col[src + 4 * q + e] - p0 : 0;
+          off[e] = (uint32_t)(uint16_t)((16 * emit_slot(cp)) |
+                                        (int)stream_chunk_meta(e, q == 0, q == nch - 1, sl, j));
+          cf[e] = !real ? 0u
+                  : coef_bytes == 4
+                      ? reinterpret_cast<const uint32_t *>(x.coef)[src + 4 * q + e]
+                      : (uint32_t)reinterpret_cast<const uint16_t *>(x.coef)[src + 4 * q + e];
+        }
+        const uint2 o{off[0] | off[1] << 16, off[2] | off[3] << 16};
+        if (coef_bytes == 2) {  // chunk record of 4 offsets then 4 coefficients
+          *reinterpret_cast<uint4 *>(bidx + 2 * at) =
+              make_uint4(o.x, o.y, cf[0] | cf[1] << 16, cf[2] | cf[3] << 16);
+        } else {
+          // FP32: offsets in stream order (the A and B chunks of a lane
+          // adjacent), coefficients in the A-then-B slots
+          *reinterpret_cast<uint2 *>(bidx + dst + 4 * q) = o;
+          *reinterpret_cast<uint4 *>(reinterpret_cast<uint32_t *>(bcoef) + at) =
+              make_uint4(cf[0], cf[1], cf[2], cf[3]);
+        }
+      }
+      continue;
+    }
+    for (int q = lane; q < plen; q += 64) {  // tiled layout: bit 0 marks the segment's first entry
       const bool real = q < len;
-      uint32_t bits;
-      int64_t at = dst + q;
-      if (tl.ostride == 16) {  // stream layout: chunk metadata, A/B chunk order per pass
-        const int pw = 128 * G, pos = ss + q, ps = pos / pw * pw, k = q / G;
-        const int sl = ss >= ps ? ((ss - ps) / G) >> 1 : 0;
-        bits = stream_chunk_meta(q % G, k == 0, k == nch - 1, sl, j);
-        const int nc = min(128, (wlen - ps) / G);
-        at = tl.bstart[blk] + bo[64 * w] + ps + G * stream_pass_slot((pos - ps) / G, nc) + q % G;
-      } else {  // tiled layout: bit 0 marks the segment's first entry
-        bits = q == 0 ? 1u : 0u;
-      }
       const int cp = real ? x.col[src + q] - p0 : 0;
-      const uint16_t off =
-          (uint16_t)((tl.ostride == 16 ? 16 * emit_slot(cp) : tl.ostride * cp) | (int)bits);
-      if (tl.ostride == 16 && coef_bytes == 2) {
-        // stream layout, 16-bit: chunk record of 4 offsets then 4 coefficients
-        // (chunks start at multiples of G = 4 entries)
-        const int64_t rec = (at >> 2) * 8, m4 = at & 3;
-        bidx[rec + m4] = off;
-        bidx[rec + 4 + m4] = real ? reinterpret_cast<const uint16_t *>(x.coef)[src + q] : (uint16_t)0;
-        continue;
-      }
-      // stream layout, FP32: offsets in stream order (the A and B chunks of a
-      // lane adjacent), coefficients in the A-then-B slots
-      bidx[tl.ostride == 16 ? dst + q : at] = off;
+      bidx[dst + q] = (uint16_t)((tl.ostride * cp) | (q == 0 ? 1 : 0));
       if (coef_bytes == 4)
-        reinterpret_cast<float *>(bcoef)[at] =
+        reinterpret_cast<float *>(bcoef)[dst + q] =
             real ? reinterpret_cast<const float *>(x.coef)[src + q] : 0.0f;
       else
-        reinterpret_cast<uint16_t *>(bcoef)[at] =
+        reinterpret_cast<uint16_t *>(bcoef)[dst + q] =
             real ? reinterpret_cast<const uint16_t *>(x.coef)[src + q] : (uint16_t)0;
     }
   }
@@ -1066,12 +1093,16 @@ void launch_block_offsets(const DevXfers &x, const DevTiles &tl, int G, int64_t 
                      boff);
 }
 
-void launch_block_fill(const DevXfers &x, const DevTiles &tl, int G, int coef_bytes,
+void launch_block_fill(const DevXfers &x, const DevTiles &tl, int coef_bytes,
                        uint16_t *bidx, void *bcoef, hipStream_t st) {
-  const int64_t waves = tl.n_chunks * (int64_t)tl.nt * 16;
+  // 16 slots a wave where that still makes 16 K waves: with a PVS most of a
+  // large system's blocks are empty, and a wave costs more than its lookups
+  const int64_t nblk = tl.n_chunks * (int64_t)tl.nt;
+  const int slots = nblk * 64 >= 16384 ? 16 : 4;
+  const int64_t waves = nblk * (1024 / slots);
   if (waves <= 0) return;
-  hipLaunchKernelGGL(k_block_fill, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, x, tl, G,
-                     coef_bytes, bidx, bcoef);
+  hipLaunchKernelGGL(k_block_fill, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, x, tl,
+                     slots, coef_bytes, bidx, bcoef);
 }
 
 // tile boundaries per row: tp[r][t] = first row position with column >= t*C

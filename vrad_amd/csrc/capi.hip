@@ -1096,17 +1096,32 @@ static PvsPlan one_group(int64_t np) {
   return P;
 }
 
+// The bit matrix: np rows of `words` words, then its tiles' flags (`fill`: 0, or
+// 1 for a trace that does not set them).
+static uint8_t *tile_flags(const DBuf &bits, int64_t np, int64_t words) {
+  return bits.as<uint8_t>() + 4 * np * words;
+}
+static int alloc_bits(DBuf &bits, int64_t np, int64_t words, int fill, hipStream_t st) {
+  const size_t b = 4 * (size_t)np * (size_t)words;
+  const size_t f = (size_t)((np + vr::kBitTile - 1) / vr::kBitTile * vr::flag_stride(words));
+  TRY(bits.alloc(std::max<size_t>(b + f, 4)));
+  if (b) VR_HIP(hipMemsetAsync(bits.p, 0, b, st));
+  if (f) VR_HIP(hipMemsetAsync(bits.as<char>() + b, fill, f, st));
+  return VR_OK;
+}
+
 // S: patches (0-6), the plan's members, table and block prefix (7-9) and the
 // segment counters (10).
 static vr::PairJob pair_job(const DevScene &sc, const DevPatches &dp, const PvsPlan &plan,
-                            const Staging &S, uint32_t *bits, int64_t words) {
+                            const Staging &S, const DBuf &bits, int64_t np, int64_t words) {
   vr::PairJob j{};
   j.sc = sc;
   j.p = dp;
   j.mem = plan.mem.empty() ? nullptr : S.ptr<int32_t>(7);
   j.tab = S.ptr<vr::PvsEntry>(8);
   j.blk_pre = S.ptr<int64_t>(9);
-  j.bits = bits;
+  j.bits = bits.as<uint32_t>();
+  j.flags = tile_flags(bits, np, words);
   j.segs = S.ptr<unsigned long long>(10);
   j.words = words;
   j.n_tab = (int32_t)plan.tab.size();
@@ -1121,7 +1136,8 @@ static int transfers_from_bits(vr_xfers *x, const DBuf &bits, int64_t words,
                                int32_t normalize, hipStream_t st) {
   const int64_t np = x->n;
   TRY(x->cnt.alloc(4 * (size_t)std::max<int64_t>(np, 1)));
-  launch_row_count(bits.as<uint32_t>(), np, words, x->cnt.as<int32_t>(), st);
+  uint8_t *const flags = tile_flags(bits, np, words);
+  launch_row_count(bits.as<uint32_t>(), flags, np, words, x->cnt.as<int32_t>(), st);
   TRY(check_launch());
   x->cnt_host.assign((size_t)np, 0);
   if (np > 0)
@@ -1136,8 +1152,8 @@ static int transfers_from_bits(vr_xfers *x, const DBuf &bits, int64_t words,
   TRY(finish_layout(x, st));
   TRY(x->col.alloc(4 * (size_t)x->stored));
   TRY(x->coef32.alloc(4 * (size_t)x->stored));
-  launch_row_fill(bits.as<uint32_t>(), np, words, dp, x->rp.as<int64_t>(), x->cnt.as<int32_t>(),
-                  x->col.as<int32_t>(), x->coef32.as<float>(), st);
+  launch_row_fill(bits.as<uint32_t>(), flags, np, words, dp, x->rp.as<int64_t>(),
+                  x->cnt.as<int32_t>(), x->col.as<int32_t>(), x->coef32.as<float>(), st);
   DBuf rowsum;
   TRY(rowsum.alloc(8 * (size_t)std::max<int64_t>(np, 1)));
   launch_row_normalize(np, x->rp.as<int64_t>(), x->coef32.as<float>(), rowsum.as<double>(),
@@ -1196,8 +1212,7 @@ static int make_transfers_impl(vr_scene *s, const vr_patches *p, int64_t np,
                 S.ptr<float>(4), S.ptr<float>(5), S.ptr<float>(6)};
   const int64_t words = (np + 31) / 32;
   DBuf bits, pairs, count;
-  TRY(bits.alloc((size_t)np * (size_t)words * 4));
-  VR_HIP(hipMemsetAsync(bits.p, 0, bits.bytes, st));
+  TRY(alloc_bits(bits, np, words, fused ? 0 : 1, st));
   unsigned long long *const segs = S.ptr<unsigned long long>(10);
   VR_HIP(hipMemsetAsync(segs, 0, seg_b, st));
   if (!fused) {
@@ -1215,10 +1230,10 @@ static int make_transfers_impl(vr_scene *s, const vr_patches *p, int64_t np,
       return check_launch();
     };
     if (fused) {
-      vr::PairJob j = pair_job(s->dev, dp, plan, S, bits.as<uint32_t>(), words);
+      vr::PairJob j = pair_job(s->dev, dp, plan, S, bits, np, words);
       launch_pair_rows(j, n_blk, P.normal_offset, P.skip_id, tuning().trace_lds_entries,
                        tuning().trace_xcd_group, st);
-      launch_bits_mirror(bits.as<uint32_t>(), np, words, st);
+      launch_bits_mirror(bits.as<uint32_t>(), j.flags, np, words, st);
       TRY(check_launch());
     } else if (nc > 0) {
       // a block keeps at most pvs_chunk(0) pairs
@@ -1360,11 +1375,10 @@ static int make_transfers_shared(vr_scene *const *scenes, const vr_patches *patc
     o.dp = DevPatches{o.S.ptr<float>(0), o.S.ptr<float>(1), o.S.ptr<float>(2), o.S.ptr<float>(3),
                       o.S.ptr<float>(4), o.S.ptr<float>(5), o.S.ptr<float>(6)};
     o.words = (np + 31) / 32;
-    TRY(o.bits.alloc((size_t)std::max<int64_t>(np, 1) * (size_t)std::max<int64_t>(o.words, 1) * 4));
-    VR_HIP(hipMemsetAsync(o.bits.p, 0, o.bits.bytes, st));
+    TRY(alloc_bits(o.bits, np, o.words, 0, st));
     if (o.plan.blk_pre.back() == 0) continue;
     jobs.push_back(pair_job(scenes[which[(size_t)k]]->dev, o.dp, o.plan, o.S,
-                            o.bits.as<uint32_t>(), o.words));
+                            o.bits, np, o.words));
     jobs.back().blk_begin = blocks;
     blocks += o.plan.blk_pre.back();
   }
@@ -1377,7 +1391,8 @@ static int make_transfers_shared(vr_scene *const *scenes, const vr_patches *patc
     TRY(check_launch());
     for (int32_t k = 0; k < n_scenes; ++k) {
       One &o = sc[(size_t)k];
-      launch_bits_mirror(o.bits.as<uint32_t>(), o.x->n, o.words, st);
+      launch_bits_mirror(o.bits.as<uint32_t>(), tile_flags(o.bits, o.x->n, o.words), o.x->n,
+                         o.words, st);
       TRY(transfers_from_bits(o.x.get(), o.bits, o.words, o.dp, o.S.ptr<unsigned long long>(10),
                               P.normalize, st));
       o.bits.release();
@@ -1866,7 +1881,7 @@ int prepare_tiles(vr_xfers *x, const TiledShape &sh, DevTiles &tl, hipStream_t s
     TRY(x->bidx.alloc((inter ? 4 : 2) * (size_t)std::max<int64_t>(run, 1) + 64));
     TRY(x->bcoef.alloc(inter ? 64 : (size_t)cb * (size_t)std::max<int64_t>(run, 1) + 64));
     tl.bstart = x->bstart.as<int64_t>();
-    launch_block_fill(dx, tl, G, cb, x->bidx.as<uint16_t>(), x->bcoef.p, st);
+    launch_block_fill(dx, tl, cb, x->bidx.as<uint16_t>(), x->bcoef.p, st);
     TRY(check_launch());
     VR_HIP(hipStreamSynchronize(st));
     x->blk_cols = cols;

@@ -116,26 +116,34 @@ struct PairJob {
   const PvsEntry *tab;
   const int64_t *blk_pre;
   uint32_t *bits;
+  uint8_t *flags;
   unsigned long long *segs;
   int64_t words;
   int64_t blk_begin;  // the scene's first block in a launch of many
   int32_t n_tab, chunk;
 };
 constexpr int kSegCounters = 64 * 8;
+// The bit matrix in tiles of 512 x 512: byte c of row r of the flags says that
+// tile (r, c) may hold bits (rows of a multiple of 4 bytes).
+constexpr int kBitTile = 512, kTileW = kBitTile / 32;
+__host__ __device__ constexpr int64_t flag_stride(int64_t words) {
+  return (words + 4 * kTileW - 1) / (4 * kTileW) * 4;
+}
 int pair_chunk(int64_t pairs);  // columns per block for a total of candidate pairs
 void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip, int lds_entries,
                       int xcd_group, hipStream_t st);
 void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float eps, int32_t skip,
                            int lds_entries, hipStream_t st);
 // bits |= transpose(bits)
-void launch_bits_mirror(uint32_t *bits, int64_t np, int64_t words, hipStream_t st);
-void launch_row_count(const uint32_t *bits, int64_t np, int64_t words, int32_t *cnt,
-                      hipStream_t st);
+void launch_bits_mirror(uint32_t *bits, uint8_t *flags, int64_t np, int64_t words,
+                        hipStream_t st);
+void launch_row_count(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
+                      int32_t *cnt, hipStream_t st);
 // exclusive scan of padded lengths (multiple of 8) into rp[0..n]
 void launch_row_scan(const int32_t *cnt, int64_t n, int64_t *rp, hipStream_t st);
-void launch_row_fill(const uint32_t *bits, int64_t np, int64_t words, const DevPatches &p,
-                     const int64_t *rp, const int32_t *cnt, int32_t *col, float *coef,
-                     hipStream_t st);
+void launch_row_fill(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
+                     const DevPatches &p, const int64_t *rp, const int32_t *cnt, int32_t *col,
+                     float *coef, hipStream_t st);
 void launch_row_normalize(int64_t n, const int64_t *rp, float *coef, double *row_sum,
                           int normalize, hipStream_t st);
 
@@ -269,7 +277,7 @@ void launch_tile_ptrs(int64_t n, const int64_t *rp, const int32_t *cnt, const in
 // blocked layout: offsets (boff) and per-block totals, then the copy
 void launch_block_offsets(const DevXfers &x, const DevTiles &tl, int G, int64_t *btot,
                           int32_t *boff, hipStream_t st);
-void launch_block_fill(const DevXfers &x, const DevTiles &tl, int G, int coef_bytes,
+void launch_block_fill(const DevXfers &x, const DevTiles &tl, int coef_bytes,
                        uint16_t *bidx, void *bcoef, hipStream_t st);
 // energy of the bounce just gathered; updates state / energy[k]
 void launch_energy(const double *e_row, int64_t n, double *scratch, double *energy, int k,

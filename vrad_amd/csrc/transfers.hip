@@ -170,6 +170,7 @@ __device__ __forceinline__ void pair_rows(const PairJob &J, int64_t gb, float ep
   BvhSpill<S, uint32_t> spill;
   BvhTracer<S, uint32_t> tr(J.sc, s_stk, lane, spill);
   uint32_t *const row = J.bits + (int64_t)i * J.words;
+  uint8_t *const flag = J.flags + (int64_t)(i / kBitTile) * flag_stride(J.words);
   for (;;) {
     while (qn < 64u && col < end) {
       // the segment runs from the smaller patch index to the larger
@@ -215,7 +216,10 @@ __device__ __forceinline__ void pair_rows(const PairJob &J, int64_t gb, float ep
     __syncthreads();
     if ((heads >> lane) & 1ull) {
       const uint32_t v = s_w[run];
-      if (v) atomicOr(row + w, v);
+      if (v) {
+        atomicOr(row + w, v);
+        flag[w / kTileW] = 1;
+      }
     }
   }
   // 64 counters, 64 bytes apart
@@ -299,12 +303,14 @@ void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float
 }
 
 // bits |= transpose(bits), in place.  A workgroup takes a tile of 512 x 512
-// bits and its mirror image (64-byte row pieces, so whole memory accesses):
-// both go to LDS (rows 17 words apart: a column of words lies in 32 banks),
-// half-waves exchange 32 x 32 bit blocks, transposed in 5 steps of the half a
-// lane pairs up with, and the tiles go back if any bit is set.  Bound by
-// reading the matrix once.
-constexpr int kMirror = 512, kMirrorW = kMirror / 32, kMirrorS = kMirrorW + 1;
+// bits and its mirror image (64-byte row pieces, so whole memory accesses) if
+// either holds a bit (flags): both go to LDS (rows 17 words apart: a column of
+// words lies in 32 banks), half-waves exchange 32 x 32 bit blocks, transposed
+// in 5 steps of the half a lane pairs up with, and the tiles go back.  Bound
+// by the memory it moves: with a PVS most of the matrix is empty (on the
+// 8x8-room level 9 rooms of 64 see a room): 9.0 ms without the flags, 1.8 with
+// them, the counting pass 3.8 and 0.5.
+constexpr int kMirrorS = kTileW + 1;
 
 __device__ __forceinline__ uint32_t transpose32(uint32_t x, int l) {
   // rows and columns whose numbers differ in bit s change places, for each s
@@ -317,9 +323,10 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x, int l) {
   return x;
 }
 
-__global__ __launch_bounds__(256) void k_bits_mirror(uint32_t *__restrict__ bits, int64_t np,
+__global__ __launch_bounds__(256) void k_bits_mirror(uint32_t *__restrict__ bits,
+                                                     uint8_t *__restrict__ flags, int64_t np,
                                                      int64_t words, uint32_t nt) {
-  __shared__ uint32_t s_a[kMirror * kMirrorS], s_b[kMirror * kMirrorS];
+  __shared__ uint32_t s_a[kBitTile * kMirrorS], s_b[kBitTile * kMirrorS];
   // tile (r, c), r <= c, of the upper triangle's row-by-row enumeration
   // folded in two: row r of the fold holds tiles (r, r..) and (nt-1-r, ..)
   const uint32_t w = nt + 1, f = blockIdx.x / w, x = blockIdx.x % w;
@@ -329,25 +336,26 @@ __global__ __launch_bounds__(256) void k_bits_mirror(uint32_t *__restrict__ bits
     c = r + (x - (nt - f));
     if (r == f) return;  // the middle row of an odd count stands alone
   }
-  const int64_t ra = (int64_t)r * kMirror, rb = (int64_t)c * kMirror;
-  const int64_t wa = (int64_t)c * kMirrorW, wb = (int64_t)r * kMirrorW;
-  const int t = (int)threadIdx.x, col = t & (kMirrorW - 1);
+  const int64_t ra = (int64_t)r * kBitTile, rb = (int64_t)c * kBitTile;
+  const int64_t wa = (int64_t)c * kTileW, wb = (int64_t)r * kTileW;
+  const int t = (int)threadIdx.x, col = t & (kTileW - 1);
   const bool diag = r == c;
-  uint32_t any = 0;
+  uint8_t *const fa = flags + r * flag_stride(words) + c, *const fb = flags + c * flag_stride(words) + r;
+  if ((*fa | *fb) == 0) return;  // read by all threads before the first barrier
 #pragma unroll 8
-  for (int k = t / kMirrorW; k < kMirror; k += 256 / kMirrorW) {
+  for (int k = t / kTileW; k < kBitTile; k += 256 / kTileW) {
     const uint32_t a = ra + k < np && wa + col < words ? bits[(ra + k) * words + wa + col] : 0u;
     const uint32_t b =
         !diag && rb + k < np && wb + col < words ? bits[(rb + k) * words + wb + col] : 0u;
     s_a[k * kMirrorS + col] = a;
     s_b[k * kMirrorS + col] = b;
-    any |= a | b;
   }
-  if (!__syncthreads_or((int)any)) return;
+  __syncthreads();
+  if (t == 0) *fa = *fb = 1;
   uint32_t *const s_m = diag ? s_a : s_b;
   const int half = t >> 5, l = t & 31;
-  for (int q = half; q < kMirrorW * kMirrorW; q += 8) {
-    const int br = q / kMirrorW, bc = q % kMirrorW;
+  for (int q = half; q < kTileW * kTileW; q += 8) {
+    const int br = q / kTileW, bc = q % kTileW;
     // both halves of a wave run the shuffles; of a diagonal tile's block pair
     // only one writes
     uint32_t *const pa = s_a + (32 * br + l) * kMirrorS + bc;
@@ -361,38 +369,63 @@ __global__ __launch_bounds__(256) void k_bits_mirror(uint32_t *__restrict__ bits
   }
   __syncthreads();
 #pragma unroll 8
-  for (int k = t / kMirrorW; k < kMirror; k += 256 / kMirrorW) {
+  for (int k = t / kTileW; k < kBitTile; k += 256 / kTileW) {
     if (ra + k < np && wa + col < words) bits[(ra + k) * words + wa + col] = s_a[k * kMirrorS + col];
     if (!diag && rb + k < np && wb + col < words)
       bits[(rb + k) * words + wb + col] = s_b[k * kMirrorS + col];
   }
 }
 
-void launch_bits_mirror(uint32_t *bits, int64_t np, int64_t words, hipStream_t st) {
+void launch_bits_mirror(uint32_t *bits, uint8_t *flags, int64_t np, int64_t words,
+                        hipStream_t st) {
   if (np <= 0) return;
-  const uint32_t nt = (uint32_t)((np + kMirror - 1) / kMirror);
+  const uint32_t nt = (uint32_t)((np + kBitTile - 1) / kBitTile);
   const uint32_t grid = (nt + 1) / 2 * (nt + 1);
-  hipLaunchKernelGGL(k_bits_mirror, dim3(grid), dim3(256), 0, st, bits, np, words, nt);
+  hipLaunchKernelGGL(k_bits_mirror, dim3(grid), dim3(256), 0, st, bits, flags, np, words,
+                     nt);
+}
+
+// Chunks of 64 words (four tiles, one flag word) of a row that hold bits: the
+// lanes look at 64 chunks' flags at once, f(chunk) runs for each with any
+// set.
+template <class F>
+__device__ __forceinline__ void for_chunks(const uint8_t *flags, int64_t row, int64_t words,
+                                           int lane, F f) {
+  const uint32_t *fl = reinterpret_cast<const uint32_t *>(flags + row / kBitTile * flag_stride(words));
+  const int64_t nq = (words + 63) / 64;
+  for (int64_t q0 = 0; q0 < nq; q0 += 64) {
+    uint64_t m = __ballot(q0 + lane < nq && fl[q0 + lane] != 0u);
+    while (m) {
+      const int64_t q = q0 + __ffsll((unsigned long long)m) - 1;
+      m &= m - 1ull;
+      f(q);
+    }
+  }
 }
 
 // one wave per row
-__global__ __launch_bounds__(256) void k_row_count(const uint32_t *__restrict__ bits, int64_t np,
+__global__ __launch_bounds__(256) void k_row_count(const uint32_t *__restrict__ bits,
+                                                   const uint8_t *__restrict__ flags, int64_t np,
                                                    int64_t words, int32_t *__restrict__ cnt) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
+  const int64_t row =
+      (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (row >= np) return;
   const uint32_t *rb = bits + row * words;
   int c = 0;
-  for (int64_t w = lane; w < words; w += 64) c += __popc(rb[w]);
+  for_chunks(flags, row, words, lane, [&](int64_t q) {
+    const int64_t w = 64 * q + lane;
+    if (w < words) c += __popc(rb[w]);
+  });
   for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
   if (lane == 0) cnt[row] = c;
 }
 
-void launch_row_count(const uint32_t *bits, int64_t np, int64_t words, int32_t *cnt,
-                      hipStream_t st) {
+void launch_row_count(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
+                      int32_t *cnt, hipStream_t st) {
   if (np <= 0) return;
-  hipLaunchKernelGGL(k_row_count, dim3((unsigned)((np + 3) / 4)), dim3(256), 0, st, bits, np,
-                     words, cnt);
+  hipLaunchKernelGGL(k_row_count, dim3((unsigned)((np + 3) / 4)), dim3(256), 0, st, bits, flags,
+                     np, words, cnt);
 }
 
 // single-block exclusive scan of padded lengths: rp[i] = sum_{k<i} pad8(cnt[k])
@@ -436,10 +469,14 @@ __device__ __forceinline__ float form_factor(const DevPatches &p, int64_t i, int
 }
 
 // One wave per row, over the bit matrix row in chunks of 64 words (2048
-// columns): each lane takes a word, the set bits' columns go to LDS at their
-// rank in the chunk (ascending), and consecutive lanes then write consecutive
-// entries (col and F_ij) to the CSR, so the stores are contiguous.
-__global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bits, int64_t np,
+// columns) that hold bits: each lane takes a word (the next chunk's is loaded
+// ahead), the set bits' columns go to LDS at their rank in the chunk
+// (ascending), and consecutive lanes then write consecutive entries (col and
+// F_ij) to the CSR, so the stores are contiguous.  A wave per row that looked
+// at every chunk in turn took 14.4 ms on the 8x8-room level, most of it the
+// wait for 167 loads one after another; 7.0 now, against 3 for the stores.
+__global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bits,
+                                                 const uint8_t *__restrict__ flags, int64_t np,
                                                  int64_t words, DevPatches p,
                                                  const int64_t *__restrict__ rp,
                                                  const int32_t *__restrict__ cnt,
@@ -452,9 +489,8 @@ __global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bi
   const uint32_t *rb = bits + row * words;
   const int64_t s = rp[row];
   int64_t run = 0;
-  for (int64_t w0 = 0; w0 < words; w0 += 64) {
-    const int64_t w = w0 + lane;
-    uint32_t m = w < words ? rb[w] : 0u;
+  auto chunk = [&](int64_t q, uint32_t m) {
+    const int64_t w = 64 * q + lane;
     const int pc = __popc(m);
     // inclusive wave scan of pc
     int inc = pc;
@@ -463,7 +499,7 @@ __global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bi
       if (lane >= off) inc += v;
     }
     const int tot = __shfl(inc, 63);
-    if (tot == 0) continue;
+    if (tot == 0) return;
     int at = inc - pc;
     while (m) {
       const int bit = __ffs(m) - 1;
@@ -478,7 +514,17 @@ __global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bi
     }
     __syncthreads();  // and read before the next chunk overwrites them
     run += tot;
-  }
+  };
+  int64_t held = -1;  // the chunk whose words are on their way
+  uint32_t mh = 0;
+  for_chunks(flags, row, words, lane, [&](int64_t q) {
+    const int64_t w = 64 * q + lane;
+    const uint32_t m = w < words ? rb[w] : 0u;
+    if (held >= 0) chunk(held, mh);
+    held = q;
+    mh = m;
+  });
+  if (held >= 0) chunk(held, mh);
   const int64_t c = cnt[row], e = rp[row + 1];
   for (int64_t k = s + c + lane; k < e; k += 64) {
     col[k] = (int32_t)row;
@@ -486,12 +532,12 @@ __global__ __launch_bounds__(64) void k_row_fill(const uint32_t *__restrict__ bi
   }
 }
 
-void launch_row_fill(const uint32_t *bits, int64_t np, int64_t words, const DevPatches &p,
-                     const int64_t *rp, const int32_t *cnt, int32_t *col, float *coef,
-                     hipStream_t st) {
+void launch_row_fill(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
+                     const DevPatches &p, const int64_t *rp, const int32_t *cnt, int32_t *col,
+                     float *coef, hipStream_t st) {
   if (np <= 0) return;
-  hipLaunchKernelGGL(k_row_fill, dim3((unsigned)np), dim3(64), 0, st, bits, np, words, p, rp, cnt,
-                     col, coef);
+  hipLaunchKernelGGL(k_row_fill, dim3((unsigned)np), dim3(64), 0, st, bits, flags, np, words, p, rp,
+                     cnt, col, coef);
 }
 
 // FP64 row sum in wave order (lane owns p with (p/4)%64 == lane), butterfly
