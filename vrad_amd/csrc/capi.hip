@@ -352,14 +352,26 @@ void layout_rows(const std::vector<int32_t> &cnt, std::vector<int64_t> &rp) {
   for (int64_t i = 0; i < n; ++i) rp[i + 1] = rp[i] + (((int64_t)cnt[i] + 7) & ~(int64_t)7);
 }
 
+// placement 0's order, on the device (row_order gives the same)
+int sort_rows(const vr_xfers *x, hipStream_t st) {
+  DBuf scratch;
+  const int rc = scratch.alloc(4 * (size_t)row_order_scratch(x->n));
+  if (rc) return rc;
+  const int32_t longest =
+      x->n ? *std::max_element(x->cnt_host.begin(), x->cnt_host.end()) : 0;
+  launch_row_order(x->cnt.as<int32_t>(), x->n, longest, x->order.as<int32_t>(),
+                   scratch.as<int32_t>(), st);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? VR_OK : fail(VR_E_HIP, std::string("row order: ") + hipGetErrorString(e));
+}
+
 int finish_layout(vr_xfers *x, hipStream_t st) {
-  std::vector<int32_t> order;
   layout_rows(x->cnt_host, x->rp_host);
-  row_order(x->cnt_host, 0, order);
   x->placement = 0;
   int rc = upload_vec(x->rp, x->rp_host, st);
-  if (!rc) rc = upload_vec(x->order, order, st);
   if (!rc) rc = upload_vec(x->cnt, x->cnt_host, st);
+  if (!rc) rc = x->order.alloc(4 * x->cnt_host.size());
+  if (!rc) rc = sort_rows(x, st);
   x->stored = x->rp_host.back();
   return rc;
 }
@@ -1832,14 +1844,18 @@ int prepare_tiles(vr_xfers *x, const TiledShape &sh, DevTiles &tl, hipStream_t s
   if (x->served && !tiles_ready(x, sh))
     return fail(VR_E_STATE, "transfers are held by a server with another gather layout");
   if (x->placement != sh.placement) {  // deal the rows again; the blocked copy follows them
-    std::vector<int32_t> order;
-    row_order(x->cnt_host, sh.placement, order);
     // into the same buffer (n rows either way), so the order pointer in every
     // DevXfers already taken of x stays valid
-    if (x->order.bytes < sizeof(int32_t) * order.size())
+    if (x->order.bytes < sizeof(int32_t) * (size_t)n)
       return fail(VR_E_STATE, "row order buffer smaller than the rows");
-    VR_HIP(hipMemcpyAsync(x->order.p, order.data(), sizeof(int32_t) * order.size(),
-                          hipMemcpyHostToDevice, st));
+    std::vector<int32_t> order;
+    if (sh.placement == 0) {
+      TRY(sort_rows(x, st));
+    } else {
+      row_order(x->cnt_host, sh.placement, order);
+      VR_HIP(hipMemcpyAsync(x->order.p, order.data(), sizeof(int32_t) * order.size(),
+                            hipMemcpyHostToDevice, st));
+    }
     VR_HIP(hipStreamSynchronize(st));
     x->placement = sh.placement;
     x->blk_cols = 0;

