@@ -190,36 +190,15 @@ __device__ __forceinline__ int64_t eval_chunks(const KNode &nd) {
   return refinable(nd) ? ((int64_t)nd.n + kEvalChunk - 1) / kEvalChunk : 0;
 }
 
-// chunk_start[i] = partition chunks of the nodes before i (ceil(n / kChunk)
-// each), eval_start[i] = evaluation chunks (ceil(n / kEvalChunk) per node to
-// refine); entry N = totals.  One block.
-__global__ __launch_bounds__(1024) void k_kd_chunks(const KNode *__restrict__ nodes, int32_t N,
-                                                    int64_t *__restrict__ chunk_start,
-                                                    int64_t *__restrict__ eval_start) {
-  __shared__ int64_t sh[1024];
-  const int t = (int)threadIdx.x;
-  const int32_t per = (N + 1023) / 1024;
-  const int32_t a = min(N, t * per), b = min(N, a + per);
-  int64_t s = 0, se = 0;
-  for (int32_t i = a; i < b; ++i) {
-    const KNode nd = nodes[i];
-    s += part_chunks(nd);
-    se += eval_chunks(nd);
-  }
-  int64_t total, etotal;
-  int64_t run = block_scan(s, sh, &total);
-  int64_t erun = block_scan(se, sh, &etotal);
-  for (int32_t i = a; i < b; ++i) {
-    const KNode nd = nodes[i];
-    chunk_start[i] = run;
-    eval_start[i] = erun;
-    run += part_chunks(nd);
-    erun += eval_chunks(nd);
-  }
-  if (t == 0) {
-    chunk_start[N] = total;
-    eval_start[N] = etotal;
-  }
+// chunk_start[i] = partition chunks of a level's nodes before i (ceil(n /
+// kChunk) each), eval_start[i] = evaluation chunks (ceil(n / kEvalChunk) per
+// node to refine); entry N = totals.  The root's, one thread; k_kd_children
+// writes every other level's.
+__global__ void k_kd_chunks(const KNode *__restrict__ root, int64_t *__restrict__ chunk_start,
+                            int64_t *__restrict__ eval_start) {
+  chunk_start[0] = eval_start[0] = 0;
+  chunk_start[1] = part_chunks(*root);
+  eval_start[1] = eval_chunks(*root);
 }
 
 // Candidate splits of node i on axis a, in the host builder's order: the
@@ -420,59 +399,97 @@ __global__ __launch_bounds__(256) void k_kd_select(
   if (lane == 0) dec[i] = d;
 }
 
-// Children slots and list offsets in the next level (one block); tot[0] =
-// next level's nodes, tot[1] = its references.
-__global__ __launch_bounds__(1024) void k_kd_nodescan(int32_t N, KDec *__restrict__ dec,
+// What a node adds to the next level: nodes, references, partition chunks and
+// evaluation chunks.
+struct KSum {
+  int64_t v[4];
+};
+__device__ __forceinline__ void kd_split(const KNode &nd, const KDec &d, KNode &L, KNode &R) {
+  L = R = nd;
+  L.n = d.nl + d.nb;
+  R.n = d.nb + d.nr;
+  L.depth = R.depth = d.cdepth;
+  L.mx[d.kind] = d.moved;
+  R.mn[d.kind] = d.moved;
+}
+__device__ __forceinline__ KSum kd_sum(const KNode &L, const KNode &R) {
+  return KSum{{2, (int64_t)L.n + R.n, part_chunks(L) + part_chunks(R),
+               eval_chunks(L) + eval_chunks(R)}};
+}
+
+// The next level's layout in three launches: sums per 256 nodes, their scan
+// (tot[0] = the next level's nodes, tot[1] = its references, tot[2], tot[3] =
+// its chunks), and the children with their slots, list offsets and chunk
+// starts.  Bound by latency; one block walking all nodes of a level, 49 per
+// thread in turn, took 31 us a level and another 27 for the chunk starts.
+__global__ __launch_bounds__(256) void k_kd_sums(const KNode *__restrict__ nodes,
+                                                 const KDec *__restrict__ dec, int32_t N,
+                                                 KSum *__restrict__ sums) {
+  __shared__ int64_t sh[256];
+  const int32_t i = (int32_t)(blockIdx.x * 256 + threadIdx.x);
+  KSum s{{0, 0, 0, 0}};
+  if (i < N && dec[i].kind != (int32_t)kLeafType) {
+    KNode L, R;
+    kd_split(nodes[i], dec[i], L, R);
+    s = kd_sum(L, R);
+  }
+  for (int q = 0; q < 4; ++q) {
+    int64_t total;
+    block_scan<256>(s.v[q], sh, &total);
+    if (threadIdx.x == 0) sums[blockIdx.x].v[q] = total;
+  }
+}
+__global__ __launch_bounds__(1024) void k_kd_nodescan(int32_t nb, KSum *__restrict__ sums,
                                                       int64_t *__restrict__ tot) {
   __shared__ int64_t sh[1024];
   const int t = (int)threadIdx.x;
-  const int32_t per = (N + 1023) / 1024;
-  const int32_t a = min(N, t * per), b = min(N, a + per);
-  int64_t sn = 0, sr = 0;
-  for (int32_t i = a; i < b; ++i) {
-    const KDec &d = dec[i];
-    if (d.kind != (int32_t)kLeafType) {
-      sn += 2;
-      sr += (int64_t)d.nl + 2 * (int64_t)d.nb + d.nr;
+  const int32_t per = (nb + 1023) / 1024;
+  const int32_t a = min(nb, t * per), b = min(nb, a + per);
+  for (int q = 0; q < 4; ++q) {
+    int64_t s = 0;
+    for (int32_t i = a; i < b; ++i) s += sums[i].v[q];
+    int64_t total;
+    int64_t run = block_scan(s, sh, &total);
+    for (int32_t i = a; i < b; ++i) {
+      const int64_t x = sums[i].v[q];
+      sums[i].v[q] = run;
+      run += x;
     }
-  }
-  int64_t tn, tr;
-  int64_t rn = block_scan(sn, sh, &tn);
-  int64_t rr = block_scan(sr, sh, &tr);
-  for (int32_t i = a; i < b; ++i) {
-    KDec &d = dec[i];
-    if (d.kind != (int32_t)kLeafType) {
-      d.child = (int32_t)rn;
-      d.loff = rr;
-      d.roff = rr + d.nl + d.nb;
-      rn += 2;
-      rr += (int64_t)d.nl + 2 * (int64_t)d.nb + d.nr;
-    }
-  }
-  if (t == 0) {
-    tot[0] = tn;
-    tot[1] = tr;
+    if (t == 0) tot[q] = total;
   }
 }
-
-__global__ void k_kd_children(const KNode *__restrict__ nodes, const KDec *__restrict__ dec,
-                              int32_t N, KNode *__restrict__ next) {
-  const int32_t i = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= N) return;
-  const KDec d = dec[i];
-  if (d.kind == (int32_t)kLeafType) return;
-  const KNode nd = nodes[i];
-  KNode L = nd, R = nd;
-  L.off = d.loff;
-  L.n = d.nl + d.nb;
-  L.depth = d.cdepth;
-  L.mx[d.kind] = d.moved;
-  R.off = d.roff;
-  R.n = d.nb + d.nr;
-  R.depth = d.cdepth;
-  R.mn[d.kind] = d.moved;
-  next[d.child] = L;
-  next[d.child + 1] = R;
+__global__ __launch_bounds__(256) void k_kd_children(
+    const KNode *__restrict__ nodes, KDec *__restrict__ dec, int32_t N,
+    const KSum *__restrict__ sums, const int64_t *__restrict__ tot, KNode *__restrict__ next,
+    int64_t *__restrict__ chunk_start, int64_t *__restrict__ eval_start) {
+  __shared__ int64_t sh[256];
+  const int32_t i = (int32_t)(blockIdx.x * 256 + threadIdx.x);
+  const bool split = i < N && dec[i].kind != (int32_t)kLeafType;
+  KNode L, R;
+  KSum s{{0, 0, 0, 0}};
+  if (split) {
+    kd_split(nodes[i], dec[i], L, R);
+    s = kd_sum(L, R);
+  }
+  int64_t at[4];
+  for (int q = 0; q < 4; ++q) at[q] = sums[blockIdx.x].v[q] + block_scan<256>(s.v[q], sh, nullptr);
+  if (i == 0) {
+    chunk_start[tot[0]] = tot[2];
+    eval_start[tot[0]] = tot[3];
+  }
+  if (!split) return;
+  const int64_t c = at[0];
+  L.off = at[1];
+  R.off = at[1] + L.n;
+  dec[i].child = (int32_t)c;
+  dec[i].loff = L.off;
+  dec[i].roff = R.off;
+  next[c] = L;
+  next[c + 1] = R;
+  chunk_start[c] = at[2];
+  chunk_start[c + 1] = at[2] + part_chunks(L);
+  eval_start[c] = at[3];
+  eval_start[c + 1] = at[3] + eval_chunks(L);
 }
 
 // Per chunk of a split node whose list spans several chunks: counts of
@@ -737,6 +754,7 @@ struct Level {
   int64_t R = 0;
   int64_t *ns = nullptr, *nr = nullptr;  // subtree totals
   int64_t *gi = nullptr, *rk = nullptr, *ro = nullptr;
+  int64_t *cs = nullptr, *es = nullptr;  // chunk starts
 };
 
 #define KD_HIP(call)                                                                    \
@@ -770,7 +788,7 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
   KD_TRY(keep.get(&hi, 3 * n));
   KD_TRY(keep.get(&err, 1));
   KD_TRY(keep.get(&rext, 6));
-  KD_TRY(keep.get(&tot, 2));
+  KD_TRY(keep.get(&tot, 4));
   std::vector<Level> lv(1);
   KD_TRY(keep.get(&lv[0].nodes, 1));
   KD_TRY(keep.get(&lv[0].refs, n));
@@ -784,6 +802,9 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
   if (n) hipLaunchKernelGGL(k_kd_root_keys, dim3(std::min(256u, grid(n, 1024))), dim3(256), 0, st,
                             lo, hi, n, rext);
   hipLaunchKernelGGL(k_kd_root, dim3(1), dim3(1), 0, st, lo, hi, n, lv[0].nodes, rext);
+  KD_TRY(keep.get(&lv[0].cs, 2));
+  KD_TRY(keep.get(&lv[0].es, 2));
+  hipLaunchKernelGGL(k_kd_chunks, dim3(1), dim3(1), 0, st, lv[0].nodes, lv[0].cs, lv[0].es);
   KD_HIP(hipGetLastError());
   for (size_t L = 0;; ++L) {
     Level &c = lv[L];
@@ -792,25 +813,25 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
     float *cv;
     int32_t *cc, *cl, *cr;
     unsigned long long *ext;
-    int64_t *cs, *es;
+    KSum *sums;
+    int64_t *const cs = c.cs, *const es = c.es;
     KD_TRY(keep.get(&c.dec, N));
     KD_TRY(tmp.get(&cv, (int64_t)N * kCands));
     KD_TRY(tmp.get(&cc, 3 * (int64_t)N));
     KD_TRY(tmp.get(&cl, (int64_t)N * kCands));
     KD_TRY(tmp.get(&cr, (int64_t)N * kCands));
     KD_TRY(tmp.get(&ext, 6 * (int64_t)N));
-    KD_TRY(tmp.get(&cs, (int64_t)N + 1));
-    KD_TRY(tmp.get(&es, (int64_t)N + 1));
+    KD_TRY(tmp.get(&sums, (int64_t)grid(N, 256)));
     const int64_t max_chunks = c.R / kChunk + N + 1;
     const int64_t max_echunks = c.R / kEvalChunk + N + 1;
-    hipLaunchKernelGGL(k_kd_chunks, dim3(1), dim3(1024), 0, st, c.nodes, N, cs, es);
     hipLaunchKernelGGL(k_kd_cands, dim3(grid(96 * (int64_t)N, 256)), dim3(256), 0, st, c.nodes, N,
                        c.refs, v9, cv, cc, cl, cr, ext);
     hipLaunchKernelGGL(k_kd_eval, dim3(grid(max_echunks, 1)), dim3(256), 0, st, c.nodes, N, es,
                        c.refs, lo, hi, cv, cc, cl, cr, ext);
     hipLaunchKernelGGL(k_kd_select, dim3(grid(N, 4)), dim3(256), 0, st, c.nodes, N, c.refs, lo,
                        hi, cv, cc, cl, cr, ext, c.dec);
-    hipLaunchKernelGGL(k_kd_nodescan, dim3(1), dim3(1024), 0, st, N, c.dec, tot);
+    hipLaunchKernelGGL(k_kd_sums, dim3(grid(N, 256)), dim3(256), 0, st, c.nodes, c.dec, N, sums);
+    hipLaunchKernelGGL(k_kd_nodescan, dim3(1), dim3(1024), 0, st, (int32_t)grid(N, 256), sums, tot);
     KD_HIP(hipGetLastError());
     int64_t th[2] = {0, 0};
     int32_t lerr = 0;
@@ -831,6 +852,8 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
     nx.R = th[1];
     KD_TRY(keep.get(&nx.nodes, nx.N));
     KD_TRY(keep.get(&nx.refs, nx.R));
+    KD_TRY(keep.get(&nx.cs, (int64_t)nx.N + 1));
+    KD_TRY(keep.get(&nx.es, (int64_t)nx.N + 1));
     // every slot is written by the partition; zero first so that even an
     // inconsistent partition (reported through err) leaves valid indices
     KD_HIP(hipMemsetAsync(nx.refs, 0, sizeof(int32_t) * (size_t)std::max<int64_t>(nx.R, 1), st));
@@ -838,7 +861,7 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
     KD_TRY(tmp.get(&ccnt, max_chunks));
     KD_TRY(tmp.get(&pfx, 3 * max_chunks));
     hipLaunchKernelGGL(k_kd_children, dim3(grid(N, 256)), dim3(256), 0, st, c2.nodes, c2.dec, N,
-                       nx.nodes);
+                       sums, tot, nx.nodes, nx.cs, nx.es);
     hipLaunchKernelGGL(k_kd_partcount, dim3(grid(max_chunks, 1)), dim3(256), 0, st, c2.nodes,
                        c2.dec, N, cs, c2.refs, lo, hi, ccnt);
     hipLaunchKernelGGL(k_kd_chunkbase, dim3(grid(N, 256)), dim3(256), 0, st, c2.nodes, c2.dec, N,
