@@ -1423,6 +1423,7 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
   if (n_scenes == 0) return VR_OK;
   if (!scenes || !samples || !n || !n_lights || !rgb) return fail(VR_E_INVALID, "NULL argument");
   int64_t ns_tot = 0, nl_tot = 0;
+  bool bvh = true;
   for (int32_t k = 0; k < n_scenes; ++k) {
     const std::string who = "scene " + std::to_string(k) + ": ";
     if (!scenes[k]) return fail(VR_E_INVALID, who + "NULL scene");
@@ -1434,9 +1435,10 @@ int vr_gather_sample_light_batch(vr_scene *const *scenes, const vr_samples *samp
     if (n_lights[k] > 0 && (!lights || !lights[k])) return fail(VR_E_INVALID, who + "NULL lights");
     ns_tot += n[k];
     nl_tot += n_lights[k];
+    bvh = bvh && scenes[k]->dev.has_bvh;
   }
   if (ns_tot == 0) return VR_OK;
-  if (g_path == VR_PATH_PLAIN) {  // the comparison path: one scene at a time
+  if (g_path == VR_PATH_PLAIN || !bvh) {  // the comparison path: one scene at a time
     for (int32_t k = 0; k < n_scenes; ++k)
       TRY(vr_gather_sample_light(scenes[k], &samples[k], n[k], lights ? lights[k] : nullptr,
                                  n_lights[k], normal_offset, skip_id, rgb[k]));

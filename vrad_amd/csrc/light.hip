@@ -294,16 +294,12 @@ void launch_gather_jobs(const GatherJob *jobs, int n_jobs, int64_t total_blocks,
 // -1, and the wave stops after the first round in which some lane's
 // segment is visible (a miss, or a sky hit before any other).  "Any" does
 // not depend on the order the directions are taken in.
-template <int S>
-__global__ __launch_bounds__(64) void k_leaf_sky(DevScene sc, const int16_t *__restrict__ mins,
-                                                 const int16_t *__restrict__ maxs, int64_t n,
-                                                 const float *__restrict__ dirs,
-                                                 uint8_t *__restrict__ out) {
-  __shared__ uint32_t s_stk[S * 64];
-  const int64_t leaf = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
-  if (leaf >= n) return;
-  BvhSpill<S, uint32_t> spill;
-  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
+template <class Tracer>
+__device__ __forceinline__ void leaf_sky(const DevScene &sc, Tracer &tr, int64_t leaf,
+                                         const int16_t *__restrict__ mins,
+                                         const int16_t *__restrict__ maxs,
+                                         const float *__restrict__ dirs,
+                                         uint8_t *__restrict__ out) {
   const float cx = (float)((int32_t)mins[3 * leaf + 0] + (int32_t)maxs[3 * leaf + 0]) * 0.5f;
   const float cy = (float)((int32_t)mins[3 * leaf + 1] + (int32_t)maxs[3 * leaf + 1]) * 0.5f;
   const float cz = (float)((int32_t)mins[3 * leaf + 2] + (int32_t)maxs[3 * leaf + 2]) * 0.5f;
@@ -323,10 +319,37 @@ __global__ __launch_bounds__(64) void k_leaf_sky(DevScene sc, const int16_t *__r
   }
   if (threadIdx.x == 0) out[leaf] = any;
 }
+template <int S>
+__global__ __launch_bounds__(64) void k_leaf_sky(DevScene sc, const int16_t *__restrict__ mins,
+                                                 const int16_t *__restrict__ maxs, int64_t n,
+                                                 const float *__restrict__ dirs,
+                                                 uint8_t *__restrict__ out) {
+  __shared__ uint32_t s_stk[S * 64];
+  const int64_t leaf = (int64_t)xcd_group_chunk(blockIdx.x, gridDim.x, kXcdGroup);
+  if (leaf >= n) return;
+  BvhSpill<S, uint32_t> spill;
+  BvhTracer<S, uint32_t> tr(sc, s_stk, (int)threadIdx.x, spill);
+  leaf_sky(sc, tr, leaf, mins, maxs, dirs, out);
+}
+// scenes too large for the hierarchy's 32-bit offsets
+template <int D>
+__global__ __launch_bounds__(64) void k_leaf_sky_kd(DevScene sc, const int16_t *__restrict__ mins,
+                                                    const int16_t *__restrict__ maxs, int64_t n,
+                                                    const float *__restrict__ dirs,
+                                                    uint8_t *__restrict__ out) {
+  if ((int64_t)blockIdx.x >= n) return;
+  KdTracer<D> tr(sc);
+  leaf_sky(sc, tr, blockIdx.x, mins, maxs, dirs, out);
+}
 
 void launch_leaf_sky(const DevScene &sc, const int16_t *mins, const int16_t *maxs, int64_t n,
                      const float *sky_dirs, uint8_t *out, hipStream_t st) {
   if (n <= 0) return;
+  if (!sc.has_bvh) {
+    hipLaunchKernelGGL((k_leaf_sky_kd<kStackDepth>), dim3((unsigned)n), dim3(64), 0, st, sc, mins,
+                       maxs, n, sky_dirs, out);
+    return;
+  }
 #define VR_LEAFSKY(S)                                                                      \
   hipLaunchKernelGGL((k_leaf_sky<S>), dim3((unsigned)n), dim3(64), 0, st, sc, \
                      mins, maxs, n, sky_dirs, out)
