@@ -1,0 +1,88 @@
+"""The pool of device blocks against a recorded stand-in for the HIP calls: what
+it hands out, keeps and gives back, without a GPU."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "vrad_amd", "csrc")
+MB, GB = 1 << 20, 1 << 30
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("devmem") / "pool.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic",
+                    "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", so,
+                    os.path.join(HERE, "devmem_harness.cpp"), os.path.join(CSRC, "devmem.cpp")],
+                   check=True)
+    return so
+
+
+@pytest.fixture
+def pool(built, tmp_path):
+    """A fresh pool (its own copy of the library) on a device of 64 GB."""
+    so = tmp_path / "pool.so"
+    so.write_bytes(open(built, "rb").read())
+    lib = C.CDLL(str(so))
+    for name in ("t_alloc",):
+        getattr(lib, name).restype = C.c_void_p
+    for name in ("t_used", "t_bytes", "t_syncs"):
+        getattr(lib, name).restype = C.c_int64
+    lib.t_alloc.argtypes = lib.t_setup.argtypes = [C.c_int64]
+    lib.t_free.argtypes = lib.t_bytes.argtypes = lib.t_block_device.argtypes = [C.c_void_p]
+    lib.t_setup(64 * GB)
+    return lib
+
+
+def test_freed_block_waits_for_the_device(pool):
+    """A block given back with work in flight is handed out after a
+    synchronisation, which one request pays for all."""
+    a, b = pool.t_alloc(MB), pool.t_alloc(3 * MB)
+    pool.t_free(a)
+    pool.t_free(b)
+    assert pool.t_syncs(0) == 0
+    assert pool.t_alloc(MB) == a and pool.t_syncs(0) == 1
+    assert pool.t_alloc(3 * MB) == b and pool.t_syncs(0) == 1
+
+
+def test_failed_synchronisation_hands_nothing_out(pool):
+    """A synchronisation that fails (a stream of the caller is capturing) says
+    nothing about the work that uses a freed block."""
+    a = pool.t_alloc(MB)
+    pool.t_free(a)
+    pool.t_sync_error(1)
+    b = pool.t_alloc(MB)
+    assert b is not None and b != a
+    assert pool.t_bytes(a) >= MB  # nor did it go back to the driver
+    pool.t_sync_error(0)
+    assert pool.t_alloc(MB) == a and pool.t_syncs(0) == 1
+
+
+def test_kept_memory_is_bounded(pool):
+    """256 MB without a live handle, an eighth of the device with one; the rest
+    goes back to the driver."""
+    blocks = [pool.t_alloc(100 * MB) for _ in range(5)]
+    for p in blocks:
+        pool.t_free(p)
+    assert pool.t_used() <= 256 * MB
+    pool.t_holder(1)
+    blocks = [pool.t_alloc(2 * GB) for _ in range(8)]
+    for p in blocks:
+        pool.t_free(p)
+    assert 6 * GB < pool.t_used() <= 8 * GB
+    big = pool.t_alloc(9 * GB)
+    pool.t_free(big)
+    assert pool.t_bytes(big) == -1
+    pool.t_holder(-1)
+    assert pool.t_used() <= 256 * MB
+
+
+def test_kept_blocks_go_back_when_memory_runs_out(pool):
+    pool.t_holder(1)
+    a = pool.t_alloc(7 * GB)
+    pool.t_free(a)
+    assert pool.t_alloc(60 * GB) is not None
+    assert pool.t_bytes(a) == -1

@@ -54,13 +54,20 @@ struct Pool {
     (void)hipFree(it->second);
     ready.erase(it);
   }
+  // The waiting blocks become ready, unless the synchronisation fails (a stream
+  // of the caller is capturing, say): then their work may still run, and they
+  // wait on.
   void settle() {
     if (waiting.empty()) return;
-    (void)hipDeviceSynchronize();
+    if (hipDeviceSynchronize() != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
     for (auto &w : waiting) ready.emplace(w.first, w.second);
     waiting.clear();
   }
-  // gives back the largest blocks until at most `most` bytes are kept
+  // gives back the largest blocks until at most `most` bytes are kept (or only
+  // waiting ones are left that do not settle)
   void trim(size_t most) {
     if (kept <= most) return;
     settle();
