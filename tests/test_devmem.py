@@ -86,3 +86,31 @@ def test_kept_blocks_go_back_when_memory_runs_out(pool):
     pool.t_free(a)
     assert pool.t_alloc(60 * GB) is not None
     assert pool.t_bytes(a) == -1
+
+
+def test_devices_do_not_share_blocks(pool):
+    """A request gets memory of the device that is current, and a freed block
+    waits for its own device, whichever is current then."""
+    pool.t_device(1)
+    a = pool.t_alloc(MB)
+    pool.t_device(0)
+    pool.t_free(a)
+    b = pool.t_alloc(MB)
+    assert b != a and pool.t_block_device(b) == 0
+    pool.t_free(b)
+    c = pool.t_alloc(MB)
+    assert c == b and (pool.t_syncs(0), pool.t_syncs(1)) == (1, 0)
+    pool.t_device(1)
+    assert pool.t_alloc(MB) == a and (pool.t_syncs(0), pool.t_syncs(1)) == (1, 1)
+
+
+def test_trim_waits_for_every_device(pool):
+    """The last handle gives back what is above 256 MB on each device, after a
+    synchronisation of that device, and leaves the current device as it was."""
+    pool.t_holder(1)
+    for dev in (1, 0):
+        pool.t_device(dev)
+        pool.t_free(pool.t_alloc(GB))
+    pool.t_holder(-1)
+    assert pool.t_used() <= 2 * 256 * MB
+    assert (pool.t_syncs(0), pool.t_syncs(1)) == (1, 1) and pool.t_current() == 0

@@ -4,19 +4,21 @@
 // GB/s: a level's bake frees 36 GB, and repeated bakes waited up to a second
 // each for that once the whole of HBM had been handed out.
 //
-// What is kept: up to 256 MiB at any time, and up to an eighth of the device's
+// What is kept on a device: up to 256 MiB at any time, and up to an eighth of its
 // memory while a scene, a transfer set or a server is alive; the rest, and
 // everything above 256 MiB when the last of them is destroyed, goes back to
 // the driver.  When the driver has no memory left, what is kept goes back
 // first.
 //
 // A block that was given back may still be read by work in flight (a caller's
-// stream, the other MakeTransfers stream), so it waits in a list of its own
-// and is handed out only after a device synchronisation, which the first
-// request that could use such a block pays for all of them.  hipFree, which
-// this stands in for, waits in the same way.
+// or a server's stream), so it waits in a list of its own and is handed out
+// only after a synchronisation of its device, which the first request that
+// could use such a block pays for all of them.  hipFree, which this stands in
+// for, waits in the same way.  Each device has its own blocks: a thread's
+// current device need not be the one a block lies on.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -29,54 +31,78 @@ namespace {
 
 constexpr size_t kKeepAlways = (size_t)256 << 20;
 
+// The blocks of one device.
+struct Device {
+  int id = 0;
+  std::multimap<size_t, void *> ready;             // blocks no work can touch
+  std::vector<std::pair<size_t, void *>> waiting;  // given back since the last synchronisation
+  size_t kept = 0, cap = 0;
+};
+struct Block {
+  size_t bytes;
+  Device *dev;
+};
+
 struct Pool {
   std::mutex mu;
-  std::multimap<size_t, void *> ready;               // blocks no work can touch
-  std::vector<std::pair<size_t, void *>> waiting;    // given back since the last synchronisation
-  std::unordered_map<void *, size_t> size;           // every block handed out or kept
-  size_t kept = 0, cap = 0;
+  std::map<int, Device> devices;
+  std::unordered_map<void *, Block> blocks;  // every block handed out or kept
   int holders = 0;
 
-  size_t limit() {
-    if (cap == 0) {
+  // the device that hipMalloc allocates on in this thread
+  Device &current() {
+    int id = 0;
+    if (hipGetDevice(&id) != hipSuccess) {
+      (void)hipGetLastError();
+      id = 0;
+    }
+    Device &D = devices[id];
+    D.id = id;
+    if (D.cap == 0) {
       size_t free_b = 0, total = 0;
       if (hipMemGetInfo(&free_b, &total) != hipSuccess) {
         (void)hipGetLastError();
         total = 0;
       }
-      cap = total / 8 > kKeepAlways ? total / 8 : kKeepAlways;
+      D.cap = std::max(total / 8, kKeepAlways);
     }
-    return holders > 0 ? cap : kKeepAlways;
+    return D;
   }
-  void drop(std::multimap<size_t, void *>::iterator it) {
-    kept -= it->first;
-    size.erase(it->second);
+  size_t limit(const Device &D) const { return holders > 0 ? D.cap : kKeepAlways; }
+  void drop(Device &D, std::multimap<size_t, void *>::iterator it) {
+    D.kept -= it->first;
+    blocks.erase(it->second);
     (void)hipFree(it->second);
-    ready.erase(it);
+    D.ready.erase(it);
   }
   // The waiting blocks become ready, unless the synchronisation fails (a stream
   // of the caller is capturing, say): then their work may still run, and they
   // wait on.
-  void settle() {
-    if (waiting.empty()) return;
-    if (hipDeviceSynchronize() != hipSuccess) {
+  void settle(Device &D) {
+    if (D.waiting.empty()) return;
+    int was = D.id;
+    (void)hipGetDevice(&was);
+    if (was != D.id) (void)hipSetDevice(D.id);
+    const hipError_t e = hipDeviceSynchronize();
+    if (was != D.id) (void)hipSetDevice(was);
+    if (e != hipSuccess) {
       (void)hipGetLastError();
       return;
     }
-    for (auto &w : waiting) ready.emplace(w.first, w.second);
-    waiting.clear();
+    for (auto &w : D.waiting) D.ready.emplace(w.first, w.second);
+    D.waiting.clear();
   }
   // gives back the largest blocks until at most `most` bytes are kept (or only
   // waiting ones are left that do not settle)
-  void trim(size_t most) {
-    if (kept <= most) return;
-    settle();
-    while (kept > most && !ready.empty()) drop(std::prev(ready.end()));
+  void trim(Device &D, size_t most) {
+    if (D.kept <= most) return;
+    settle(D);
+    while (D.kept > most && !D.ready.empty()) drop(D, std::prev(D.ready.end()));
   }
   // a kept block for a request of n bytes: at most an eighth (and a page) larger
-  std::multimap<size_t, void *>::iterator fit(size_t n) {
-    auto it = ready.lower_bound(n);
-    return it != ready.end() && it->first <= n + n / 8 + 65536 ? it : ready.end();
+  std::multimap<size_t, void *>::iterator fit(Device &D, size_t n) {
+    auto it = D.ready.lower_bound(n);
+    return it != D.ready.end() && it->first <= n + n / 8 + 65536 ? it : D.ready.end();
   }
 };
 Pool &pool() {
@@ -89,29 +115,30 @@ Pool &pool() {
 int dev_alloc(void **out, size_t n) {
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);
+  Device &D = P.current();
   // sizes step by a sixteenth, so that calls of similar sizes share blocks
   size_t step = 4096;
   while (step * 32 <= n) step *= 2;
   n = (n + step - 1) / step * step;
-  auto it = P.fit(n);
-  if (it == P.ready.end()) {
-    for (auto &w : P.waiting)
+  auto it = P.fit(D, n);
+  if (it == D.ready.end()) {
+    for (auto &w : D.waiting)
       if (w.first >= n && w.first <= n + n / 8 + 65536) {
-        P.settle();
-        it = P.fit(n);
+        P.settle(D);
+        it = P.fit(D, n);
         break;
       }
   }
-  if (it != P.ready.end()) {
+  if (it != D.ready.end()) {
     *out = it->second;
-    P.kept -= it->first;
-    P.ready.erase(it);
+    D.kept -= it->first;
+    D.ready.erase(it);
     return 0;
   }
   hipError_t e = hipMalloc(out, n);
-  if (e == hipErrorOutOfMemory && P.kept > 0) {
+  if (e == hipErrorOutOfMemory && D.kept > 0) {
     (void)hipGetLastError();
-    P.trim(0);
+    P.trim(D, 0);
     e = hipMalloc(out, n);
   }
   if (e != hipSuccess) {
@@ -119,7 +146,7 @@ int dev_alloc(void **out, size_t n) {
     (void)hipGetLastError();
     return (int)e;
   }
-  P.size[*out] = n;
+  P.blocks[*out] = Block{n, &D};
   return 0;
 }
 
@@ -127,24 +154,26 @@ void dev_free(void *p) {
   if (!p) return;
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);
-  auto it = P.size.find(p);
-  if (it == P.size.end()) return;
-  const size_t n = it->second, lim = P.limit();
+  auto it = P.blocks.find(p);
+  if (it == P.blocks.end()) return;
+  Device &D = *it->second.dev;
+  const size_t n = it->second.bytes, lim = P.limit(D);
   if (n > lim) {
-    P.size.erase(it);
+    P.blocks.erase(it);
     (void)hipFree(p);
     return;
   }
-  P.trim(lim - n);
-  P.waiting.emplace_back(n, p);
-  P.kept += n;
+  P.trim(D, lim - n);
+  D.waiting.emplace_back(n, p);
+  D.kept += n;
 }
 
 void dev_holder(int delta) {
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);
   P.holders += delta;
-  if (P.holders <= 0) P.trim(kKeepAlways);
+  if (P.holders <= 0)
+    for (auto &d : P.devices) P.trim(d.second, kKeepAlways);
 }
 
 }  // namespace vr
