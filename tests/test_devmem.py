@@ -114,3 +114,22 @@ def test_trim_waits_for_every_device(pool):
     pool.t_holder(-1)
     assert pool.t_used() <= 2 * 256 * MB
     assert (pool.t_syncs(0), pool.t_syncs(1)) == (1, 1) and pool.t_current() == 0
+
+
+def test_requests_that_fit_the_device_are_served(pool):
+    """Sizes are rounded up so that similar requests share blocks, but what that
+    adds is bounded (1/128 of the device), so it does not take the memory that a
+    set near the device's capacity needs."""
+    pool.t_holder(1)
+    blocks = [pool.t_alloc(6300 * MB) for _ in range(10)]  # 61.5 of 64 GB
+    assert all(blocks) and pool.t_used() <= 63000 * MB + 512 * MB
+    assert pool.t_alloc(64 * GB - pool.t_used()) is not None  # to the last byte
+    assert pool.t_used() == 64 * GB
+
+
+def test_similar_requests_share_a_block(pool):
+    pool.t_holder(1)
+    for n in (1001 * MB, 1010 * MB, 990 * MB):
+        a = pool.t_alloc(n)
+        pool.t_free(a)
+    assert pool.t_used() < 1100 * MB

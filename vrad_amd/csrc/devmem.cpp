@@ -37,9 +37,10 @@ struct Device {
   std::multimap<size_t, void *> ready;             // blocks no work can touch
   std::vector<std::pair<size_t, void *>> waiting;  // given back since the last synchronisation
   size_t kept = 0, cap = 0;
+  size_t spare = 0;  // bytes of handed-out blocks beyond what was asked for
 };
 struct Block {
-  size_t bytes;
+  size_t bytes, spare;
   Device *dev;
 };
 
@@ -99,10 +100,21 @@ struct Pool {
     settle(D);
     while (D.kept > most && !D.ready.empty()) drop(D, std::prev(D.ready.end()));
   }
-  // a kept block for a request of n bytes: at most an eighth (and a page) larger
-  std::multimap<size_t, void *>::iterator fit(Device &D, size_t n) {
+  // Whether n more bytes than asked for may be handed out: 1/128 of the device
+  // in all, so that a set of blocks near its capacity still fits.
+  static bool can_spare(const Device &D, size_t n) { return D.spare + n <= D.cap / 16; }
+  // a kept block for a request of n bytes rounded to r: at most an eighth (and
+  // a page) larger
+  static std::multimap<size_t, void *>::iterator fit(Device &D, size_t n, size_t r) {
     auto it = D.ready.lower_bound(n);
-    return it != D.ready.end() && it->first <= n + n / 8 + 65536 ? it : D.ready.end();
+    return it != D.ready.end() && fits(D, it->first, n, r) ? it : D.ready.end();
+  }
+  static bool fits(const Device &D, size_t have, size_t n, size_t r) {
+    return have >= n && have <= r + r / 8 + 65536 && can_spare(D, have - n);
+  }
+  void hand_out(Device &D, void *p, size_t bytes, size_t n) {
+    blocks[p] = Block{bytes, bytes - n, &D};
+    D.spare += bytes - n;
   }
 };
 Pool &pool() {
@@ -119,34 +131,40 @@ int dev_alloc(void **out, size_t n) {
   // sizes step by a sixteenth, so that calls of similar sizes share blocks
   size_t step = 4096;
   while (step * 32 <= n) step *= 2;
-  n = (n + step - 1) / step * step;
-  auto it = P.fit(D, n);
+  const size_t r = (n + step - 1) / step * step;
+  auto it = P.fit(D, n, r);
   if (it == D.ready.end()) {
     for (auto &w : D.waiting)
-      if (w.first >= n && w.first <= n + n / 8 + 65536) {
+      if (P.fits(D, w.first, n, r)) {
         P.settle(D);
-        it = P.fit(D, n);
+        it = P.fit(D, n, r);
         break;
       }
   }
   if (it != D.ready.end()) {
     *out = it->second;
+    P.hand_out(D, it->second, it->first, n);
     D.kept -= it->first;
     D.ready.erase(it);
     return 0;
   }
-  hipError_t e = hipMalloc(out, n);
+  size_t bytes = P.can_spare(D, r - n) ? r : n;
+  hipError_t e = hipMalloc(out, bytes);
   if (e == hipErrorOutOfMemory && D.kept > 0) {
     (void)hipGetLastError();
     P.trim(D, 0);
-    e = hipMalloc(out, n);
+    e = hipMalloc(out, bytes);
+  }
+  if (e == hipErrorOutOfMemory && bytes > n) {
+    (void)hipGetLastError();
+    e = hipMalloc(out, bytes = n);
   }
   if (e != hipSuccess) {
     *out = nullptr;
     (void)hipGetLastError();
     return (int)e;
   }
-  P.blocks[*out] = Block{n, &D};
+  P.hand_out(D, *out, bytes, n);
   return 0;
 }
 
@@ -158,6 +176,8 @@ void dev_free(void *p) {
   if (it == P.blocks.end()) return;
   Device &D = *it->second.dev;
   const size_t n = it->second.bytes, lim = P.limit(D);
+  D.spare -= it->second.spare;
+  it->second.spare = 0;
   if (n > lim) {
     P.blocks.erase(it);
     (void)hipFree(p);
