@@ -71,6 +71,13 @@ const char *vr_last_error(void);
  * by the first entry point that needs the GPU.  No reference counterpart
  * (the reference is single-process CPU code). */
 int vr_init(int device);
+/* Device memory that the library has freed stays with it for its next calls:
+ * up to 256 MiB at any time, and up to an eighth of the device's memory while
+ * a scene built on the device, a transfer set or a server is alive.  It goes
+ * back by itself when a call of the library needs memory or the last such
+ * handle is destroyed; this call gives all of it back now, for other
+ * allocators of the process.  Waits for the device.  No reference counterpart. */
+int vr_release_memory(void);
 /* Select VR_PATH_OPT / VR_PATH_PLAIN for the calls that follow. */
 int vr_set_path(int path);
 /* Kernel-shape knobs (the autotuner's interface; no reference counterpart).

@@ -29,7 +29,7 @@ def pool(built, tmp_path):
     lib = C.CDLL(str(so))
     for name in ("t_alloc",):
         getattr(lib, name).restype = C.c_void_p
-    for name in ("t_used", "t_bytes", "t_syncs"):
+    for name in ("t_used", "t_bytes", "t_syncs", "t_release"):
         getattr(lib, name).restype = C.c_int64
     lib.t_alloc.argtypes = lib.t_setup.argtypes = [C.c_int64]
     lib.t_free.argtypes = lib.t_bytes.argtypes = lib.t_block_device.argtypes = [C.c_void_p]
@@ -133,3 +133,41 @@ def test_similar_requests_share_a_block(pool):
         a = pool.t_alloc(n)
         pool.t_free(a)
     assert pool.t_used() < 1100 * MB
+
+
+def test_release_gives_everything_back(pool):
+    """All kept blocks of every device; those whose work may still run stay."""
+    pool.t_holder(1)
+    for dev in (1, 0):
+        pool.t_device(dev)
+        pool.t_free(pool.t_alloc(GB))
+    pool.t_sync_error(1)
+    assert pool.t_release() == 2 * GB == pool.t_used()
+    pool.t_sync_error(0)
+    assert pool.t_release() == 0 == pool.t_used()
+
+
+@pytest.mark.gpu
+def test_released_memory_is_there_for_others():
+    """With a scene alive, freed transfers stay with the library until they are
+    asked for; then another allocator of the process gets them."""
+    import torch
+    import vrad_amd
+    from vrad_amd import _lib, scenes
+    from vrad_amd.patches import Transfers
+    from vrad_amd.raytracer import Environment
+    _lib.check(_lib.lib.vr_init(0))
+    s = scenes.room(seed=1, n_pillars=2, chop=128.0, tess=128.0)
+    env = Environment()
+    env.AddTriangles(s.verts9, s.ids)
+    env.SetupAccelerationStructure()
+    vrad_amd.release_memory()
+    xf = Transfers.synthetic(seed=1, n_rows=1 << 18, mean_len=512.0, sigma=0.0, max_len=600)
+    held = xf.info().stored_bytes
+    assert held > GB
+    before = torch.cuda.mem_get_info()[0]
+    xf.close()
+    kept = torch.cuda.mem_get_info()[0]
+    assert kept - before < held // 2
+    vrad_amd.release_memory()
+    assert torch.cuda.mem_get_info()[0] - before >= held * 9 // 10

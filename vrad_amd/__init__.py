@@ -7,6 +7,15 @@ from .trace import TestLineDoesHitSky
 from .patches import MakeTransfers, Transfers
 from .lightmap import GatherSampleLight, BounceLight
 
+
+
+def release_memory():
+    """Gives the device memory that the library keeps for its next calls (up to
+    an eighth of the device) back to the driver, for the process's other
+    allocators."""
+    _lib.check(_lib.lib.vr_release_memory())
+
+
 __all__ = ["Environment", "GetEnvironment", "FourRays", "RayTracingResult",
            "TestLineDoesHitSky", "MakeTransfers", "Transfers", "GatherSampleLight",
-           "BounceLight", "VrError"]
+           "BounceLight", "VrError", "release_memory"]

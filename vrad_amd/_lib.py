@@ -134,6 +134,7 @@ _P = C.c_void_p
 _SIGS = {
     "vr_last_error": (C.c_char_p, []),
     "vr_init": (C.c_int, [C.c_int]),
+    "vr_release_memory": (C.c_int, []),
     "vr_set_path": (C.c_int, [C.c_int]),
     "vr_set_tuning": (C.c_int, [C.c_char_p, C.c_int]),
     "vr_get_tuning": (C.c_int, [C.c_char_p, C.POINTER(C.c_int)]),

@@ -557,6 +557,13 @@ int vr_init(int device) {
   return ensure_init();
 }
 
+int vr_release_memory(void) {
+  LOCK;
+  if (dev_release() != 0)
+    return fail(VR_E_HIP, "memory still in use: the device does not synchronise");
+  return VR_OK;
+}
+
 int vr_set_path(int path) {
   LOCK;
   if (path != VR_PATH_OPT && path != VR_PATH_PLAIN) return fail(VR_E_INVALID, "unknown path");

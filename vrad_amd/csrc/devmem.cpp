@@ -8,7 +8,7 @@
 // memory while a scene, a transfer set or a server is alive; the rest, and
 // everything above 256 MiB when the last of them is destroyed, goes back to
 // the driver.  When the driver has no memory left, what is kept goes back
-// first.
+// first, and dev_release gives it back at any time.
 //
 // A block that was given back may still be read by work in flight (a caller's
 // or a server's stream), so it waits in a list of its own and is handed out
@@ -188,12 +188,24 @@ void dev_free(void *p) {
   D.kept += n;
 }
 
-void dev_holder(int delta) {
+int dev_holder(int delta) {
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);
   P.holders += delta;
   if (P.holders <= 0)
     for (auto &d : P.devices) P.trim(d.second, kKeepAlways);
+  return P.holders;
+}
+
+size_t dev_release() {
+  Pool &P = pool();
+  std::lock_guard<std::mutex> lock(P.mu);
+  size_t left = 0;
+  for (auto &d : P.devices) {
+    P.trim(d.second, 0);
+    left += d.second.kept;
+  }
+  return left;
 }
 
 }  // namespace vr

@@ -19,7 +19,11 @@ int fail(int code, const std::string &msg);
 // Blocks are kept and handed out again; dev_alloc returns 0 or the hipError_t.
 int dev_alloc(void **out, size_t n);
 void dev_free(void *p);  // work in flight may still use the block
-void dev_holder(int delta);  // scenes, transfer sets and servers alive
+// scenes built on the device, transfer sets and servers alive, after the change
+int dev_holder(int delta);
+// gives every kept block back to the driver; the bytes that could not be (their
+// device does not synchronise, say while a stream is being captured)
+size_t dev_release();
 struct DevHolder {
   DevHolder() { dev_holder(1); }
   ~DevHolder() { dev_holder(-1); }
