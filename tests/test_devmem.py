@@ -171,3 +171,18 @@ def test_released_memory_is_there_for_others():
     assert kept - before < held // 2
     vrad_amd.release_memory()
     assert torch.cuda.mem_get_info()[0] - before >= held * 9 // 10
+
+
+def test_host_scenes_hold_no_memory():
+    """A scene that was never built on the device does not raise what is kept."""
+    from vrad_amd import _lib
+    import numpy as np
+    count = getattr(_lib.lib, "_ZN2vr10dev_holderEi")
+    before = count(0)
+    h, v9, ids = C.c_void_p(), np.zeros((1, 9), np.float32), np.zeros(1, np.int32)
+    v9[0, 3] = v9[0, 7] = 1.0
+    _lib.check(_lib.lib.vr_scene_create(C.byref(h), _lib.ptr(v9), _lib.ptr(ids), None, 1))
+    _lib.check(_lib.lib.vr_scene_build_host(h, 1))
+    assert count(0) == before
+    _lib.check(_lib.lib.vr_scene_destroy(h))
+    assert count(0) == before

@@ -233,7 +233,7 @@ using namespace vr;
 
 // ---------------------------------------------------------------------------
 struct vr_scene {
-  DevHolder holder;
+  std::unique_ptr<DevHolder> holder;  // once built on the device
   int64_t n_tri = 0;
   std::vector<float> v9;
   std::vector<int32_t> ids;
@@ -781,6 +781,7 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
   LOCK;
   if (!s) return fail(VR_E_INVALID, "scene is NULL");
   TRY(ensure_init());
+  if (!s->holder) s->holder.reset(new DevHolder);
   g_pin.begin();
   const int kb = tuning().kd_build;
   const bool device = kb == 1 || (kb == 2 && s->n_tri >= tuning().kd_build_device_min);
