@@ -11,6 +11,7 @@
 #include <hip/hip_fp16.h>
 
 #include "kernels.h"
+#include "launch_plan.h"
 
 namespace vr {
 
@@ -953,12 +954,13 @@ __global__ __launch_bounds__(1024 / SP) void k_bounce_stream(const BounceJob *__
 // Blocked layout, pass 1: one workgroup per block (c, t): padded segment
 // lengths of the 1024 owner slots, exclusive scan -> boff (stride 1028),
 // total -> btot.
-__global__ __launch_bounds__(1024) void k_block_offsets(DevXfers x, DevTiles tl, int G,
+__global__ __launch_bounds__(1024) void k_block_offsets(DevXfers x, DevTiles tl,
+                                                        int64_t block0, int G,
                                                         int64_t *__restrict__ btot,
                                                         int32_t *__restrict__ boff) {
   __shared__ int64_t sc[1024];
   const int R = 1024, RS = R + 4;
-  const int64_t blk = blockIdx.x;  // c * nt + t
+  const int64_t blk = block0 + blockIdx.x;  // c * nt + t
   const int64_t c = blk / tl.nt;
   const int t = (int)(blk % tl.nt);
   const int u = threadIdx.x;
@@ -998,13 +1000,15 @@ __global__ __launch_bounds__(1024) void k_block_offsets(DevXfers x, DevTiles tl,
 // offsets and one of coefficients.  Bound by latency and, before chunks per
 // lane, by index arithmetic: entry by entry with a wave per 64 slots 5,970
 // rows of 3.2 M transfers took 116 us (now 45), 341,299 rows of 1.56 G 10.4 ms
-// (now 8.4).
-__global__ __launch_bounds__(256) void k_block_fill(DevXfers x, DevTiles tl, int slots,
-                                                    int coef_bytes, uint16_t *__restrict__ bidx,
+// (now 8.4).  group0: the launch's first workgroup (long grids go in parts).
+__global__ __launch_bounds__(256) void k_block_fill(DevXfers x, DevTiles tl, int64_t group0,
+                                                    int slots, int coef_bytes,
+                                                    uint16_t *__restrict__ bidx,
                                                     void *__restrict__ bcoef) {
   const int lane = threadIdx.x & 63;
   const int R = 1024, RS = R + 4, nw = R / slots;
-  const int64_t gw = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t gw =
+      (group0 + blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t nblk = tl.n_chunks * (int64_t)tl.nt;
   if (gw >= nblk * nw) return;
   const int64_t blk = gw / nw;
@@ -1088,21 +1092,17 @@ __global__ __launch_bounds__(256) void k_block_fill(DevXfers x, DevTiles tl, int
 void launch_block_offsets(const DevXfers &x, const DevTiles &tl, int G, int64_t *btot,
                           int32_t *boff, hipStream_t st) {
   const int64_t nblk = tl.n_chunks * (int64_t)tl.nt;
-  if (nblk <= 0) return;
-  hipLaunchKernelGGL(k_block_offsets, dim3((unsigned)nblk), dim3(1024), 0, st, x, tl, G, btot,
-                     boff);
+  for (int64_t b = 0; b < nblk; b += grid_part(b, nblk, 1024))
+    hipLaunchKernelGGL(k_block_offsets, dim3((unsigned)grid_part(b, nblk, 1024)), dim3(1024), 0, st,
+                       x, tl, b, G, btot, boff);
 }
 
 void launch_block_fill(const DevXfers &x, const DevTiles &tl, int coef_bytes,
                        uint16_t *bidx, void *bcoef, hipStream_t st) {
-  // 16 slots a wave where that still makes 16 K waves: with a PVS most of a
-  // large system's blocks are empty, and a wave costs more than its lookups
-  const int64_t nblk = tl.n_chunks * (int64_t)tl.nt;
-  const int slots = nblk * 64 >= 16384 ? 16 : 4;
-  const int64_t waves = nblk * (1024 / slots);
-  if (waves <= 0) return;
-  hipLaunchKernelGGL(k_block_fill, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, x, tl,
-                     slots, coef_bytes, bidx, bcoef);
+  const int64_t nblk = tl.n_chunks * (int64_t)tl.nt, groups = block_fill_groups(nblk);
+  for (int64_t g = 0; g < groups; g += grid_part(g, groups, 256))
+    hipLaunchKernelGGL(k_block_fill, dim3((unsigned)grid_part(g, groups, 256)), dim3(256), 0, st, x,
+                       tl, g, block_fill_slots(nblk), coef_bytes, bidx, bcoef);
 }
 
 // tile boundaries per row: tp[r][t] = first row position with column >= t*C
