@@ -177,14 +177,17 @@ def MakePatches(faces, max_chop=MAX_CHOP, min_chop=MIN_CHOP, vertex_normals=None
             raise ValueError(f"vertex_normals: shape {vn.shape}, want "
                              f"({len(f)}, {_lib.VR_FACE_MAX_POINTS}, 3)")
     n = C.c_int64()
-    # room for the patches a face of these lightmap extents usually gives (pages
-    # that are not written cost nothing); a count that exceeds it comes back
-    # with the capacity error and is asked for again
-    out = np.empty(_patch_room(f, float(max_chop)), _lib.PATCH_DTYPE)
+    # room for the patches that faces of these lightmap extents usually give
+    # (pages that are not written cost nothing); without it, or when there are
+    # more, the library says how many
+    try:
+        out = np.empty(_patch_room(f, float(max_chop)), _lib.PATCH_DTYPE)
+    except MemoryError:  # the room is generous
+        out = np.empty(0, _lib.PATCH_DTYPE)
     for _ in range(2):
         rc = lib.vr_make_patches_phong(ptr(f), len(f), float(max_chop), float(min_chop), ptr(vn),
-                                       ptr(out), len(out), C.byref(n))
-        if rc != _lib.VR_E_CAPACITY or n.value <= len(out):
+                                       ptr(out) if len(out) else None, len(out), C.byref(n))
+        if rc not in (_lib.VR_OK, _lib.VR_E_CAPACITY) or n.value <= len(out):
             break
         out = np.empty(n.value, _lib.PATCH_DTYPE)
     check(rc)
@@ -193,8 +196,8 @@ def MakePatches(faces, max_chop=MAX_CHOP, min_chop=MIN_CHOP, vertex_normals=None
 
 def _patch_room(faces, max_chop):
     """Patches the faces may give: leaves of at least half a chop a side, and
-    as many inner patches again."""
-    if len(faces) == 0:
+    as many inner patches again; 0 when max_chop gives no estimate."""
+    if len(faces) == 0 or not max_chop > 0.0:
         return 0
     used = np.arange(_lib.VR_FACE_MAX_POINTS)[None, :, None] < faces["n_points"][:, None, None]
     lux = np.stack([faces["lux_s"], faces["lux_t"]], 2)
