@@ -35,4 +35,5 @@ def test_any_room_gives_the_same_patches(monkeypatch, room):
     monkeypatch.setattr(patches, "_patch_room", lambda *_: room)
     got = patches.MakePatches(f, max_chop=4.0, min_chop=4.0)
     assert got.tobytes() == want.tobytes()
+    assert got.base is None and got.flags.owndata and want.base is None
     assert len(patches.MakePatches(f[:0])) == 0

@@ -191,7 +191,8 @@ def MakePatches(faces, max_chop=MAX_CHOP, min_chop=MIN_CHOP, vertex_normals=None
             break
         out = np.empty(n.value, _lib.PATCH_DTYPE)
     check(rc)
-    return out[:n.value]
+    out.resize(n.value, refcheck=False)  # in place: the rest of the room goes back
+    return out
 
 
 def _patch_room(faces, max_chop):
