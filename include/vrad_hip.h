@@ -226,7 +226,11 @@ typedef struct {
   float normal_offset;  /* segment end offset along each normal (0.1) */
   int32_t skip_id;
   int32_t normalize;    /* scale rows with FP64 sum > 1 by 1/sum */
-  int64_t batch_pairs;  /* candidate pairs per visibility batch (<=0: 32M); no effect on results */
+  /* candidate pairs per visibility launch, at least one row's run of them
+   * (<=0: no bound where rows are culled and traced in one launch, 32M where
+   * the pairs are listed first: the plain path, trees too large for the
+   * hierarchy); no effect on results */
+  int64_t batch_pairs;
 } vr_xfer_params;
 typedef struct vr_xfers vr_xfers;
 typedef struct {
@@ -245,10 +249,10 @@ int vr_make_transfers(vr_scene *s, const vr_patches *p, int64_t n_patches,
 /* MakeTransfers for many scenes at once (no reference counterpart): scene
  * k's patches[k] (n_patches[k] of them) give out[k],
  * equal bit for bit to vr_make_transfers(scenes[k], ...).  One visibility
- * launch culls and traces the scenes' candidate pairs through a table of
- * scene descriptors.  A scene with params->batch_pairs candidate pairs
- * (default 32M) or more fills the GPU alone and runs as vr_make_transfers
- * would.  The plain path runs the scenes one by
+ * launch (of at most params->batch_pairs pairs, if set) culls and traces the
+ * scenes' candidate pairs through a table of scene descriptors.  A scene with
+ * params->batch_pairs candidate pairs (default 32M) or more fills the GPU
+ * alone and runs as vr_make_transfers would.  The plain path runs the scenes one by
  * one.
  * On failure no out[k] is set. */
 int vr_make_transfers_batch(vr_scene *const *scenes, const vr_patches *patches,

@@ -12,6 +12,7 @@ extern "C" {
 int64_t grid_part(int64_t at, int64_t n, int t) { return vr::grid_part(at, n, t); }
 int block_fill_slots(int64_t b) { return vr::block_fill_slots(b); }
 int64_t block_fill_groups(int64_t b) { return vr::block_fill_groups(b); }
+int64_t pair_launch_groups(int64_t p, int c) { return vr::pair_launch_groups(p, c); }
 }
 """
 
@@ -26,6 +27,8 @@ def plan(tmp_path_factory):
     lib = C.CDLL(so)
     for f in (lib.grid_part, lib.block_fill_slots, lib.block_fill_groups):
         f.restype = C.c_int64
+    lib.pair_launch_groups.restype = C.c_int64
+    lib.pair_launch_groups.argtypes = [C.c_int64, C.c_int]
     lib.grid_part.argtypes = [C.c_int64, C.c_int64, C.c_int]
     lib.block_fill_slots.argtypes = lib.block_fill_groups.argtypes = [C.c_int64]
     return lib
@@ -56,3 +59,14 @@ def test_blocked_copy_launches(plan, rows, cols):
     fill = parts(plan, plan.block_fill_groups(blocks), 256)
     assert len(fill) == 1 or rows > 2 ** 20  # ordinary sets: one launch
     parts(plan, blocks, 1024)  # the offsets' launch, a workgroup per block
+
+
+@pytest.mark.parametrize("chunk", [256, 1024, 8192])
+@pytest.mark.parametrize("batch", [-1, 0, 1, 5000, 50000, 32 << 20, 2 ** 31 - 1])
+def test_pair_launch_is_bounded(plan, batch, chunk):
+    """A launch of MakeTransfers' trace holds batch_pairs candidate pairs at
+    most, or one workgroup's run of them; in any case it fits a launch."""
+    groups = plan.pair_launch_groups(batch, chunk)
+    assert groups >= 1 and groups * 64 < 2 ** 32
+    if batch > 0:
+        assert groups == 1 or groups * chunk <= batch

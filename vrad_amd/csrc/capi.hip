@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "kernels.h"
+#include "launch_plan.h"
 #include "vr_internal.h"
 
 namespace vr {
@@ -1251,8 +1252,8 @@ static int make_transfers_impl(vr_scene *s, const vr_patches *p, int64_t np,
     };
     if (fused) {
       vr::PairJob j = pair_job(s->dev, dp, plan, S, bits, np, words);
-      launch_pair_rows(j, n_blk, P.normal_offset, P.skip_id, tuning().trace_lds_entries,
-                       tuning().trace_xcd_group, st);
+      launch_pair_rows(j, n_blk, pair_launch_groups(P.batch_pairs, j.chunk), P.normal_offset,
+                       P.skip_id, tuning().trace_lds_entries, tuning().trace_xcd_group, st);
       launch_bits_mirror(bits.as<uint32_t>(), j.flags, np, words, st);
       TRY(check_launch());
     } else if (nc > 0) {
@@ -1372,6 +1373,7 @@ static int make_transfers_shared(vr_scene *const *scenes, const vr_patches *patc
   std::vector<One> sc((size_t)n_scenes);
   std::vector<vr::PairJob> jobs;
   int64_t blocks = 0;
+  int chunk = 1;  // the most columns of any scene's block
   if (budget >= (1ll << 31)) return fail(VR_E_INVALID, "batch_pairs too large");
   for (int32_t k = 0; k < n_scenes; ++k) {
     One &o = sc[(size_t)k];
@@ -1401,13 +1403,15 @@ static int make_transfers_shared(vr_scene *const *scenes, const vr_patches *patc
                             o.bits, np, o.words));
     jobs.back().blk_begin = blocks;
     blocks += o.plan.blk_pre.back();
+    chunk = std::max(chunk, o.plan.chunk);
   }
   DBuf d_jobs;
   TRY(upload_vec(d_jobs, jobs, st));
   {
     Prof pr("make_transfers", st);
-    launch_pair_rows_jobs(d_jobs.as<vr::PairJob>(), (int)jobs.size(), blocks, P.normal_offset,
-                          P.skip_id, tuning().trace_lds_entries, st);
+    launch_pair_rows_jobs(d_jobs.as<vr::PairJob>(), (int)jobs.size(), blocks,
+                          pair_launch_groups(P.batch_pairs, chunk), P.normal_offset, P.skip_id,
+                          tuning().trace_lds_entries, st);
     TRY(check_launch());
     for (int32_t k = 0; k < n_scenes; ++k) {
       One &o = sc[(size_t)k];

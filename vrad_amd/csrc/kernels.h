@@ -130,10 +130,11 @@ __host__ __device__ constexpr int64_t flag_stride(int64_t words) {
   return (words + 4 * kTileW - 1) / (4 * kTileW) * 4;
 }
 int pair_chunk(int64_t pairs);  // columns per block for a total of candidate pairs
-void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip, int lds_entries,
-                      int xcd_group, hipStream_t st);
-void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float eps, int32_t skip,
-                           int lds_entries, hipStream_t st);
+// per: blocks per launch (pair_launch_groups)
+void launch_pair_rows(const PairJob &job, int64_t n_blk, int64_t per, float eps, int32_t skip,
+                      int lds_entries, int xcd_group, hipStream_t st);
+void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, int64_t per, float eps,
+                           int32_t skip, int lds_entries, hipStream_t st);
 // bits |= transpose(bits)
 void launch_bits_mirror(uint32_t *bits, uint8_t *flags, int64_t np, int64_t words,
                         hipStream_t st);

@@ -21,4 +21,13 @@ inline int64_t block_fill_groups(int64_t blocks) {
   return blocks * (1024 / block_fill_slots(blocks)) / 4;
 }
 
+// Workgroups per launch of MakeTransfers' trace, of `chunk` candidate pairs
+// each: 16 M (a launch's tail costs more than it could give back), or as many
+// as the caller's batch_pairs (> 0) allow, at least one.
+inline int64_t pair_launch_groups(int64_t batch_pairs, int chunk) {
+  constexpr int64_t kMost = (int64_t)1 << 24;
+  if (batch_pairs <= 0) return kMost;
+  return std::min(kMost, std::max<int64_t>(1, batch_pairs / chunk));
+}
+
 }  // namespace vr

@@ -278,12 +278,11 @@ int pair_chunk(int64_t pairs) {
     case 24: X(24); break;                                                                 \
     default: X(8); break;                                                                  \
   }
-constexpr int64_t kGridMax = (int64_t)1 << 24;  // workgroups per launch
 
-void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip, int lds_entries,
-                      int xcd_group, hipStream_t st) {
-  for (int64_t b = 0; b < n_blk; b += kGridMax) {
-    const dim3 grid((unsigned)std::min(kGridMax, n_blk - b));
+void launch_pair_rows(const PairJob &job, int64_t n_blk, int64_t per, float eps, int32_t skip,
+                      int lds_entries, int xcd_group, hipStream_t st) {
+  for (int64_t b = 0; b < n_blk; b += per) {
+    const dim3 grid((unsigned)std::min(per, n_blk - b));
 #define VR_ROWS(S)                                                                        \
   hipLaunchKernelGGL((k_pair_rows<S>), grid, dim3(64), 0, st, job, b, eps, skip, (uint32_t)xcd_group)
     VR_BY_LDS(VR_ROWS)
@@ -291,10 +290,10 @@ void launch_pair_rows(const PairJob &job, int64_t n_blk, float eps, int32_t skip
   }
 }
 
-void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, float eps, int32_t skip,
-                           int lds_entries, hipStream_t st) {
-  for (int64_t b = 0; n_jobs > 0 && b < n_blk; b += kGridMax) {
-    const dim3 grid((unsigned)std::min(kGridMax, n_blk - b));
+void launch_pair_rows_jobs(const PairJob *jobs, int n_jobs, int64_t n_blk, int64_t per, float eps,
+                           int32_t skip, int lds_entries, hipStream_t st) {
+  for (int64_t b = 0; n_jobs > 0 && b < n_blk; b += per) {
+    const dim3 grid((unsigned)std::min(per, n_blk - b));
 #define VR_ROWS(S) \
   hipLaunchKernelGGL((k_pair_rows_jobs<S>), grid, dim3(64), 0, st, jobs, n_jobs, b, eps, skip)
     VR_BY_LDS(VR_ROWS)
