@@ -101,6 +101,11 @@ int vr_set_path(int path);
  *                        (main or sky) of "kd_build_device_min" (default
  *                        2048) triangles or more; the tree is the same bit
  *                        for bit
+ *   "bvh_levels"         levels (1..21, default 21) that vr_scene_build takes
+ *                        from the clustered visibility hierarchy; a deeper
+ *                        one is built balanced instead
+ *   "bvh_max_nodes"      hierarchy nodes (0..2^25, default 2^25) from which a
+ *                        scene built after it walks the kd-tree
  *   "patch_build"        vr_make_patches: 1 (default) = level-parallel (every
  *                        patch of a subdivision level split by its own
  *                        thread, then renumbered), 0 = a thread per face;

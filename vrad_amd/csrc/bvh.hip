@@ -679,7 +679,8 @@ int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, 
     int levels = 0;
     int64_t total = 0;
     while (levels < 126 && hl[levels] > 0) total += hl[levels++];
-    if (levels <= kMaxLevels && hl[level] == 0) {
+    const int most = pass == 0 ? std::min(kMaxLevels, tuning().bvh_levels) : kMaxLevels;
+    if (levels <= most && hl[level] == 0) {
       out->n_nodes = total;
       out->n_refs = hl[127];
       out->levels = levels;

@@ -622,6 +622,13 @@ int vr_set_tuning(const char *name, int value) {
   } else if (k == "kd_build_device_min") {
     if (value < 0) return fail(VR_E_INVALID, "kd_build_device_min must be >= 0");
     tuning().kd_build_device_min = value;
+  } else if (k == "bvh_levels") {
+    if (value < 1 || value > kBvhStack / 3)
+      return fail(VR_E_INVALID, "bvh_levels must be 1.." + std::to_string(kBvhStack / 3));
+    tuning().bvh_levels = value;
+  } else if (k == "bvh_max_nodes") {
+    if (value < 0 || value > 1 << 25) return fail(VR_E_INVALID, "bvh_max_nodes must be 0..2^25");
+    tuning().bvh_max_nodes = value;
   } else if (k == "patch_build") {
     if (value < 0 || value > 1)
       return fail(VR_E_INVALID, "patch_build must be 0 (a thread per face) or 1 (level-parallel)");
@@ -648,6 +655,8 @@ int vr_get_tuning(const char *name, int *value) {
   else if (k == "bounce_placement") *value = tuning().bounce_placement;
   else if (k == "kd_build") *value = tuning().kd_build;
   else if (k == "kd_build_device_min") *value = tuning().kd_build_device_min;
+  else if (k == "bvh_levels") *value = tuning().bvh_levels;
+  else if (k == "bvh_max_nodes") *value = tuning().bvh_max_nodes;
   else if (k == "patch_build") *value = tuning().patch_build;
   else return fail(VR_E_INVALID, "unknown tuning knob " + k);
   return VR_OK;
@@ -820,7 +829,7 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
     bvh.bytes = 128 * (size_t)b.n_nodes;
     bvh_refs.p = b.refs;
     bvh_refs.bytes = 48 * (size_t)b.n_refs;
-    if (b.n_nodes >= (1 << 25)) d.has_bvh = 0;
+    if (b.n_nodes >= tuning().bvh_max_nodes) d.has_bvh = 0;
     return rc;
   };
   d.has_bvh = 1;

@@ -37,6 +37,9 @@ struct Tuning {
   // kd-tree construction in vr_scene_build (the same tree either way)
   int kd_build = 2;                 // 0 = host threads, 1 = GPU, 2 = GPU from a size on
   int kd_build_device_min = 2048;   // triangles at which kd_build = 2 uses the GPU
+  // the visibility hierarchy (the same results either way)
+  int bvh_levels = kBvhStack / 3;   // a deeper clustered tree is built balanced instead
+  int bvh_max_nodes = 1 << 25;      // 128-byte nodes from which scenes walk the kd-tree
   // patch generation in vr_make_patches (the same patches either way)
   int patch_build = 1;              // 0 = a thread per face, 1 = level-parallel
 };
