@@ -841,8 +841,11 @@ int build(const float *v9_host, int64_t n, hipStream_t st, KdTree *out) {
     if (lerr)
       return fail(VR_E_STATE, "kd-tree build: inconsistent partition (" + std::to_string(lerr) + ")");
     if (th[0] == 0) break;
-    if (th[0] >= ((int64_t)1 << 30) || th[1] >= ((int64_t)1 << 31) - 1)
-      KD_TRY(fail(VR_E_CAPACITY, "kd-tree level exceeds 2^30 nodes or 2^31 references"));
+    // a scene's tree holds fewer than 2^24 nodes in all, so that a level's
+    // launches fit (32 lanes per node and axis)
+    static_assert(((int64_t)96 << kStackNodeBits) < ((int64_t)1 << 32), "k_kd_cands' grid");
+    if (th[0] >= ((int64_t)1 << kStackNodeBits) || th[1] >= ((int64_t)1 << 31) - 1)
+      KD_TRY(fail(VR_E_CAPACITY, "kd-tree level of 2^24 nodes or 2^31 references"));
     if (L + 1 > (size_t)kKdMaxDepth + 2)
       KD_TRY(fail(VR_E_STATE, "kd-tree build: more levels than the depth limit allows"));
     lv.emplace_back();
