@@ -147,8 +147,6 @@ void launch_row_count(const uint32_t *bits, const uint8_t *flags, int64_t np, in
 int64_t row_order_scratch(int64_t n);
 void launch_row_order(const int32_t *cnt, int64_t n, int32_t longest, int32_t *order,
                       int32_t *scratch, hipStream_t st);
-// exclusive scan of padded lengths (multiple of 8) into rp[0..n]
-void launch_row_scan(const int32_t *cnt, int64_t n, int64_t *rp, hipStream_t st);
 void launch_row_fill(const uint32_t *bits, const uint8_t *flags, int64_t np, int64_t words,
                      const DevPatches &p, const int64_t *rp, const int32_t *cnt, int32_t *col,
                      float *coef, hipStream_t st);

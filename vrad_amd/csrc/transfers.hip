@@ -7,7 +7,8 @@
 //                   holds with room to spare).  The plain path lists the pairs
 //                   (k_pair_cull) and traces the list (k_pair_trace_plain).
 //  2. k_bits_mirror makes the matrix symmetric.
-//  3. k_row_count   popcount per row; k_row_scan pads lengths to 8 and scans.
+//  3. k_row_count   popcount per row; the host pads the lengths to 8 and sums
+//                   them up, k_sort_* order the rows longest first.
 //  4. k_row_fill    columns in ascending order, F_ij in FP32.
 //  5. k_row_norm    FP64 row sum in the bounce-kernel wave order (G = 4);
 //                   rows with sum > 1 are scaled by 1/sum.
@@ -425,38 +426,6 @@ void launch_row_count(const uint32_t *bits, const uint8_t *flags, int64_t np, in
   if (np <= 0) return;
   hipLaunchKernelGGL(k_row_count, dim3((unsigned)((np + 3) / 4)), dim3(256), 0, st, bits, flags,
                      np, words, cnt);
-}
-
-// single-block exclusive scan of padded lengths: rp[i] = sum_{k<i} pad8(cnt[k])
-__global__ __launch_bounds__(1024) void k_row_scan(const int32_t *__restrict__ cnt, int64_t n,
-                                                   int64_t *__restrict__ rp) {
-  __shared__ int64_t part[1024];
-  const int t = threadIdx.x;
-  const int64_t per = (n + 1023) / 1024;
-  const int64_t b = t * per, e = min(n, b + per);
-  int64_t s = 0;
-  for (int64_t k = b; k < e; ++k) s += ((int64_t)cnt[k] + 7) & ~(int64_t)7;
-  part[t] = s;
-  __syncthreads();
-  if (t == 0) {
-    int64_t run = 0;
-    for (int k = 0; k < 1024; ++k) {
-      int64_t v = part[k];
-      part[k] = run;
-      run += v;
-    }
-    rp[n] = run;
-  }
-  __syncthreads();
-  int64_t run = part[t];
-  for (int64_t k = b; k < e; ++k) {
-    rp[k] = run;
-    run += ((int64_t)cnt[k] + 7) & ~(int64_t)7;
-  }
-}
-
-void launch_row_scan(const int32_t *cnt, int64_t n, int64_t *rp, hipStream_t st) {
-  hipLaunchKernelGGL(k_row_scan, dim3(1), dim3(1024), 0, st, cnt, n, rp);
 }
 
 // Rows longest first, ties by index: a radix sort of the row numbers on their
