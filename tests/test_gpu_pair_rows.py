@@ -1,7 +1,7 @@
-"""MakeTransfers' row-by-row trace (packets, queued survivors, one direction of
-the bits and their mirror image) against the plain path's pair list: the same
-CSR, bit for bit, where tiles and words end and for orders, groups and targets
-the packets do not suit."""
+"""MakeTransfers' row-by-row trace (queued survivors, one direction of the bits
+and their mirror image) against the plain path's pair list: the same CSR, bit
+for bit, where tiles and words end, for patches out of order and for scattered
+groups."""
 import numpy as np
 import pytest
 
@@ -37,8 +37,8 @@ def same(a, b):
 
 
 # 32-column words, 512-row mirror tiles (one, an even and an odd number of
-# them), 64-segment batches; patches in order, shuffled (packets run out of
-# nodes) and with one group scattered over the indices
+# them), 64-segment batches; patches in order, shuffled (a wave's segments
+# run everywhere) and with one group scattered over the indices
 @pytest.mark.parametrize("order", ["listed", "shuffled"])
 @pytest.mark.parametrize("grouped", [False, True])
 @pytest.mark.parametrize("n", [1, 2, 31, 33, 65, 511, 513, 1024, 1537, 3001])

@@ -42,8 +42,7 @@ def test_room_transfers_bitexact(room_scene, path, batch):
     n = len(s.p_area)
     assert info.pairs_considered == n * (n - 1) // 2
     # segments traced = pairs i < j passing the facing cull, in the cull
-    # kernel's float32 arithmetic (the rounds' counts add up exactly, on one
-    # stream or two)
+    # kernel's float32 arithmetic (the launches' counts add up exactly)
     o = s.p_origin.astype(np.float32)
     nr = s.p_normal.astype(np.float32)
     want = 0

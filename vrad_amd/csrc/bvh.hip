@@ -1,18 +1,21 @@
 // Device builder of the 4-wide bounding-volume hierarchy the visibility
-// kernels walk (trace_dev.h::bvh_walk).  Results do not depend on the tree:
+// kernels walk (trace_dev.h::BvhTracer).  Results do not depend on the tree:
 // a walk returns the first hit in (t, triangle) order among all triangles, as
 // long as every box holds every point at which the triangle test can accept a
-// hit.  The kd-tree stays for the plain path and for vr_scene_get_kdtree.
+// hit.  The kd-tree stays for the plain path, for scenes past the hierarchy's
+// node limit and for vr_scene_get_kdtree.
 //
 //  k_bvh_bounds   per triangle, the box of its acceptance region (below)
 //  k_bvh_first    first position of each triangle in the kd-tree's index
 //  k_bvh_flag /   list: its leaves in depth-first order are a spatial order,
 //  k_bvh_order    so no sort is needed
-//  k_ploc_nn /    bottom-up clustering: every cluster looks kPlocR places to
-//  k_ploc_merge   either side for the neighbour whose union box has the least
-//                 area, mutual choices merge, the rest is compacted; two
-//                 launches per round, the last 2048 clusters in one workgroup
-//  k_ploc_final   (k_ploc_final)
+//  k_ploc_nn /    bottom-up clustering (after Meister and Bittner, "Parallel
+//  k_ploc_merge   Locally-Ordered Clustering for Bounding Volume Hierarchy
+//  k_ploc_final   Construction", IEEE TVCG 2018): every cluster looks kPlocR
+//                 places to either side for the neighbour whose union box has
+//                 the least area, mutual choices merge, the rest is compacted;
+//                 two launches per round, the last 2048 clusters in one
+//                 workgroup (k_ploc_final)
 //  k_bvh_collapse binary tree to 4-wide nodes, level by level from the root,
 //                 opening the child with the largest area first
 //
@@ -71,7 +74,7 @@ __device__ __forceinline__ float box_area(const Box &b) {
 
 // The box of every point p = o + t d at which tri_test can accept a hit at
 // the t it computes, for origins with |o| <= M (M: the scene's largest
-// coordinate; farther origins widen the walk's slabs instead, ray_slabs).
+// coordinate; farther origins widen the walk's slabs instead, BvhTracer::begin).
 // With u = 2^-24:
 //  - The test accepts when the rounded b0 = E0 h0 + E1 h1 + E2 >= 0, b1 >= 0
 //    and b0 + b1 <= 1.  For |h| <= 2M the rounding of b0 is at most
@@ -610,7 +613,8 @@ int build_bvh(const float4 *tris, int64_t n, const int32_t *idx, int64_t n_idx, 
   };
   const int64_t order_blocks = (src + 1023) / 1024, ploc_blocks = (cap + kPlocB - 1) / kPlocB;
   const size_t o_box = carve(sizeof(Box) * (size_t)n), o_live = carve((size_t)n);
-  const size_t o_first = carve(4 * (size_t)n), o_cnt = carve(4 * (size_t)std::max(order_blocks, 2 * ploc_blocks));
+  const size_t o_first = carve(4 * (size_t)n);
+  const size_t o_cnt = carve(4 * (size_t)std::max(order_blocks, 2 * ploc_blocks));
   const size_t o_order = carve(4 * (size_t)cap), o_nodes = carve(sizeof(Node2) * 2 * (size_t)cap);
   const size_t o_cb0 = carve(sizeof(Box) * (size_t)cap), o_cb1 = carve(sizeof(Box) * (size_t)cap);
   const size_t o_ci0 = carve(4 * (size_t)cap), o_ci1 = carve(4 * (size_t)cap);

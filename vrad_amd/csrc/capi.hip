@@ -1341,9 +1341,9 @@ int vr_make_transfers_batch(vr_scene *const *scenes, const vr_patches *patches,
   vr_xfer_params P{0.1f, -1, 1, 0};
   if (prm) P = *prm;
   const int64_t budget = P.batch_pairs > 0 ? P.batch_pairs : (int64_t)32 << 20;
-  // A scene with a whole round's budget of candidate pairs fills the GPU on
-  // its own: it takes the single-scene path (the same result), one launch
-  // per round of its own, and the shared launches serve the smaller scenes.
+  // A scene with a whole budget of candidate pairs fills the GPU on its own: it
+  // takes the single-scene path (the same result), and the shared launch
+  // serves the smaller scenes.
   std::vector<int32_t> shared;
   int rc = VR_OK;
   for (int32_t k = 0; k < n_scenes && rc == VR_OK; ++k) {

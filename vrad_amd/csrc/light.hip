@@ -87,7 +87,7 @@ constexpr int kGatherBatch = 192;  // lights between two sums of a workgroup
 //
 // Bound by the walks' latency: a wave alone walks light after light.  60,013
 // samples (938 groups on 1,024 SIMDs) with 9 lights and sky ambient took 2.07
-// ms with one wave per group; the rule for W is at launch_gather_light.
+// ms with one wave per group; the rule for W is at gather_waves.
 template <int W, class Tracer>
 __device__ void gather_group(const DevScene &sc, Tracer &tr, int wave, bool live, float px,
                              float py, float pz, float nx, float ny, float nz,
@@ -164,11 +164,9 @@ __device__ void gather_group(const DevScene &sc, Tracer &tr, int wave, bool live
 }
 
 template <int S, int W>
-__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_lds(DevScene sc, DevSamples s, int64_t n,
-                                                       const vr_light *__restrict__ lights,
-                                                       int32_t n_lights,
-                                                       const float *__restrict__ dirs, float eps,
-                                                       int32_t skip, float *__restrict__ rgb) {
+__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_lds(
+    DevScene sc, DevSamples s, int64_t n, const vr_light *__restrict__ lights, int32_t n_lights,
+    const float *__restrict__ dirs, float eps, int32_t skip, float *__restrict__ rgb) {
   __shared__ uint32_t s_stk[W * S * 64];
   __shared__ uint64_t s_vis[W > 1 ? kGatherBatch : 1];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -210,10 +208,9 @@ __global__ __launch_bounds__(256) void k_gather_plain(DevScene sc, DevSamples s,
 // uniform per wave), and lane l gathers that job's sample
 // (b - first block) * 64 + l from the job's scene and lights.
 template <int S, int W>
-__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_jobs(const GatherJob *__restrict__ jobs,
-                                                        int n_jobs,
-                                                        const float *__restrict__ dirs, float eps,
-                                                        int32_t skip) {
+__global__ __launch_bounds__(64 * W, W >= 16 ? 4 : 6) void k_gather_jobs(
+    const GatherJob *__restrict__ jobs, int n_jobs, const float *__restrict__ dirs, float eps,
+    int32_t skip) {
   __shared__ uint32_t s_stk[W * S * 64];
   __shared__ uint64_t s_vis[W > 1 ? kGatherBatch : 1];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -376,7 +373,9 @@ void launch_gather_light(const DevScene &sc, const DevSamples &s, int64_t n,
                        0, st, sc, s, n, lights, n_lights, sky_dirs, eps, skip, rgb);
   else {
     // the traversal-stack entries kept in LDS: the caller's (autotuned) knob
-#define VR_GATHER(S, W)                                                                        hipLaunchKernelGGL((k_gather_lds<S, W>), dim3((unsigned)((n + 63) / 64)), dim3(64 * W), 0, st,                      sc, s, n, lights, n_lights, sky_dirs, eps, skip, rgb)
+#define VR_GATHER(S, W)                                                                       \
+  hipLaunchKernelGGL((k_gather_lds<S, W>), dim3((unsigned)((n + 63) / 64)), dim3(64 * W), 0,  \
+                     st, sc, s, n, lights, n_lights, sky_dirs, eps, skip, rgb)
     VR_GATHER_W(VR_GATHER, gather_waves((n + 63) / 64, walks))
 #undef VR_GATHER
   }

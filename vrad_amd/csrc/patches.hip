@@ -577,7 +577,9 @@ static int make_patches_levels(const vr_face *faces, int64_t n_faces, float max_
     return fail(e == hipErrorOutOfMemory ? VR_E_NOMEM : VR_E_HIP,
                 std::string("make patches: ") + what + ": " + hipGetErrorString(e));
   };
-  auto M = [&](Buf &b, size_t bytes) { return H((hipError_t)dev_alloc(&b.p, bytes ? bytes : 16), "hipMalloc"); };
+  auto M = [&](Buf &b, size_t bytes) {
+    return H((hipError_t)dev_alloc(&b.p, bytes ? bytes : 16), "hipMalloc");
+  };
   const unsigned gf = (unsigned)((n_faces + 63) / 64);
   if ((rc = M(d_faces, sizeof(vr_face) * n_faces)) || (rc = M(d_tmp, sizeof(vr_patch) * n_faces)) ||
       (rc = M(d_has, n_faces)) || (rc = M(d_fb, 36 * n_faces)) || (rc = M(d_err, 4)) ||
@@ -744,7 +746,8 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
   };
   const size_t fb = sizeof(vr_face) * (size_t)n_faces;
   const size_t sb = sizeof(Pending) * kMaxDepth * (size_t)n_faces;
-  if ((rc = H((hipError_t)dev_alloc(&d_faces, fb), "hipMalloc")) || (rc = H((hipError_t)dev_alloc(&d_base, 4 * n_faces), "hipMalloc")) ||
+  if ((rc = H((hipError_t)dev_alloc(&d_faces, fb), "hipMalloc")) ||
+      (rc = H((hipError_t)dev_alloc(&d_base, 4 * n_faces), "hipMalloc")) ||
       (rc = H((hipError_t)dev_alloc(&d_cnt, 8 * n_faces), "hipMalloc")) ||
       (rc = H((hipError_t)dev_alloc(&d_ofs, 16 * n_faces), "hipMalloc")) ||
       (rc = H((hipError_t)dev_alloc(&d_stk, sb), "hipMalloc")) ||

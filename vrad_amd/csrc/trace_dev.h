@@ -175,14 +175,6 @@ __device__ __forceinline__ float tmax_wide(float a, float b) {
   return __int_as_float(max(__float_as_int(a), __float_as_int(b)));
 }
 
-// Walks one kd-tree (nodes/refs/bounds) for hits with tmin <= t < tmax that
-// come before (tbest, best) in (t, triangle index) order, updating them; the
-// result is the first of the hits in that order, bit for bit the brute-force
-// result.  ANY: return at the first accepted hit.  SKIPSKY: ignore
-// TRACE_ID_SKY triangles.  POSTPONE: lanes hold their next leaf and walk on
-// until every lane of the wave holds one (below).  Returns whether a hit was accepted (best_ref =
-// its leaf-reference index).  D = stack capacity; the host guarantees tree
-// depth < D.
 // What a walk needs of its ray besides origin and direction, the same for
 // every tree of a scene (the margin dl depends on the scene's extent M):
 // the reciprocal direction, and the slab terms of a split plane s on axis a,
@@ -211,12 +203,22 @@ __device__ __forceinline__ RayPre ray_pre(float M, float ox, float oy, float oz,
   return r;
 }
 
+// Walks one kd-tree (nodes/refs/bounds) for hits with tmin <= t < tmax that
+// come before (tbest, best) in (t, triangle index) order, updating them; the
+// result is the first of the hits in that order, bit for bit the brute-force
+// result.  The plain path and scenes past the hierarchy's node limit take this
+// walk.  ANY: return at the first accepted hit.  SKIPSKY: ignore TRACE_ID_SKY
+// triangles.  POSTPONE (closest hits): lanes hold their next leaf and walk on
+// until every lane of the wave holds one (below).  Returns whether a hit was
+// accepted (best_ref = its leaf-reference index).  D = stack capacity; the host
+// guarantees tree depth < D.
 template <int D, bool ANY, bool SKIPSKY, bool POSTPONE, class Stack>
 __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restrict__ refs,
                           const float *bmin, const float *bmax, const RayPre &rp, Stack &st,
                           float ox, float oy, float oz, float dx, float dy, float dz,
                           float tmin, float tmax, int32_t skip, float &tbest, int32_t &best,
                           int32_t &best_id, uint32_t &best_ref) {
+  static_assert(!(ANY && POSTPONE), "any-hit walks return at their first leaf's hit");
   const int32_t best0 = best;
   const float dl = rp.dl, ix = rp.ix, iy = rp.iy, iz = rp.iz;
   float ta = tmin, tb = tmax;
@@ -268,9 +270,8 @@ __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restr
     // have pruned them; the result is the least hit in (t, triangle) order
     // either way.  A step assigns each loop value once, by selects, and the
     // push is a predicated store.  Closest hits take this walk: their long
-    // walks through many leaves keep more lanes busy (4 M hemisphere rays on
-    // an 8x8-room level: 1.59 against 1.87 ms).  Any-hit walks, which mostly
-    // end at their first leaf, do not (0.73 against 0.64 ms on 4 M segments).
+    // walks through many leaves keep more lanes busy.  Any-hit walks, which
+    // mostly end at their first leaf, do not.
     uint32_t lstart = 0, lcnt = 0;  // the held leaf's triangles (none: lcnt 0)
     bool live = true;               // node, ta, tb: the next node to visit
     for (;;) {
@@ -296,7 +297,7 @@ __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restr
           const uint32_t left = nd.x >> 2;
           const bool fwd = i_a >= 0.0f;
           const uint32_t near_n = fwd ? left : left + 1, far_n = fwd ? left + 1 : left;
-          const float tbe = ANY ? tb : tmin_wide(tb, tbest);
+          const float tbe = tmin_wide(tb, tbest);
           const bool near_ok = ta <= tmin_wide(near_end, tbe);
           const float fs = tmax_wide(far_start, ta);
           const bool far_ok = fs <= tbe;
@@ -321,7 +322,6 @@ __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restr
       for (uint32_t k = lstart; k < lstart + lcnt; ++k)
         tri_test<SKIPSKY>(refs, k, ox, oy, oz, dx, dy, dz, tmin, skip, tbest, best, best_id,
                           best_ref);
-      if (ANY && best != best0) return true;
       lcnt = 0u;
       if (!live) break;
     }

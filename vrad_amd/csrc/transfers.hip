@@ -228,7 +228,8 @@ __device__ __forceinline__ void pair_rows(const PairJob &J, int64_t gb, float ep
     atomicAdd(J.segs + 8 * (blockIdx.x & 63u), (unsigned long long)total);
 }
 
-// 6 waves per SIMD: 186 ms on the level, 189 with 5, 198 with 8 (and spills)
+// 6 waves per SIMD: before waves of several octants took scalar node loads,
+// 186 ms on the level, against 189 with 5 and 198 with 8 (and spills)
 template <int S>
 __global__ __launch_bounds__(64, 6) void k_pair_rows(PairJob job, int64_t blk0, float eps,
                                                   int32_t skip, uint32_t xg) {
