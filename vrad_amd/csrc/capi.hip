@@ -443,7 +443,10 @@ std::vector<float> sky_dirs() {
   return std::vector<float>(&kAnorms[0][0], &kAnorms[0][0] + 162 * 3);
 }
 
-constexpr size_t kPackMost = (size_t)1 << 20;  // bytes of one packed copy
+// Bytes of one packed copy.  TestLine from host arrays: 32,768 segments (790 KB)
+// 104 us packed, 174 with a copy per array; 65,536 (1.6 MB) 170 as they are,
+// and 134 if a larger pinned block took them too.
+constexpr size_t kPackMost = (size_t)1 << 20;
 
 struct HostPart {  // part k of a staging block, in host memory (null or 0: skipped)
   int k;
@@ -914,7 +917,10 @@ int vr_scene_destroy(vr_scene *s) {
 }
 
 // ---- visibility ---------------------------------------------------------
-// Items of a host batch that the kernel reads from pinned memory itself.
+// Items of a host batch that the kernel reads from pinned memory itself: TestLine
+// of 4 / 2,048 segments takes 25 / 45 us so, 28 / 54 with a packed copy each way
+// and 84 / 104 with a copy per array.  Larger batches gain too (32,768: 82
+// against 104), but need more pinned memory than is kept.
 constexpr int64_t kDirectItems = 2048;
 
 int vr_trace_closest_dev(vr_scene *s, const vr_rays *r, int64_t n, int32_t skip_id,

@@ -194,7 +194,8 @@ __global__ __launch_bounds__(256) void k_gather_plain(DevScene sc, DevSamples s,
                                                       int32_t skip, float *__restrict__ rgb) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  KdTracer<D> tr(sc);
+  ScratchStack<D> st;
+  KdTracer<D> tr(sc, st);
   float r, g, b;
   gather_group<1>(sc, tr, 0, true, s.px[i], s.py[i], s.pz[i], s.nx[i], s.ny[i], s.nz[i], lights,
                   n_lights, dirs, eps, skip, nullptr, r, g, b);
@@ -335,7 +336,8 @@ __global__ __launch_bounds__(64) void k_leaf_sky_kd(DevScene sc, const int16_t *
                                                     const float *__restrict__ dirs,
                                                     uint8_t *__restrict__ out) {
   if ((int64_t)blockIdx.x >= n) return;
-  KdTracer<D> tr(sc);
+  ScratchStack<D> st;
+  KdTracer<D> tr(sc, st);
   leaf_sky(sc, tr, blockIdx.x, mins, maxs, dirs, out);
 }
 

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void k_trace_closest_plain(DevScene sc, DevRay
                                                              float *hit_t, float *hit_n) {
   const int64_t i = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  KdTracer<D> tr(sc);
+  ScratchStack<D> st;
+  KdTracer<D> tr(sc, st);
   float t;
   int32_t best, id;
   trace_ray(sc, tr, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.tmin[i],
@@ -138,7 +139,8 @@ __global__ __launch_bounds__(256) void k_test_line_plain(DevScene sc, DevSegs s,
                                                          uint8_t *sky) {
   const int64_t i = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  KdTracer<D> tr(sc);
+  ScratchStack<D> st;
+  KdTracer<D> tr(sc, st);
   bool hs;
   bool v = test_line(sc, tr, s.sx[i], s.sy[i], s.sz[i], s.ex[i], s.ey[i], s.ez[i], skip, hs);
   vis[i] = v ? 1 : 0;

@@ -62,9 +62,10 @@ __device__ __forceinline__ uint32_t xcd_chunk(uint32_t b, uint32_t nb) {
 // contiguous range would hold more work than the others' does not set the
 // launch's end; chunks of a group stay on one XCD.  g = 0 is xcd_chunk.  The
 // blocks past the last whole round of 8 g take xcd_chunk over the rest.
-// A bijection on [0, nb).  Groups of 256 chunks (16 K rays) took the
-// 8x8-room level's TestLine batch from 0.766 to 0.638 ms and its PVS
-// MakeTransfers from 0.615 to 0.530 s against one range per XCD.
+// A bijection on [0, nb).  On the 8x8-room level, with the hierarchy: PVS
+// MakeTransfers 217.6 ms with one range per XCD, 181.5 with groups of 256
+// chunks, 179 with 16 or 64, 199 with 4096; a TestLine batch of 4 M segments
+// 275, 281, 257 and 283 us; closest hits 182-185 us with any of them.
 constexpr uint32_t kXcdGroup = 256;
 __device__ __forceinline__ uint32_t xcd_group_chunk(uint32_t b, uint32_t nb, uint32_t g) {
   if (g == 0) return xcd_chunk(b, nb);
@@ -386,10 +387,10 @@ __device__ bool walk_tree(const uint2 *__restrict__ nodes, const float4 *__restr
 template <int D>
 struct KdTracer {
   const DevScene &sc;
-  ScratchStack<D> st;
+  ScratchStack<D> &st;  // not a member: the ray would move to private memory with it
   RayPre rp;
   float ox, oy, oz, dx, dy, dz;
-  __device__ explicit KdTracer(const DevScene &s) : sc(s) {}
+  __device__ KdTracer(const DevScene &s, ScratchStack<D> &stack) : sc(s), st(stack) {}
   __device__ __forceinline__ void begin(float ox_, float oy_, float oz_, float dx_, float dy_,
                                         float dz_) {
     ox = ox_;

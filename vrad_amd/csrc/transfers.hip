@@ -101,7 +101,8 @@ __global__ __launch_bounds__(256) void k_pair_trace_plain(DevScene sc, DevPatche
   if (k >= n) return;
   const int2 ij = pairs[k];
   const int i = ij.x, j = ij.y;
-  KdTracer<D> tr(sc);
+  ScratchStack<D> st;
+  KdTracer<D> tr(sc, st);
   const bool vis = segment_visible(sc, tr, p.ox[i] + eps * p.nx[i],
                                       p.oy[i] + eps * p.ny[i], p.oz[i] + eps * p.nz[i],
                                       p.ox[j] + eps * p.nx[j], p.oy[j] + eps * p.ny[j],
