@@ -64,6 +64,7 @@ void *t_alloc(int64_t n) {
   return vr::dev_alloc(&p, (size_t)n) == 0 ? p : nullptr;
 }
 void t_free(void *p) { vr::dev_free(p); }
+void t_free_idle(void *p) { vr::dev_free(p, true); }
 int64_t t_release() { return (int64_t)vr::dev_release(); }
 void t_holder(int delta) { vr::dev_holder(delta); }
 }

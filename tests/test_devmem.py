@@ -32,7 +32,7 @@ def pool(built, tmp_path):
     for name in ("t_used", "t_bytes", "t_syncs", "t_release"):
         getattr(lib, name).restype = C.c_int64
     lib.t_alloc.argtypes = lib.t_setup.argtypes = [C.c_int64]
-    lib.t_free.argtypes = lib.t_bytes.argtypes = lib.t_block_device.argtypes = [C.c_void_p]
+    lib.t_free_idle.argtypes = lib.t_free.argtypes = lib.t_bytes.argtypes = lib.t_block_device.argtypes = [C.c_void_p]
     lib.t_setup(64 * GB)
     return lib
 
@@ -207,6 +207,18 @@ def test_released_memory_is_there_for_others(hip):
     assert hip.free() - before < held // 2
     vrad_amd.release_memory()
     assert hip.free() - before >= held * 9 // 10
+
+
+def test_idle_blocks_need_no_synchronisation(pool):
+    """A block whose work the caller has waited for is available at once; others
+    still wait."""
+    a, b = pool.t_alloc(MB), pool.t_alloc(3 * MB)
+    pool.t_free_idle(a)
+    pool.t_free(b)
+    assert pool.t_alloc(MB) == a and pool.t_syncs(0) == 0
+    assert pool.t_alloc(3 * MB) == b and pool.t_syncs(0) == 1
+    pool.t_free_idle(a)
+    assert pool.t_release() == 0 and pool.t_bytes(a) == -1
 
 
 def test_host_scenes_hold_no_memory():

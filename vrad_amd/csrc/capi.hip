@@ -186,14 +186,16 @@ Pinned g_pin;
 struct DBuf {
   void *p = nullptr;
   size_t bytes = 0;
+  bool idle = false;  // the work that used it is known to be done (finish)
   DBuf() = default;
   DBuf(const DBuf &) = delete;
   DBuf &operator=(const DBuf &) = delete;
   ~DBuf() { release(); }
   void release() {
-    dev_free(p);
+    dev_free(p, idle);
     p = nullptr;
     bytes = 0;
+    idle = false;
   }
   int alloc(size_t n) {
     release();
@@ -222,6 +224,12 @@ struct DBuf {
   }
 };
 
+// The end of a call whose temporaries `bufs` were used on stream st alone.
+int finish(hipStream_t st, std::initializer_list<DBuf *> bufs) {
+  VR_HIP(hipStreamSynchronize(st));
+  for (DBuf *b : bufs) b->idle = true;
+  return VR_OK;
+}
 template <class T>
 int upload_vec(DBuf &b, const std::vector<T> &v, hipStream_t st) {
   return b.upload(v.data(), v.size() * sizeof(T), st);
@@ -3103,8 +3111,7 @@ int vr_cluster_from_points(const vr_bsp *bsp, const float *xyz, int64_t n, int16
     TRY(check_launch());
   }
   VR_HIP(hipMemcpyAsync(cluster, out.p, 2 * (size_t)n, hipMemcpyDeviceToHost, st));
-  VR_HIP(hipStreamSynchronize(st));
-  return VR_OK;
+  return finish(st, {&d.planes, &d.nodes, &d.leaves, &pts, &out});
 }
 
 int vr_patch_clusters(const vr_bsp *bsp, const vr_patch *patches, int64_t n, int32_t *cluster) {
@@ -3126,8 +3133,7 @@ int vr_patch_clusters(const vr_bsp *bsp, const vr_patch *patches, int64_t n, int
     TRY(check_launch());
   }
   VR_HIP(hipMemcpyAsync(cluster, out.p, 4 * (size_t)n, hipMemcpyDeviceToHost, st));
-  VR_HIP(hipStreamSynchronize(st));
-  return VR_OK;
+  return finish(st, {&d.planes, &d.nodes, &d.leaves, &pp, &out});
 }
 
 int vr_decompress_vis(const uint8_t *visdata, int64_t vis_len, const int32_t *pvs_ofs,
@@ -3162,7 +3168,7 @@ int vr_decompress_vis(const uint8_t *visdata, int64_t vis_len, const int32_t *pv
   unsigned long long f[2] = {0, 0};
   VR_HIP(hipMemcpyAsync(f, flags.p, 16, hipMemcpyDeviceToHost, st));
   VR_HIP(hipMemcpyAsync(rows, out.p, row * (size_t)n_clusters, hipMemcpyDeviceToHost, st));
-  VR_HIP(hipStreamSynchronize(st));
+  TRY(finish(st, {&vis, &ofs, &out, &flags}));
   const uint32_t err = (uint32_t)f[1];
   if (err & 1u) return fail(VR_E_INVALID, "DecompressVis: 0 repeat");
   if (err & 2u) return fail(VR_E_INVALID, "DecompressVis: run-length data ends inside a row");

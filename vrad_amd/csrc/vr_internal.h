@@ -18,7 +18,8 @@ int fail(int code, const std::string &msg);
 // ---- device memory (devmem.cpp) ---------------------------------------------
 // Blocks are kept and handed out again; dev_alloc returns 0 or the hipError_t.
 int dev_alloc(void **out, size_t n);
-void dev_free(void *p);  // work in flight may still use the block
+// Work in flight may still use the block, unless it is idle.
+void dev_free(void *p, bool idle = false);
 // scenes built on the device, transfer sets and servers alive, after the change
 int dev_holder(int delta);
 // gives every kept block back to the driver; the bytes that could not be (their
