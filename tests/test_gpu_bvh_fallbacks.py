@@ -126,3 +126,19 @@ def test_kd_fallback_light_and_sky(both):
     hi = lo + 8
     want, got = [lightmap.CanLeafTraceToSky(env, lo, hi) for env in envs]
     assert np.array_equal(want, got)
+
+
+@pytest.mark.parametrize("n", [1, 5, 3000])
+def test_no_triangle_can_be_hit(n):
+    """Triangles of no area (all points equal) have no normal: the scene has a
+    tree and no hierarchy."""
+    v9 = np.repeat(np.float32([[1, 2, 3]]), 3 * n, 0).reshape(n, 9)
+    ids = np.where(np.arange(n) % 2, H.SKY, H.OPAQUE).astype(np.int32)
+    env = Environment()
+    env.AddTriangles(v9, ids)
+    env.SetupAccelerationStructure()
+    o = np.float32([[0, 0, 0], [1, 2, 3], [1, 2, 0]])
+    d = np.float32([[0.267, 0.534, 0.802], [1, 0, 0], [0, 0, 1]])
+    hit, _ = env.TraceRays(o, d, 0.0, 1e30)
+    vis, sky = env.TestLines(o, o + 10 * d)
+    assert (np.asarray(hit) == -1).all() and np.asarray(vis).all() and not np.asarray(sky).any()

@@ -816,24 +816,33 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
   // whose meta holds the triangle's index in OptimizedTriangleList), planes,
   // and the hierarchies the optimised path walks.
   hipStream_t st = g_stream;
-  DBuf tris, children, split, idx, map;
+  DBuf tris, map;
   TRY(tris.upload(s->tris.data(), sizeof(TriIntersect) * s->tris.size(), st));
   const float4 *dt = tris.as<float4>();
+  TRY(s->planes.alloc(16 * (size_t)s->n_tri));
+  launch_planes(dt, s->n_tri, s->planes.as<float4>(), st);
+  TRY(check_launch());
   DevScene d{};
   auto tree = [&](const KdTree &t, const int32_t *own, DBuf &nodes, DBuf &refs, DBuf &bvh,
                   DBuf &bvh_refs, bool all) -> int {
     const int64_t nn = (int64_t)t.children.size(), ni = (int64_t)t.idx.size();
-    TRY(children.upload(t.children.data(), 4 * (size_t)nn, st));
-    TRY(split.upload(t.split.data(), 4 * (size_t)nn, st));
-    TRY(idx.upload(t.idx.data(), 4 * (size_t)ni, st));
+    Staging S;
+    const size_t nb = 4 * (size_t)nn, ib = 4 * (size_t)ni;
+    TRY(S.make({nb, nb, ib}));
+    TRY(S.upload({{0, const_cast<uint32_t *>(t.children.data()), nb},
+                  {1, const_cast<float *>(t.split.data()), nb},
+                  {2, const_cast<int32_t *>(t.idx.data()), ib}},
+                 st));
+    const int32_t *const idx = S.ptr<int32_t>(2);
     TRY(nodes.alloc(8 * (size_t)nn));
     TRY(refs.alloc(48 * (size_t)ni));
-    launch_kd_records(children.as<uint32_t>(), split.as<float>(), nn, idx.as<int32_t>(), ni, own,
-                      dt, nodes.as<uint2>(), refs.as<float4>(), st);
+    launch_kd_records(S.ptr<uint32_t>(0), S.ptr<float>(1), nn, idx, ni, own, dt,
+                      nodes.as<uint2>(), refs.as<float4>(), st);
     TRY(check_launch());
     BvhBuild b;
+    b.host = reinterpret_cast<int32_t *>(g_pin.take(512));
     const int rc = own ? build_bvh(dt, s->n_tri, own, (int64_t)s->sky_index.size(), all, M, st, &b)
-                       : build_bvh(dt, s->n_tri, idx.as<int32_t>(), ni, all, M, st, &b);
+                       : build_bvh(dt, s->n_tri, idx, ni, all, M, st, &b);
     bvh.release();
     bvh_refs.release();
     bvh.p = b.nodes;
@@ -850,9 +859,6 @@ int vr_scene_build(vr_scene *s, int32_t n_threads) {
     TRY(tree(s->kd_sky, map.as<int32_t>(), s->sky_nodes, s->sky_refs, s->sky_bvh,
              s->sky_bvh_refs, false));
   }
-  TRY(s->planes.alloc(16 * (size_t)s->n_tri));
-  launch_planes(dt, s->n_tri, s->planes.as<float4>(), st);
-  TRY(check_launch());
   VR_HIP(hipStreamSynchronize(st));
   d.nodes = s->nodes.as<uint2>();
   d.refs = s->refs.as<float4>();

@@ -61,6 +61,7 @@ int make_patches_device(const vr_face *faces, int64_t n_faces, float max_chop, f
 // memory, M the scene's largest coordinate (at least 1).  Allocates nodes and
 // refs with dev_alloc; none when no triangle can be hit.
 struct BvhBuild {
+  int32_t *host = nullptr;  // 128 words of pinned memory for the counts (nullable)
   void *nodes = nullptr, *refs = nullptr;
   int64_t n_nodes = 0, n_refs = 0;
   int levels = 0;
