@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256) void k_bvh_collapse(
 // launch per level was 12 launches of some 5 us, 78 us for 1,584 triangles
 // against 45.  With the small scenes' records written in place, one upload per
 // tree and their counts read into pinned memory, the build of 96 triangles went
-// from 235 to 180 us and that of 1,584 from 1.82 to 1.66 ms (86 us and 1.55 ms
+// from 235 to 172 us and that of 1,584 from 1.82 to 1.66 ms (86 us and 1.55 ms
 // without the hierarchy).
 __global__ __launch_bounds__(1024) void k_bvh_collapse_all(
     const Node2 *__restrict__ nodes, const int32_t *__restrict__ order,

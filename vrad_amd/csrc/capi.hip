@@ -1074,7 +1074,7 @@ int vr_test_line(vr_scene *s, const vr_segs *g, int64_t n, int32_t skip_id, uint
 
 // ---- transfers ------------------------------------------------------------
 __global__ void k_add_count(const uint32_t *c, uint32_t cap, unsigned long long *tot) {
-  atomicAdd(tot, (unsigned long long)min(*c, cap));  // rounds on two streams add here
+  atomicAdd(tot, (unsigned long long)min(*c, cap));  // every round adds here
 }
 
 // The candidate-pair plan of a PVS: patches grouped by cluster, the group
