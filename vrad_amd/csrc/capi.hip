@@ -145,8 +145,9 @@ int check_launch() {
 }
 
 // Pinned host memory of the host-pointer calls, one block until the process
-// ends, used under the library lock by one call at a time (every such call
-// leaves its stream drained).  A copy from or to pageable memory costs some 25
+// ends, used under the library lock by one call at a time (a call that returns
+// VR_OK has drained its stream; what a failed one still copies from here goes
+// to blocks that wait for the device).  A copy from or to pageable memory costs some 25
 // us whatever its size; small calls pack their arrays here and pay one copy
 // each way, or let the kernel read and write this block itself.
 struct Pinned {
