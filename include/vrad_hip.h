@@ -199,6 +199,9 @@ typedef struct {
  * NTriangleID == skip_id.  hit_idx = -1 for no hit, else the index into
  * OptimizedTriangleList (raytracer/types/result.go:8-12);
  * hit_normal (3n, nullable) = the hit triangle's plane normal.
+ * Directions need not be of unit length, but the walk takes a component below
+ * 1e-20 as 1e-20 of its sign: of a direction whose largest component is below
+ * some 1e-13, hits can be missed.
  * A non-NULL transparency callback has no C form (VR_E_UNSUPPORTED is
  * returned by the Go wrapper before calling here). */
 int vr_trace_closest(vr_scene *s, const vr_rays *rays, int64_t n,
