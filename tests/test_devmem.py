@@ -127,6 +127,20 @@ def test_requests_that_fit_the_device_are_served(pool):
     assert pool.t_used() == 64 * GB
 
 
+def test_small_requests_share_blocks_when_nothing_is_spare(pool):
+    """The bound is for what counts: up to 64 KiB a block is always rounded."""
+    pool.t_holder(1)
+    for n in (6300 * MB, 200 * MB + 1, 3 * MB + 1, MB + 1, 300001, 70001, 5000):
+        while True:  # until the size is no longer rounded, or often enough
+            p = pool.t_alloc(n)
+            if pool.t_bytes(p) == n or pool.t_used() > 60 * GB or n <= 70001:
+                break
+    a = pool.t_alloc(37000)
+    assert pool.t_bytes(a) == 40960
+    pool.t_free(a)
+    assert pool.t_alloc(39000) == a
+
+
 def test_similar_requests_share_a_block(pool):
     pool.t_holder(1)
     for n in (1001 * MB, 1010 * MB, 990 * MB):

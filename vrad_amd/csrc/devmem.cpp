@@ -103,8 +103,10 @@ struct Pool {
     while (D.kept > most && !D.ready.empty()) drop(D, std::prev(D.ready.end()));
   }
   // Whether n more bytes than asked for may be handed out: 1/128 of the device
-  // in all, so that a set of blocks near its capacity still fits.
-  static bool can_spare(const Device &D, size_t n) { return D.spare + n <= D.cap / 16; }
+  // in all, so that a set of blocks near its capacity still fits; 64 KiB always.
+  static bool can_spare(const Device &D, size_t n) {
+    return n <= 65536 || D.spare + n <= D.cap / 16;
+  }
   // a kept block for a request of n bytes rounded to r: at most an eighth (and
   // a page) larger
   static std::multimap<size_t, void *>::iterator fit(Device &D, size_t n, size_t r) {
